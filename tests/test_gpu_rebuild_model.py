@@ -35,6 +35,36 @@ def test_forward_and_gradient_match_cpu_reference():
     assert np.max(np.abs(g - gr)) < 1e-4 * np.max(np.abs(gr))
 
 
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 255, 256, 257, 1000])
+def test_sample_tiles_and_gradient_chunks(n):
+    """Counts around the tiles of 16 samples and the chunks of 256: forward,
+    loss and gradient against the float64 reference (the bounds of the test
+    above), and three Adam steps over the whole set against the reference's
+    gradients.  A step moves a parameter by at most lr, and by rounding alone
+    only where its gradient is of the rounding's size: the bound is a
+    thousandth of the way taken plus one such parameter's six lr."""
+    from rockable_amd.engine import Mlp
+    p, X, t = _rand(seed=n, n=n)
+    mlp = Mlp(seed=3)
+    mlp.set_params(p)
+    x64, t64 = X.astype(np.float64), t.astype(np.float64)
+    yr, _ = M.forward(p.astype(np.float64), x64)
+    assert np.max(np.abs(mlp.forward(X) - yr)) < 1e-5 * max(1.0, np.max(np.abs(yr)))
+    loss, g = mlp.loss_grad(X, t)
+    lr_, gr = M.loss_grad(p.astype(np.float64), x64, t64)
+    assert abs(loss - lr_) < 1e-5 * max(1.0, lr_)
+    assert np.max(np.abs(g - gr)) < 1e-4 * np.max(np.abs(gr))
+    lr = 1e-3
+    final = mlp.train(X, t, epochs=3, batch=n, lr=lr, seed=1)
+    q, m, v = p.astype(np.float64), np.zeros(M.NPARAMS), np.zeros(M.NPARAMS)
+    for k in range(1, 4):
+        gk = M.loss_grad(q, x64, t64)[1]
+        m, v = 0.9 * m + 0.1 * gk, 0.999 * v + 0.001 * gk * gk
+        q = q - lr * (m / (1 - 0.9 ** k)) / (np.sqrt(v / (1 - 0.999 ** k)) + 1e-8)
+    assert np.linalg.norm(mlp.params() - q) < 1e-3 * np.linalg.norm(q - p) + 6 * lr
+    assert abs(final - M.loss_grad(q, x64, t64)[0]) < 1e-3 * max(1.0, final)
+
+
 def test_training_fits_a_smooth_function():
     """Adam with the library's kernels: on t = sin(2 x0) + x1^2 / 2 the loss
     falls by more than 20x."""
