@@ -166,18 +166,16 @@ int rk_set_body_force(rk_engine* eng, const char* name, const double* args, int 
  * a block's entries by contact type; 0: in list order), "law_group" (geometry blocks per force-law
  * wavefront when not fused: 1, 2, 4, 8; default 1), "geom_block"
  * (contact-kinematics workgroup when not fused: 64, 128, 256, 512; default
- * 256), "gather_lanes" (lanes per body in the resultant sums: 8, 16; default
- * 16), "gather_groups" (groups of 64 / gather_lanes bodies per resultant
- * wavefront: 1, 2, 4, 8, 16, at most gather_lanes; 0, the default: 1 below
- * 262144 bodies, gather_lanes from there), "fuse_glob" (1: the predictor
+ * 256), "gather_lanes" (8, 16), "gather_groups" (0, 1, 2, 4, 8, 16) and
+ * "gather_waves" (1, 2, 4) (kept for callers that set them, without effect:
+ * the resultant kernel has one shape), "fuse_glob" (1: the predictor
  * writes the free bodies' global vertices, one thread per body; 2: one
  * thread per vertex; 3: workgroups of 64 bodies, their vertices shared by the
  * workgroup; 0: a kernel of its own; -1, the default: 0 from 262144
- * bodies, else 3), "gather_waves" (wavefronts per resultant
- * workgroup: 1, 2, 4; default 4), "body_block" (per-body kernels: 64, 128,
+ * bodies, else 3), "body_block" (per-body kernels: 64, 128,
  * 256; default 256), "persistent" (0, the default: one tile per workgroup;
  * n in [8, 1048576]: the step kernels' grids capped at n workgroups, each
- * looping over its tiles), "narrow_pairs" (candidate body pairs per
+ * looping over its tiles; the resultant kernel's are not capped), "narrow_pairs" (candidate body pairs per
  * narrow-phase wavefront: 1, 2; 0, the default: 2 for shapes of up to 8
  * vertices, else 1).  No option changes results. */
 int rk_set_option(rk_engine* eng, const char* name, double value);
@@ -185,8 +183,7 @@ int rk_set_option(rk_engine* eng, const char* name, double value);
  * "dVerlet" and "tmax". */
 int rk_get_option(rk_engine* eng, const char* name, double* value);
 /* Autotuner (no counterpart in the reference) of fuse_law, law_group,
- * geom_block, gather_lanes, gather_groups, fuse_glob, gather_waves,
- * body_block, persistent, graph_steps, type_sort and skip_segment, one after the other: the
+ * geom_block, fuse_glob, body_block, persistent, graph_steps, type_sort and skip_segment, one after the other: the
  * simulation runs on, trial after trial of steps_per_trial steps, each
  * candidate value twice, and the fastest is kept: by the step kernels' own
  * durations per step (events around each kernel) for the kernel shapes, by

@@ -42,11 +42,13 @@ struct rk_engine {
   int profile = 0;
   std::map<std::string, KernelTimer> timers;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  int law_group = 1, geom_block = 256, gather_waves = 4, body_block = 256, fuse_law = 1, gather_lanes = 16;
-  // 0 / -1: chosen from the packing's size (large packings: 64 bodies per
-  // resultant wavefront, global vertices written by the predictor per body;
-  // smaller ones: by the predictor's workgroups of 64 bodies)
-  int gather_groups = 0, fuse_glob = -1;
+  int law_group = 1, geom_block = 256, body_block = 256, fuse_law = 1;
+  // accepted and read back, without effect: the resultant kernel has one shape
+  int gather_waves = 4, gather_lanes = 16, gather_groups = 0;
+  // -1: chosen from the packing's size (large packings: global vertices by a
+  // kernel of their own; smaller ones: by the predictor's workgroups of 64
+  // bodies)
+  int fuse_glob = -1;
   int type_sort = 1;
   int persist = 0;
   // host wall time of the rebuilds while the autotuner runs (it synchronises
@@ -422,15 +424,11 @@ void assemble_dev(rk_engine* eng) {
   d.exact_sums = eng->exact_sums;
   d.law_group = eng->law_group;
   d.geom_block = eng->geom_block;
-  d.gather_waves = eng->gather_waves;
   d.body_block = eng->body_block;
   d.fuse_law = eng->fuse_law;
-  d.gather_lanes = eng->gather_lanes;
   d.type_sort = eng->type_sort;
   {
     const bool large = d.nb >= kLargePacking;
-    const int g = eng->gather_groups > 0 ? eng->gather_groups : large ? eng->gather_lanes : 1;
-    d.gather_groups = std::min(g, eng->gather_lanes);
     d.fuse_glob = eng->fuse_glob >= 0 ? eng->fuse_glob : large ? 0 : 3;
   }
   d.persist = eng->persist;
@@ -2080,7 +2078,6 @@ int rk_set_option(rk_engine* eng, const char* name, double value) {
   } else if (n == "gather_lanes") {
     if (!(value == 8.0 || value == 16.0)) return fail(eng, "gather_lanes must be 8 or 16");
     eng->gather_lanes = (int)value;
-    if (eng->loaded) assemble_dev(eng);
   } else if (n == "type_sort") {
     if (!(value == 0.0 || value == 1.0)) return fail(eng, "type_sort must be 0 or 1");
     eng->type_sort = (int)value;
@@ -2093,7 +2090,6 @@ int rk_set_option(rk_engine* eng, const char* name, double value) {
     if (!(value == 0.0 || value == 1.0 || value == 2.0 || value == 4.0 || value == 8.0 || value == 16.0))
       return fail(eng, "gather_groups must be 0 (by size), 1, 2, 4, 8 or 16");
     eng->gather_groups = (int)value;
-    if (eng->loaded) assemble_dev(eng);
   } else if (n == "fuse_glob") {
     if (!(value == -1.0 || value == 0.0 || value == 1.0 || value == 2.0 || value == 3.0))
       return fail(eng, "fuse_glob must be -1 (by size), 0, 1, 2 or 3");
@@ -2202,10 +2198,7 @@ int rk_autotune(rk_engine* eng, int steps_per_trial, int64_t* steps_done) {
                         {"skip_segment", {1024, 2048, 512, 4096, 256}},
                         {"law_group", {1, 2, 4, 8}},
                         {"geom_block", {64, 128, 256, 512}},
-                        {"gather_lanes", {8, 16}},
-                        {"gather_groups", {1, 4, 16}},
                         {"fuse_glob", {0, 1, 2, 3}},
-                        {"gather_waves", {1, 2, 4}},
                         {"body_block", {64, 128, 256}},
                         {"persistent", {0, 2048, 8192}},
                         {"graph_steps", {0, 8, 32}}};

@@ -1990,7 +1990,7 @@ int entries_reserve(NLWork& w, EntryArrays& E, int n) {
             hipMalloc(&E.estick, c * sizeof(int32_t)) == hipSuccess && hipMalloc(&E.eact, c * sizeof(uint8_t)) == hipSuccess &&
             hipMalloc(&E.ekey, c * sizeof(double)) == hipSuccess &&
             hipMalloc(&E.spos, c * 2 * sizeof(int32_t)) == hipSuccess &&
-            hipMalloc(&E.sact, c * 2 * sizeof(uint8_t)) == hipSuccess &&
+            hipMalloc(&E.sact, c * 2 * sizeof(uint8_t) + 64) == hipSuccess  /* read 16 bytes at a time */ &&
             hipMalloc(&E.sval, c * 12 * sizeof(double)) == hipSuccess &&
             hipMalloc(&E.akin, (c + 512) * sizeof(ActiveKin)) == hipSuccess &&
             hipMalloc(&E.acount, (c / 64 + 2) * sizeof(int32_t)) == hipSuccess;

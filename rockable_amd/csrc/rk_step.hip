@@ -905,15 +905,12 @@ __device__ __forceinline__ double pick(const v3& F, const v3& M, int c) {
   return c == 0 ? F.x : c == 1 ? F.y : c == 2 ? F.z : c == 3 ? M.x : c == 4 ? M.y : M.z;
 }
 
-// Stores the resultants, compute_accelerations_from_resultants
-// (Rockable.cpp:3419-3552) and the closing half kick (2120-2155).
+// compute_accelerations_from_resultants (Rockable.cpp:3419-3552) into acc and
+// arot, and with kick the closing half kick (2120-2155) of P's velocities.
 // m, I: the body's mass and principal inertia (loaded by the caller, early)
-__device__ __forceinline__ void finish_body(const Dev& d, const StepParams& sp, int kick, int b, BodyKin& P,
-                                            bool driven, v3 F, v3 M, int c0, int c1, double m, v3 I) {
-  st3(d.force + 3 * (size_t)b, F);
-  st3(d.moment + 3 * (size_t)b, M);
+__device__ __forceinline__ void accelerate(const Dev& d, const StepParams& sp, int kick, BodyKin& P, bool driven, v3 F,
+                                           v3 M, int c0, int c1, double m, v3 I, v3& acc, v3& arot) {
   const qt Q = kq(P);
-  v3 acc, arot;
   if (driven) {
     acc = V(0.0, 0.0, 0.0);
     arot = V(0.0, 0.0, 0.0);
@@ -945,8 +942,6 @@ __device__ __forceinline__ void finish_body(const Dev& d, const StepParams& sp, 
     v3 Mb = qrot(Qinv, M);
     arot = qrot(Q, euler_domega(I, omega, Mb));
   }
-  st3(d.acc + 3 * (size_t)b, acc);
-  st3(d.arot + 3 * (size_t)b, arot);
   if (!kick) return;
   if (driven) {
     for (int qq = c0; qq < c1; qq++) {
@@ -970,6 +965,21 @@ __device__ __forceinline__ void finish_body(const Dev& d, const StepParams& sp, 
     P.wy = w.y;
     P.wz = w.z;
   }
+}
+__device__ __forceinline__ void store_resultants(const Dev& d, int b, v3 F, v3 M, v3 acc, v3 arot) {
+  st3(d.force + 3 * (size_t)b, F);
+  st3(d.moment + 3 * (size_t)b, M);
+  st3(d.acc + 3 * (size_t)b, acc);
+  st3(d.arot + 3 * (size_t)b, arot);
+}
+
+// A body finished by itself: resultants, accelerations, kicked velocities.
+__device__ __forceinline__ void finish_body(const Dev& d, const StepParams& sp, int kick, int b, BodyKin& P,
+                                            bool driven, v3 F, v3 M, int c0, int c1, double m, v3 I) {
+  v3 acc, arot;
+  accelerate(d, sp, kick, P, driven, F, M, c0, c1, m, I, acc, arot);
+  store_resultants(d, b, F, M, acc, arot);
+  if (!kick) return;
   BodyKin* out = d.kin + b;
   out->vx = P.vx;
   out->vy = P.vy;
@@ -1031,157 +1041,332 @@ __device__ __forceinline__ void guard_body(const Dev& d, const StepParams& sp, i
 }
 __device__ __forceinline__ bool guard_reset(const Dev& d) { return *(volatile const int*)&d.guard->reset != 0; }
 
-// compute_resultants (Rockable.cpp:3267-3272).  L lanes per body (8 or 16;
-// 64 / L bodies per wavefront).  The lanes read the slot activity bytes 64
-// at a time (64 / L each) and join them into one mask; lanes 0-5, one per
-// component of (F, M), then fetch the terms of the active slots eight at a
-// time (independent loads) and add them in slot order.  Called by every
-// lane of the wavefront; returns the updated sum in lanes gl < 6.
-template <int L>  // lanes per body: 8 or 16 (windows of 64 slots, 64 / L per lane)
-__device__ __forceinline__ double sum_slots(const Dev& d, bool run, int k0, int k1, int gl, double s) {
-  constexpr int B = 64 / L;  // activity bytes read per lane and window
-  const double* val = d.sval + (gl < 6 ? gl : 0);
-  for (int it = 0;; it++) {
-    const int w = k0 + 64 * it;
-    const bool live = run && w < k1;
-    if (!__any(live)) break;
-    unsigned mb = 0u;
-    if (live) {
+// predict_free: the new pose and velocities of free body b (Rockable.cpp:
+// 2036-2055) in P; store_predicted writes them back
+__device__ __forceinline__ void predict_free_with(const StepParams& sp, BodyKin& P, v3 a, v3 ar) {
+  v3 pos = vadd(kpos(P), vadd(vsc(sp.dt, kvel(P)), vsc(sp.dt2_2, a)));
+  v3 vel = vadd(kvel(P), vsc(sp.dt_2, a));
+  qt Q = kq(P);
+  const v3 w = kvrot(P);
+  Q = qadd_scaled(Q, qdot(Q, w), sp.dt);
+  Q = qadd_scaled(Q, qddot(Q, w, ar), sp.dt2_2);
+  qnormalize(&Q);
+  v3 w2 = vadd(w, vsc(sp.dt_2, ar));
+  P.px = pos.x;
+  P.py = pos.y;
+  P.pz = pos.z;
+  P.qw = Q.w;
+  P.qx = Q.x;
+  P.qy = Q.y;
+  P.qz = Q.z;
+  P.vx = vel.x;
+  P.vy = vel.y;
+  P.vz = vel.z;
+  P.wx = w2.x;
+  P.wy = w2.y;
+  P.wz = w2.z;
+}
+__device__ __forceinline__ void predict_free(const Dev& d, const StepParams& sp, int b, BodyKin& P) {
+  predict_free_with(sp, P, ld3(d.acc + 3 * (size_t)b), ld3(d.arot + 3 * (size_t)b));
+}
+// The far-entry skip's motion bound of one predicted body: no vertex of it
+// moved by more than |dx| + 2 |dQ| rmax in this step (for unit quaternions
+// |Q' v Q'* - Q v Q*| <= 2 |Q' - Q| |v|), plus a rounding allowance.
+__device__ __forceinline__ void add_motion_bound_with(const Dev& d, int b, const BodyKin& old, const BodyKin& P,
+                                                      double cb, double rmax) {
+  if (!d.skip_far) return;
+  const double dx = P.px - old.px, dy = P.py - old.py, dz = P.pz - old.pz;
+  const double qw = P.qw - old.qw, qx = P.qx - old.qx, qy = P.qy - old.qy, qz = P.qz - old.qz;
+  const double step = sqrt(dx * dx + dy * dy + dz * dz) + 2.0 * sqrt(qw * qw + qx * qx + qy * qy + qz * qz) * rmax;
+  const double mag = fabs(P.px) + fabs(P.py) + fabs(P.pz);
+  d.cbound[b] = cb + (step + 1e-15 * (1.0 + mag));
+}
+__device__ __forceinline__ void add_motion_bound(const Dev& d, int b, const BodyKin& old, const BodyKin& P) {
+  if (!d.skip_far) return;
+  add_motion_bound_with(d, b, old, P, d.cbound[b], d.rmax[b]);
+}
+
+typedef double d2 __attribute__((ext_vector_type(2)));  // one 16-byte access
+
+// A body record (BodyKin, 16 doubles) in LDS at r.
+__device__ __forceinline__ BodyKin rec_load(const double* r) {
+  BodyKin P;
+  P.px = r[0];
+  P.py = r[1];
+  P.pz = r[2];
+  P.qw = r[3];
+  P.qx = r[4];
+  P.qy = r[5];
+  P.qz = r[6];
+  P.vx = r[7];
+  P.vy = r[8];
+  P.vz = r[9];
+  P.wx = r[10];
+  P.wy = r[11];
+  P.wz = r[12];
+  P.R = r[13];
+  P.h = r[14];
+  P.shape = __double2loint(r[15]);
+  P.group = __double2hiint(r[15]);
+  return P;
+}
+__device__ __forceinline__ void rec_store_motion(double* r, const BodyKin& P) {
+  r[0] = P.px;
+  r[1] = P.py;
+  r[2] = P.pz;
+  r[3] = P.qw;
+  r[4] = P.qx;
+  r[5] = P.qy;
+  r[6] = P.qz;
+  r[7] = P.vx;
+  r[8] = P.vy;
+  r[9] = P.vz;
+  r[10] = P.wx;
+  r[11] = P.wy;
+  r[12] = P.wz;
+}
+constexpr int kRec = 17;  // LDS doubles per record (16, and one so that the per-body reads spread over the banks)
+static_assert(sizeof(BodyKin) == 16 * sizeof(double), "a body record is 16 doubles");
+
+// Bit k of the result: byte k of x (each 0 or 1).
+__device__ __forceinline__ unsigned byte_bits(unsigned x) { return ((x & 0x01010101u) * 0x10204080u) >> 28; }
+
+// compute_resultants (Rockable.cpp:3267-3272) as a per-body sum in slot
+// order, with initialise_particle_forces_and_moments, the accelerations and
+// the closing kick.  A workgroup takes NB free bodies, whose slots are
+// consecutive, or one driven body:
+//   1. the 256 threads read all the slots' activity bytes (16 each, up to
+//      4 096 slots at a time) and rank the active ones into an LDS list;
+//   2. they read the active slots' terms (48 bytes each), 512 slots at a
+//      time, into LDS;
+//   3. lanes of each body, one per component of (F, M), add its terms in
+//      slot order, so every component is the reference's bit for bit;
+//   4. one thread per body finishes it.  The records (128 bytes) are read at
+//      the start and written back whole, in contiguous doubles, through LDS.
+// What bounds it is the chain of dependent loads (slot range, activity,
+// terms): here three, whatever the bodies' slot counts.  Before, 16 lanes
+// took one body, read its activity 64 bytes and its terms 8 slots at a time,
+// so a wall with 200 slots or a bonded cube with 18 active ones waited for
+// many loads in turn, and 4 of a wavefront's lanes finished its bodies:
+// 15.7 us for 706 bodies, 22.6 us for 50 005, 40.3 us for 90 006 with the
+// displacement check, 13.7 us for 13 001 bonded cubes; now 6.6, 14.8, 23.4 and
+// 10.3 us.
+// Driven bodies come first, one workgroup each (a wall's many slots fill it);
+// then, a wavefront each, the 64-slot chunks of the heavy bodies, whose
+// partial sums (from -0.0, the identity of addition) k_heavy_finish takes.
+// Bodies with more than heavy_min slots are left to the heavy kernels.  With
+// guard, the displacement check accumulates each finished body and every
+// workgroup stores its maxima in gpart[2 blockIdx.x].  One tile per workgroup
+// whatever the persistent option: in a loop over tiles the compiler keeps the
+// loop's invariants in 196 registers (102 without).
+constexpr int kGatherCap = 512;   // slots' terms in LDS
+constexpr int kGatherWin = 4096;  // slots scanned at a time: 16 per thread
+
+// The sum of one component (lanes gl < 6) over the slots [k0, k1) of one
+// chunk of at most 64 slots by one wavefront, from -0.0, in slot order
+// (inactive slots as -0.0: x + (-0.0) == x for every x).
+__device__ __forceinline__ double sum_chunk(const Dev& d, int k0, int k1, int lane, double* lds) {
+  const int k = k0 + lane;
+  d2 v[3];
 #pragma unroll
-      for (int q = 0; q < B; q++) {
-        const int k = w + B * gl + q;
-        if (k < k1 && d.sact[k]) mb |= 1u << q;
-      }
-    }
-    unsigned long long rest = (unsigned long long)mb << (B * gl);
-    for (int o = 1; o < L; o <<= 1) rest |= __shfl_xor(rest, o, L);
-    if (gl < 6) {
-      while (rest) {
-        double x[8];
-        int n = 0;
+  for (int q = 0; q < 3; q++) v[q] = d2{-0.0, -0.0};
+  if (k < k1 && d.sact[k]) {
+    const d2* t = reinterpret_cast<const d2*>(d.sval + 6 * (size_t)k);
 #pragma unroll
-        for (int t = 0; t < 8; t++) {
-          x[t] = 0.0;
-          if (rest) {
-            const int pbit = __ffsll((long long)rest) - 1;
-            rest &= rest - 1ull;
-            x[t] = val[6 * (size_t)(w + pbit)];
-            n = t + 1;
-          }
-        }
+    for (int q = 0; q < 3; q++) v[q] = t[q];
+  }
+  d2* out = reinterpret_cast<d2*>(lds + 6 * lane);
 #pragma unroll
-        for (int t = 0; t < 8; t++)
-          if (t < n) s += x[t];
-      }
-    }
+  for (int q = 0; q < 3; q++) out[q] = v[q];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  double s = -0.0;
+  if (lane < 6) {
+#pragma unroll 16
+    for (int q = 0; q < 64; q++) s += lds[6 * q + lane];
   }
   return s;
 }
 
-// Bodies with at most heavy_min slots: the serial sum, so every component is
-// the reference's bit for bit.  A body wavefront takes G groups of 64 / L
-// bodies (G from 1 to L, so 64 / L to 64 bodies), one per lane: each lane
-// loads its body's slot range and initial force and moment, the slots are
-// summed group after group (L lanes per body; groups with no slot are
-// skipped), and each lane then finishes its own body.  Few groups keep more
-// wavefronts in flight (small packings), many use every lane for the
-// per-body work (large ones).  The
-// wavefronts after the bodies' take the 64-slot chunks of the heavy bodies
-// and store each chunk's partial sums (from -0.0, the identity of addition)
-// for k_heavy_finish.  With guard, the displacement check accumulates each
-// finished body and every workgroup stores its maxima in gpart[2 blockIdx.x].
-// Occupancy asked of the compiler: 5 wavefronts per SIMD without a body force
-// (96 VGPRs, no spill), 3 with one (its code needs more registers).
-template <int L, bool BF>  // BF: the deck has a body force
-__global__ void __launch_bounds__(kBlock, BF ? 3 : 5) k_gather(Dev d, StepParams sp, int kick, int guard) {
-  constexpr int kPer = 64 / L;  // bodies per slot group (chunks per chunk wavefront)
-  __shared__ unsigned long long red[2][kBlock / 64];
+template <int NB, bool BF>  // BF: the deck has a body force
+__global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, int kick, int guard) {
+  constexpr int kLanes = kBlock / NB;      // lanes per body in the sums (8 or 4)
+  constexpr int kComp = kLanes >= 6 ? 1 : 2;  // components per lane
+  __shared__ double rec[NB * kRec];
+  __shared__ __align__(16) double vals[kGatherCap * 6];
+  __shared__ unsigned short list[kGatherWin];
+  __shared__ int pre[kBlock + 1];
+  __shared__ unsigned short act[kBlock];
+  __shared__ int wsum[kBlock / 64];
+  __shared__ double fm[NB][6];
   if (frozen(d)) return;
-  const int lane = threadIdx.x & 63;
-  const int gl = lane & (L - 1), sub = lane / L;
-  const int wpb = (int)(blockDim.x >> 6);
-  const int G = d.gather_groups;  // slot groups per body wavefront (1..L)
-  const int NB = kPer * G;        // bodies per body wavefront
-  const int body_waves = (d.nb + NB - 1) / NB;
-  const int waves = body_waves + (d.nhch + kPer - 1) / kPer;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const bool rst = guard && guard_reset(d);
   GuardAcc ga;
   ga.kp = 0ull;
   ga.kw = ~0ull;
-  for (TileLoop T = xcd_tiles((waves + wpb - 1) / wpb); T.t < T.end; T.t += T.step) {
-    const int wave = (int)((T.t * (unsigned)blockDim.x + threadIdx.x) >> 6);
-    if (wave >= body_waves) {
-      const int c = (wave - body_waves) * kPer + sub;
-      const bool run = c < d.nhch;
-      int2 r = make_int2(0, 0);
-      if (run) r = d.hch[c];
-      const double sc = sum_slots<L>(d, run, r.x, r.y, gl, -0.0);
-      if (run && gl < 6) d.hpart[6 * (size_t)c + gl] = sc;
-      continue;
+  const int nchunk = (d.nhch + kBlock / 64 - 1) / (kBlock / 64);
+  const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
+  const bool driven = tile < d.nDriven, chunks = !driven && tile < d.nDriven + nchunk;
+  const int b0 = driven ? tile : d.nDriven + (tile - d.nDriven - nchunk) * NB;
+  const int nbk = driven ? 1 : min(NB, d.nb - b0);
+  int k0 = 0, kend = 0;
+  if (chunks) {
+    const int c = (tile - d.nDriven) * (kBlock / 64) + wv;
+    if (c < d.nhch) {
+      const int2 r = d.hch[c];
+      const double s = sum_chunk(d, r.x, r.y, lane, vals + 64 * 6 * wv);
+      if (lane < 6) d.hpart[6 * (size_t)c + lane] = s;
     }
-    const int b = wave * NB + lane;
-    int k0 = 0, k1 = 0, c0 = 0, c1 = 0;
-    bool run = false, driven = false;
-    if (lane < NB && b < d.nb) {
-      k0 = d.soff[b];
-      k1 = d.soff[b + 1];
-      run = (k1 - k0) <= d.heavy_min;
+  } else {
+    k0 = d.soff[b0];
+    kend = d.soff[b0 + nbk];
+  }
+  if (chunks || (driven && kend - k0 > d.heavy_min)) {  // no body to finish
+    if (guard && t == 0) {
+      d.gpart[2 * (size_t)blockIdx.x] = ga.kp;
+      d.gpart[2 * (size_t)blockIdx.x + 1] = ga.kw;
     }
-    v3 F = V(0.0, 0.0, 0.0), M = V(0.0, 0.0, 0.0);
-    BodyKin P;
-    double mb = 0.0;
-    v3 Ib = V(0.0, 0.0, 0.0);
-    if (run) {
-      // the body's state, mass and inertia are loaded before the sums, so
-      // that their latency overlaps the slot loads
-      P = d.kin[b];
-      mb = d.mass[b];
-      Ib = ld3(d.inertia + 3 * (size_t)b);
-      driven = b < d.nDriven;
-      init_resultants<BF>(d, b, P, driven, F, M, c0, c1);
+    return;
+  }
+  // the records, and what finishing a body needs, ahead of the sums
+  d2* kd = reinterpret_cast<d2*>(d.kin + b0);
+  for (int k = t; k < 8 * nbk; k += kBlock) {
+    const d2 x = kd[k];
+    double* r = rec + (k >> 3) * kRec + 2 * (k & 7);
+    r[0] = x.x;
+    r[1] = x.y;
+  }
+  const int b = b0 + t;
+  double mb = 1.0;
+  v3 Ib = V(1.0, 1.0, 1.0);
+  bool run = false;
+  if (t < nbk) {
+    mb = d.mass[b];
+    Ib = ld3(d.inertia + 3 * (size_t)b);
+    run = d.soff[b + 1] - d.soff[b] <= d.heavy_min;
+  }
+  // the summing lanes' bodies and slot ranges
+  const int lb = t / kLanes, lc = t % kLanes;
+  const bool sums = lb < nbk && lc * kComp < 6;
+  const int sb0 = sums ? d.soff[b0 + lb] : 0, sb1 = sums ? d.soff[b0 + lb + 1] : 0;
+  __syncthreads();
+  int c0 = 0, c1 = 0;
+  if (t < nbk) {
+    v3 F, M;
+    init_resultants<BF>(d, b, rec_load(rec + t * kRec), driven, F, M, c0, c1);
+    fm[t][0] = F.x;
+    fm[t][1] = F.y;
+    fm[t][2] = F.z;
+    fm[t][3] = M.x;
+    fm[t][4] = M.y;
+    fm[t][5] = M.z;
+  }
+  double s[kComp];
+  bool first = true;
+  for (int w0 = k0 & ~15; w0 < kend; w0 += kGatherWin) {
+    const int pos = w0 + 16 * t;
+    unsigned m = 0u;
+    if (pos < kend) {
+      const uint4 x = *reinterpret_cast<const uint4*>(d.sact + pos);
+      m = byte_bits(x.x) | byte_bits(x.y) << 4 | byte_bits(x.z) << 8 | byte_bits(x.w) << 12;
+      if (pos < k0) m &= 0xffffu << (k0 - pos);
+      if (pos + 16 > kend) m &= 0xffffu >> (pos + 16 - kend);
     }
-    const unsigned long long busy = __ballot(run && k1 > k0);
-    for (int g = 0; g < G; g++) {
-      if (((busy >> (g * kPer)) & ((1ull << kPer) - 1ull)) == 0ull) continue;  // uniform
-      // lane (sub, gl) sums component gl of body lane g kPer + sub
-      const int src = g * kPer + sub;
-      const int s0 = __shfl(k0, src), s1 = __shfl(k1, src);
-      const bool r2 = __shfl(run ? 1 : 0, src) != 0;
-      const v3 Fs = V(__shfl(F.x, src), __shfl(F.y, src), __shfl(F.z, src));
-      const v3 Ms = V(__shfl(M.x, src), __shfl(M.y, src), __shfl(M.z, src));
-      const double sg = sum_slots<L>(d, r2, s0, s1, gl, pick(Fs, Ms, gl < 6 ? gl : 0));
-      // back to the body lanes of group g: component c of body lane l is in
-      // lane (l - g kPer) L + c
-      const int base = (lane & (kPer - 1)) * L;
-      const double fx = __shfl(sg, base), fy = __shfl(sg, base + 1), fz = __shfl(sg, base + 2);
-      const double mx = __shfl(sg, base + 3), my = __shfl(sg, base + 4), mz = __shfl(sg, base + 5);
-      if (lane / kPer == g) {
-        F = V(fx, fy, fz);
-        M = V(mx, my, mz);
+    int incl = __popc(m);
+    const int mine = incl;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += y;
+    }
+    if (lane == 63) wsum[wv] = incl;
+    __syncthreads();
+    int base = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; w++) {
+      base += w < wv ? wsum[w] : 0;
+      total += wsum[w];
+    }
+    int r = base + incl - mine;
+    pre[t] = r;
+    act[t] = (unsigned short)m;
+    if (t == 0) pre[kBlock] = total;
+    for (unsigned rest = m; rest; rest &= rest - 1u) list[r++] = (unsigned short)(16 * t + __ffs((int)rest) - 1);
+    __syncthreads();
+    // ranks of a body's slots within the window's list
+    auto rank = [&](int k) -> int {
+      const int q = min(max(k - w0, 0), kGatherWin);
+      if (q == kGatherWin) return pre[kBlock];
+      return pre[q >> 4] + __popc((unsigned)act[q >> 4] & ((1u << (q & 15)) - 1u));
+    };
+    int lo = 0, hi = 0;
+    if (sums) {
+      if (first)
+#pragma unroll
+        for (int c = 0; c < kComp; c++) s[c] = fm[lb][lc * kComp + c];
+      lo = rank(sb0);
+      hi = rank(sb1);
+    }
+    first = false;
+    for (int p0 = 0; p0 < total; p0 += kGatherCap) {
+      const int n = min(kGatherCap, total - p0);
+      d2 v[2][3];
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        if (t + h * kBlock < n) {
+          const d2* x =
+              reinterpret_cast<const d2*>(d.sval + 6 * (size_t)(w0 + (int)list[p0 + t + h * kBlock]));
+#pragma unroll
+          for (int q = 0; q < 3; q++) v[h][q] = x[q];
+        }
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        if (t + h * kBlock < n) {
+          d2* x = reinterpret_cast<d2*>(vals + 6 * (t + h * kBlock));
+#pragma unroll
+          for (int q = 0; q < 3; q++) x[q] = v[h][q];
+        }
+      __syncthreads();
+      if (sums) {
+        const int e = min(hi - p0, n);
+        const double* x = vals + lc * kComp;
+#pragma unroll 4
+        for (int q = max(lo - p0, 0); q < e; q++)
+#pragma unroll
+          for (int c = 0; c < kComp; c++) s[c] += x[6 * q + c];
       }
-    }
-    if (run) {
-      finish_body(d, sp, kick, b, P, driven, F, M, c0, c1, mb, Ib);
-      if (guard) guard_body(d, sp, b, P, rst, ga);
+      __syncthreads();
     }
   }
+  if (sums && !first)
+#pragma unroll
+    for (int c = 0; c < kComp; c++) fm[lb][lc * kComp + c] = s[c];
+  __syncthreads();
+  if (run) {
+    BodyKin P = rec_load(rec + t * kRec);  // (again: not held in registers over the sums)
+    const v3 F = V(fm[t][0], fm[t][1], fm[t][2]), M = V(fm[t][3], fm[t][4], fm[t][5]);
+    v3 acc, arot;
+    accelerate(d, sp, kick, P, driven, F, M, c0, c1, mb, Ib, acc, arot);
+    store_resultants(d, b, F, M, acc, arot);
+    if (guard) guard_body(d, sp, b, P, rst, ga);
+    if (kick) rec_store_motion(rec + t * kRec, P);
+  }
+  __syncthreads();
+  if (kick)
+    for (int k = t; k < 8 * nbk; k += kBlock) {
+      const double* r = rec + (k >> 3) * kRec + 2 * (k & 7);
+      kd[k] = d2{r[0], r[1]};
+    }
   if (!guard) return;
+  // only the threads t < NB (the first wavefront) finish bodies
+  static_assert(NB <= 64, "the first wavefront finishes the bodies");
   for (int off = 32; off > 0; off >>= 1) {
     const unsigned long long op = __shfl_xor(ga.kp, off, 64), ow = __shfl_xor(ga.kw, off, 64);
     ga.kp = op > ga.kp ? op : ga.kp;
     ga.kw = ow < ga.kw ? ow : ga.kw;
   }
-  const int wv = threadIdx.x >> 6;
-  if (lane == 0) {
-    red[0][wv] = ga.kp;
-    red[1][wv] = ga.kw;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 1; k < wpb; k++) {
-      ga.kp = red[0][k] > ga.kp ? red[0][k] : ga.kp;
-      ga.kw = red[1][k] < ga.kw ? red[1][k] : ga.kw;
-    }
+  if (t == 0) {
     d.gpart[2 * (size_t)blockIdx.x] = ga.kp;
     d.gpart[2 * (size_t)blockIdx.x + 1] = ga.kw;
   }
@@ -1651,51 +1836,6 @@ __device__ void drive_controls_block(const Dev& d, const StepParams& sp) {
   }
 }
 
-// predict_free: the new pose and velocities of free body b (Rockable.cpp:
-// 2036-2055) in P; store_predicted writes them back
-__device__ __forceinline__ void predict_free_with(const StepParams& sp, BodyKin& P, v3 a, v3 ar) {
-  v3 pos = vadd(kpos(P), vadd(vsc(sp.dt, kvel(P)), vsc(sp.dt2_2, a)));
-  v3 vel = vadd(kvel(P), vsc(sp.dt_2, a));
-  qt Q = kq(P);
-  const v3 w = kvrot(P);
-  Q = qadd_scaled(Q, qdot(Q, w), sp.dt);
-  Q = qadd_scaled(Q, qddot(Q, w, ar), sp.dt2_2);
-  qnormalize(&Q);
-  v3 w2 = vadd(w, vsc(sp.dt_2, ar));
-  P.px = pos.x;
-  P.py = pos.y;
-  P.pz = pos.z;
-  P.qw = Q.w;
-  P.qx = Q.x;
-  P.qy = Q.y;
-  P.qz = Q.z;
-  P.vx = vel.x;
-  P.vy = vel.y;
-  P.vz = vel.z;
-  P.wx = w2.x;
-  P.wy = w2.y;
-  P.wz = w2.z;
-}
-__device__ __forceinline__ void predict_free(const Dev& d, const StepParams& sp, int b, BodyKin& P) {
-  predict_free_with(sp, P, ld3(d.acc + 3 * (size_t)b), ld3(d.arot + 3 * (size_t)b));
-}
-// The far-entry skip's motion bound of one predicted body: no vertex of it
-// moved by more than |dx| + 2 |dQ| rmax in this step (for unit quaternions
-// |Q' v Q'* - Q v Q*| <= 2 |Q' - Q| |v|), plus a rounding allowance.
-__device__ __forceinline__ void add_motion_bound_with(const Dev& d, int b, const BodyKin& old, const BodyKin& P,
-                                                      double cb, double rmax) {
-  if (!d.skip_far) return;
-  const double dx = P.px - old.px, dy = P.py - old.py, dz = P.pz - old.pz;
-  const double qw = P.qw - old.qw, qx = P.qx - old.qx, qy = P.qy - old.qy, qz = P.qz - old.qz;
-  const double step = sqrt(dx * dx + dy * dy + dz * dz) + 2.0 * sqrt(qw * qw + qx * qx + qy * qy + qz * qz) * rmax;
-  const double mag = fabs(P.px) + fabs(P.py) + fabs(P.pz);
-  d.cbound[b] = cb + (step + 1e-15 * (1.0 + mag));
-}
-__device__ __forceinline__ void add_motion_bound(const Dev& d, int b, const BodyKin& old, const BodyKin& P) {
-  if (!d.skip_far) return;
-  add_motion_bound_with(d, b, old, P, d.cbound[b], d.rmax[b]);
-}
-
 __device__ __forceinline__ void store_predicted(const Dev& d, int b, const BodyKin& P) {
   BodyKin* out = d.kin + b;
   out->px = P.px;
@@ -1745,11 +1885,9 @@ __global__ void __launch_bounds__(kBlock) k_predict(Dev d, StepParams sp, int gl
 // driven_glob, workgroup 0 then writes their listed global vertices (else
 // k_glob does after this kernel).
 __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, int driven_glob) {
-  constexpr int kRec = 17;          // LDS doubles per record
   __shared__ double rec[64 * kRec];
   __shared__ double pose[64][8];    // px py pz qw qx qy qz h
   __shared__ int shp[64];           // shape, or -1 if the body is not listed
-  static_assert(sizeof(BodyKin) == 16 * sizeof(double), "a body record is 16 doubles");
   if (frozen(d)) return;
   const int t = threadIdx.x;
   if (blockIdx.x == 0) {
@@ -1792,39 +1930,10 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
       shp[t] = -1;
       if (b < bend) {
         double* r = rec + t * kRec;
-        BodyKin P;
-        P.px = r[0];
-        P.py = r[1];
-        P.pz = r[2];
-        P.qw = r[3];
-        P.qx = r[4];
-        P.qy = r[5];
-        P.qz = r[6];
-        P.vx = r[7];
-        P.vy = r[8];
-        P.vz = r[9];
-        P.wx = r[10];
-        P.wy = r[11];
-        P.wz = r[12];
-        P.R = r[13];
-        P.h = r[14];
-        P.shape = __double2loint(r[15]);
-        P.group = __double2hiint(r[15]);
+        BodyKin P = rec_load(r);
         const BodyKin old = P;
         predict_free_with(sp, P, acc, arot);
-        r[0] = P.px;
-        r[1] = P.py;
-        r[2] = P.pz;
-        r[3] = P.qw;
-        r[4] = P.qx;
-        r[5] = P.qy;
-        r[6] = P.qz;
-        r[7] = P.vx;
-        r[8] = P.vy;
-        r[9] = P.vz;
-        r[10] = P.wx;
-        r[11] = P.wy;
-        r[12] = P.wz;
+        rec_store_motion(r, P);
         add_motion_bound_with(d, b, old, P, cb, rmx);
         if (listed) {
           pose[t][0] = P.px;
@@ -2077,33 +2186,35 @@ void launch_interact(const Dev& d, const StepParams& sp, int write_geom_all, hip
     hipLaunchKernelGGL(k_law<LAW_DEFAULT>, gl, bl, 0, s, d, sp, write_geom_all, 0, ngeom, W);
 }
 
-// k_gather's workgroups: 64 / lanes x gather_groups bodies per body
-// wavefront, 64 / lanes heavy chunks per chunk wavefront, gather_waves
-// wavefronts per workgroup
+// k_gather's free bodies per workgroup: 32, so that a small packing spreads
+// over more workgroups and a bonded body's many terms fit one LDS pass; 64
+// from 131 072 bodies, where workgroups abound and the lanes that finish
+// the bodies count.
+constexpr int kGatherLarge = 1 << 17;
+int gather_bodies(const Dev& d) { return d.nb - d.nDriven >= kGatherLarge ? 64 : 32; }
+
+// k_gather's workgroups: one per driven body, the heavy chunks four to one,
+// the free bodies
 int gather_blocks(const Dev& d) {
-  const int per = d.gather_lanes == 8 ? 8 : 4;
-  const long nbw = (long)per * d.gather_groups;
-  const long waves = ((long)d.nb + nbw - 1) / nbw + ((long)d.nhch + per - 1) / per;
-  const int wpb = d.gather_waves == 1 || d.gather_waves == 2 ? d.gather_waves : 4;
-  return (int)grid_for(d, (waves + wpb - 1) / wpb).x;
+  const int nb = gather_bodies(d);
+  return d.nDriven + (d.nhch + 3) / 4 + (d.nb - d.nDriven + nb - 1) / nb;
 }
 
-int gather_blocks_max(int nb, int nhch) { return (nb + 3) / 4 + (nhch + 3) / 4 + 8; }
+int gather_blocks_max(int nb, int nhch) { return nb + (nhch + 3) / 4 + 8; }
 
 void launch_gather(const Dev& d, const StepParams& sp, int kick, int guard, hipStream_t s) {
   if (d.nb <= 0) return;
   guard = guard && kick;
-  const int wpb = d.gather_waves == 1 || d.gather_waves == 2 ? d.gather_waves : 4;
   const dim3 blocks(gather_blocks(d));
-  const bool bf = d.bf != BF_NONE;
-  if (d.gather_lanes == 8 && bf)
-    hipLaunchKernelGGL((k_gather<8, true>), blocks, dim3(64 * wpb), 0, s, d, sp, kick, guard);
-  else if (d.gather_lanes == 8)
-    hipLaunchKernelGGL((k_gather<8, false>), blocks, dim3(64 * wpb), 0, s, d, sp, kick, guard);
+  const bool bf = d.bf != BF_NONE, large = gather_bodies(d) == 64;
+  if (large && bf)
+    hipLaunchKernelGGL((k_gather<64, true>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard);
+  else if (large)
+    hipLaunchKernelGGL((k_gather<64, false>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard);
   else if (bf)
-    hipLaunchKernelGGL((k_gather<16, true>), blocks, dim3(64 * wpb), 0, s, d, sp, kick, guard);
+    hipLaunchKernelGGL((k_gather<32, true>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard);
   else
-    hipLaunchKernelGGL((k_gather<16, false>), blocks, dim3(64 * wpb), 0, s, d, sp, kick, guard);
+    hipLaunchKernelGGL((k_gather<32, false>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard);
   if (d.nheavy > 0) {
     hipLaunchKernelGGL(k_heavy_finish, grid_for(d, d.nheavy), dim3(kBlock), 0, s, d, sp, kick, guard);
     if (d.nheavy_exact > 0)
