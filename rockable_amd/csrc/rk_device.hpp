@@ -334,8 +334,12 @@ void launch_refresh_gaps(const Dev& d, hipStream_t s);
 // Every entry evaluated at the next step (after the poses were set from outside).
 void launch_reset_keys(const Dev& d, hipStream_t s);
 // kick: the closing half kick; guard: also the displacement check's
-// accumulation (k_guard_check then follows)
-void launch_gather(const Dev& d, const StepParams& sp, int kick, int guard, hipStream_t s);
+// accumulation (k_guard_check then follows); fuse: the free bodies also take
+// the next step's predictor, unless a rebuild falls due after this one
+// (launch_drive then follows, after the check)
+void launch_gather(const Dev& d, const StepParams& sp, int kick, int guard, int fuse, hipStream_t s);
+// the driven bodies' part of that predictor
+void launch_drive(const Dev& d, const StepParams& sp, hipStream_t s);
 // capacity of gpart for any launch shape
 int gather_blocks_max(int nb, int nhch);
 void launch_breakage(const Dev& d, const StepParams& sp, hipStream_t s);

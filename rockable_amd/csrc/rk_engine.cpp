@@ -149,6 +149,9 @@ struct rk_engine {
   int graph_steps = 0;
   int64_t pending = 0;
   bool pending_guard = false;
+  // the bodies already stand at the next step's predicted poses (within a run
+  // of steps only: its last step leaves them at its end)
+  bool predicted = false;
   struct StepGraph {
     std::vector<unsigned char> key;
     hipGraphExec_t exec = nullptr;
@@ -952,27 +955,31 @@ int account_breakage(rk_engine* eng) {
 // half kick of velocityVerletStep.  guard: a step of the guarded loop (the
 // guard kernel follows; it turns a breakage into a freeze that the host
 // reads with the guard); other calls account a breakage at once.
-int run_accelerations(rk_engine* eng, int kick, int write_geom, bool guard = false) {
+// fuse: the next step's predictor runs with the resultants.
+int run_accelerations(rk_engine* eng, int kick, int write_geom, bool guard = false, bool fuse = false) {
   const StepParams sp = step_params(eng);
   ensure_gv(eng, false);
   tic(eng, 1);
   tic(eng, 2);
   launch_interact(eng->d, sp, write_geom || eng->record_geometry, eng->stream);
   toc(eng, "interact", 2);
-  tic(eng, 2);
-  launch_gather(eng->d, sp, kick, guard && eng->d.disp_check ? 1 : 0, eng->stream);
-  toc(eng, "gather", 2);
-  toc(eng, "force", 1);
-  if (eng->m.law == LAW_STICKED && eng->live_interfaces > 0) {
+  const bool bonds = eng->m.law == LAW_STICKED && eng->live_interfaces > 0;
+  if (bonds) {
+    // before the resultants (it touches the bonds' state, which they do not
+    // read), so that their fused predictor knows of a breakage
     tic(eng, 2);
     launch_breakage(eng->d, sp, eng->stream);
     toc(eng, "breakage", 2);
-    if (!guard) {
-      int32_t fl = 0;
-      HIPCHK(hipMemcpyAsync(&fl, eng->flags, sizeof(int32_t), hipMemcpyDeviceToHost, eng->stream));
-      HIPCHK(hipStreamSynchronize(eng->stream));
-      if (fl && account_breakage(eng) != 0) return -1;
-    }
+  }
+  tic(eng, 2);
+  launch_gather(eng->d, sp, kick, guard && eng->d.disp_check ? 1 : 0, fuse ? 1 : 0, eng->stream);
+  toc(eng, "gather", 2);
+  toc(eng, "force", 1);
+  if (bonds && !guard) {
+    int32_t fl = 0;
+    HIPCHK(hipMemcpyAsync(&fl, eng->flags, sizeof(int32_t), hipMemcpyDeviceToHost, eng->stream));
+    HIPCHK(hipStreamSynchronize(eng->stream));
+    if (fl && account_breakage(eng) != 0) return -1;
   }
   HIPCHK(hipGetLastError());
   return 0;
@@ -1009,33 +1016,53 @@ int do_update_nl(rk_engine* eng) {
   return 0;
 }
 
+// Whether the next step's predictor may run with this step's resultants: the
+// resultant kernel finishes every free body (none is left to the serial
+// heavy-body kernel), the controls need no host value (servo_timed), and no
+// host action can fall between the steps (bonds without the guard).
+bool can_fuse(const rk_engine* eng, bool guard) {
+  return eng->d.soff && eng->d.nheavy_exact == 0 && !eng->m.servo_timed() &&
+         (guard || !(eng->m.law == LAW_STICKED && eng->live_interfaces > 0));
+}
+
 // guard: the step ends with the guard kernel (the displacement check of
 // dynamicUpdateNL, its accumulation fused into the resultant kernels, and
-// the freeze after a bond breakage)
-int vv_step(rk_engine* eng, int write_geom, bool guard) {
+// the freeze after a bond breakage).  next: another step follows with no host
+// action in between, so that its predictor may run with this one's
+// resultants; eng->predicted then tells it.  After the last step of a run the
+// bodies are at its end.
+int vv_step(rk_engine* eng, int write_geom, bool guard, bool next) {
   const StepParams sp = step_params(eng);
   if (guard && !eng->guard) return fail(eng, "device guard: not allocated");
   if (guard && eng->d.disp_check && eng->gpart_cap < gather_blocks_max(eng->d.nb, eng->d.nhch))
     return fail(eng, "device guard: no room for the gather's maxima");
-  tic(eng, 2);
-  launch_predict(eng->d, sp, 1, eng->stream);
-  toc(eng, "predict", 2);
-  // the predictor leaves the listed bodies' global vertices current (every
-  // body's while there is no list)
-  eng->gv_state = eng->d.soff ? rk_engine::GV_LISTED : rk_engine::GV_ALL;
-  if (run_accelerations(eng, 1, write_geom, guard) != 0) return -1;
+  if (!eng->predicted) {
+    tic(eng, 2);
+    launch_predict(eng->d, sp, 1, eng->stream);
+    toc(eng, "predict", 2);
+    // the predictor leaves the listed bodies' global vertices current (every
+    // body's while there is no list)
+    eng->gv_state = eng->d.soff ? rk_engine::GV_LISTED : rk_engine::GV_ALL;
+  }
+  const bool fuse = next && can_fuse(eng, guard);
+  eng->predicted = fuse;
+  if (run_accelerations(eng, 1, write_geom, guard, fuse) != 0) return -1;
   if (guard) {
     tic(eng, 2);
     launch_guard(eng->d, eng->stream);
     toc(eng, "guard", 2);
+  }
+  if (fuse) {
+    launch_drive(eng->d, sp, eng->stream);
+    eng->gv_state = rk_engine::GV_LISTED;
   }
   return 0;
 }
 
 // One step of the loop as the device runs it (write_geom 0): the
 // velocity-Verlet step, and the guard kernel in the guarded loop.
-int launch_one_step(rk_engine* eng, bool with_guard) {
-  return vv_step(eng, 0, with_guard);
+int launch_one_step(rk_engine* eng, bool with_guard, bool next) {
+  return vv_step(eng, 0, with_guard, next);
 }
 
 // What a captured run of steps depends on: the device view (pointers and
@@ -1065,7 +1092,7 @@ int step_graph(rk_engine* eng, int n, bool with_guard, hipGraphExec_t* out) {
     }
   HIPCHK(hipStreamBeginCapture(eng->stream, hipStreamCaptureModeThreadLocal));
   int rc = 0;
-  for (int k = 0; k < n && rc == 0; k++) rc = launch_one_step(eng, with_guard);
+  for (int k = 0; k < n && rc == 0; k++) rc = launch_one_step(eng, with_guard, k + 1 < n);
   hipGraph_t graph = nullptr;
   const hipError_t ec = hipStreamEndCapture(eng->stream, &graph);
   eng->gv_state = rk_engine::GV_LISTED;  // each step of the graph ends with the listed bodies' fresh
@@ -1136,20 +1163,20 @@ int flush_steps(rk_engine* eng) {
     eng->gv_state = rk_engine::GV_LISTED;
   }
   for (; n > 0; n--)
-    if (launch_one_step(eng, with_guard) != 0) return -1;
+    if (launch_one_step(eng, with_guard, n > 1) != 0) return -1;
   return 0;
 }
 
 // One step of the loop from the host's side: deferred when nothing on the
 // host depends on it (no conf file written at it, no bonds outside the
 // guarded loop, whose breakage the host accounts after the step), launched
-// now otherwise.
-int enqueue_step(rk_engine* eng, bool write_geom, bool with_guard) {
+// now otherwise.  next: no host action follows before the next step.
+int enqueue_step(rk_engine* eng, bool write_geom, bool with_guard, bool next) {
   const bool bonds = !with_guard && eng->m.law == LAW_STICKED && eng->live_interfaces > 0;
   if (eng->pending > 0 && eng->pending_guard != with_guard && flush_steps(eng) != 0) return -1;
   if (write_geom || bonds || eng->graph_steps <= 1 || eng->m.servo_timed()) {
     if (flush_steps(eng) != 0) return -1;
-    return vv_step(eng, write_geom ? 1 : 0, with_guard);
+    return vv_step(eng, write_geom ? 1 : 0, with_guard, next && eng->graph_steps <= 1);
   }
   eng->pending_guard = with_guard;
   eng->pending++;
@@ -1461,8 +1488,9 @@ int reread_driving(rk_engine* eng) {
   return upload_controls(eng);
 }
 
-// one iteration of the integrate() loop (Rockable.cpp:2584-2745)
-int loop_body(rk_engine* eng, const char* outdir) {
+// one iteration of the integrate() loop (Rockable.cpp:2584-2745); more:
+// another one follows
+int loop_body(rk_engine* eng, const char* outdir, bool more) {
   Model& m = eng->m;
   m.t += m.dt;
   m.interConfC += m.dt;
@@ -1470,7 +1498,8 @@ int loop_body(rk_engine* eng, const char* outdir) {
   const bool conf_due = m.interConfC >= m.interConf - m.dt_2;
   bool rec_geo = false;
   const bool rec = outdir && record_due(eng, &rec_geo);
-  if (enqueue_step(eng, (conf_due && outdir) || rec_geo, false) != 0) return -1;
+  const bool rebuild = eng->needUpdate || m.interVerletC >= m.interVerlet - m.dt_2;
+  if (enqueue_step(eng, (conf_due && outdir) || rec_geo, false, more && !conf_due && !rec && !rebuild) != 0) return -1;
   eng->steps++;
   if (conf_due) {
     m.iconf++;
@@ -1619,7 +1648,9 @@ int run_guarded(rk_engine* eng, const char* outdir, int64_t nmax, bool until_tma
       const bool conf_due = m.interConfC >= m.interConf - m.dt_2;
       bool rec_geo = false;
       const bool rec = outdir && record_due(eng, &rec_geo);
-      if (enqueue_step(eng, (conf_due && outdir) || rec_geo, true) != 0) return -1;
+      const bool last = (conf_due && (outdir || !m.driving_path.empty())) || rec || eng->needUpdate ||
+                        m.interVerletC >= m.interVerlet - m.dt_2 || (until_tmax && m.t > m.tmax) || k + 1 >= B;
+      if (enqueue_step(eng, (conf_due && outdir) || rec_geo, true, !last) != 0) return -1;
       eng->steps++;
       if (conf_due) {
         m.iconf++;
@@ -1629,9 +1660,7 @@ int run_guarded(rk_engine* eng, const char* outdir, int64_t nmax, bool until_tma
       hist.push_back(loop_scalars(eng));
       conf_at.push_back(conf_due ? 1 : 0);
       k++;
-      if ((conf_due && (outdir || !m.driving_path.empty())) || rec || eng->needUpdate ||
-          m.interVerletC >= m.interVerlet - m.dt_2 || (until_tmax && m.t > m.tmax))
-        break;
+      if (last) break;
       if (pipe && eng->note) {
         const volatile HostNote* n = eng->note;
         if (n->frozen) break;
@@ -1684,6 +1713,7 @@ int run_guarded(rk_engine* eng, const char* outdir, int64_t nmax, bool until_tma
       executed = g.frozen_step - hist[0].steps + 1;
       if (executed < 1 || executed > k) return fail(eng, "device guard: inconsistent frozen step");
       set_loop_scalars(eng, hist[executed]);
+      eng->predicted = false;  // the frozen step's resultants took no predictor
       eng->guard_wasted += k - executed;
       if (eng->model && k - executed > 1) eng->model_trust = std::max(0.05, eng->model_trust * 0.7);
       need = true;
@@ -1823,6 +1853,7 @@ void reset_engine(rk_engine* eng) {
   eng->loaded = false;
   eng->cur = 0;
   eng->needUpdate = false;
+  eng->predicted = false;
   eng->steps = 0;
   eng->nl_updates = 0;
   eng->packings.clear();
@@ -2162,7 +2193,7 @@ int rk_step(rk_engine* eng, int64_t nsteps) {
   if (integrate_prepare(eng, false) != 0) return -1;
   if (eng->guard) return run_guarded(eng, nullptr, nsteps, false, nullptr);
   for (int64_t k = 0; k < nsteps; k++)
-    if (loop_body(eng, nullptr) != 0) return -1;
+    if (loop_body(eng, nullptr, k + 1 < nsteps) != 0) return -1;
   return flush_steps(eng);
 }
 
@@ -2390,7 +2421,8 @@ int rk_integrate(rk_engine* eng, const char* outdir, int64_t max_steps, int64_t*
     if (run_guarded(eng, outdir, max_steps < 0 ? INT64_MAX : max_steps, true, &n) != 0) return -1;
   } else {
     while (eng->m.t <= eng->m.tmax && (max_steps < 0 || n < max_steps)) {
-      if (loop_body(eng, outdir) != 0) return -1;
+      const bool more = eng->m.t + eng->m.dt <= eng->m.tmax && (max_steps < 0 || n + 1 < max_steps);
+      if (loop_body(eng, outdir, more) != 0) return -1;
       n++;
     }
     if (flush_steps(eng) != 0) return -1;

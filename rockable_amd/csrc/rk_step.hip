@@ -1039,6 +1039,11 @@ __device__ __forceinline__ void guard_body(const Dev& d, const StepParams& sp, i
     a.kw = k2 < a.kw ? k2 : a.kw;
   }
 }
+// A rebuild falls due after the current step: the check of the step before
+// asked for it, or a bond broke in this one.
+__device__ __forceinline__ bool rebuild_due(const Dev& d) {
+  return d.guard_on && (*(volatile const int*)&d.guard->nu != 0 || *(volatile const int*)d.flags != 0);
+}
 __device__ __forceinline__ bool guard_reset(const Dev& d) { return *(volatile const int*)&d.guard->reset != 0; }
 
 // predict_free: the new pose and velocities of free body b (Rockable.cpp:
@@ -1151,6 +1156,13 @@ __device__ __forceinline__ unsigned byte_bits(unsigned x) { return ((x & 0x01010
 // 15.7 us for 706 bodies, 22.6 us for 50 005, 40.3 us for 90 006 with the
 // displacement check, 13.7 us for 13 001 bonded cubes; now 6.6, 14.8, 23.4 and
 // 10.3 us.
+// With fuse the step after this one follows at once, and the free bodies take
+// its predictor (and their listed vertices) here, while their records and
+// accelerations are at hand: one launch and one pass over the records less,
+// and the resultants and accelerations, which only the predictor or a read-out
+// uses, are not stored.  Apart, the two kernels took 14.8 + 11.3 us for
+// 50 005 bodies, fused 22.4 us; 6.6 + 7.5 and 8.7 us for 706 bodies, where a
+// launch counts most.
 // Driven bodies come first, one workgroup each (a wall's many slots fill it);
 // then, a wavefront each, the 64-slot chunks of the heavy bodies, whose
 // partial sums (from -0.0, the identity of addition) k_heavy_finish takes.
@@ -1189,7 +1201,7 @@ __device__ __forceinline__ double sum_chunk(const Dev& d, int k0, int k1, int la
 }
 
 template <int NB, bool BF>  // BF: the deck has a body force
-__global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, int kick, int guard) {
+__global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, int kick, int guard, int fuse) {
   constexpr int kLanes = kBlock / NB;      // lanes per body in the sums (8 or 4)
   constexpr int kComp = kLanes >= 6 ? 1 : 2;  // components per lane
   __shared__ double rec[NB * kRec];
@@ -1202,6 +1214,8 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, int 
   if (frozen(d)) return;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const bool rst = guard && guard_reset(d);
+  // (the check that follows this step freezes the later ones on the same words)
+  const bool predict = fuse && !rebuild_due(d);
   GuardAcc ga;
   ga.kp = 0ull;
   ga.kw = ~0ull;
@@ -1238,13 +1252,17 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, int 
     r[1] = x.y;
   }
   const int b = b0 + t;
-  double mb = 1.0;
+  double mb = 1.0, cb = 0.0, rmx = 0.0;
   v3 Ib = V(1.0, 1.0, 1.0);
   bool run = false;
   if (t < nbk) {
     mb = d.mass[b];
     Ib = ld3(d.inertia + 3 * (size_t)b);
     run = d.soff[b + 1] - d.soff[b] <= d.heavy_min;
+    if (predict && d.skip_far) {
+      cb = d.cbound[b];
+      rmx = d.rmax[b];
+    }
   }
   // the summing lanes' bodies and slot ranges
   const int lb = t / kLanes, lc = t % kLanes;
@@ -1348,8 +1366,14 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, int 
     const v3 F = V(fm[t][0], fm[t][1], fm[t][2]), M = V(fm[t][3], fm[t][4], fm[t][5]);
     v3 acc, arot;
     accelerate(d, sp, kick, P, driven, F, M, c0, c1, mb, Ib, acc, arot);
-    store_resultants(d, b, F, M, acc, arot);
     if (guard) guard_body(d, sp, b, P, rst, ga);
+    if (predict && !driven) {
+      const BodyKin old = P;
+      predict_free_with(sp, P, acc, arot);
+      add_motion_bound_with(d, b, old, P, cb, rmx);
+    } else {
+      store_resultants(d, b, F, M, acc, arot);
+    }
     if (kick) rec_store_motion(rec + t * kRec, P);
   }
   __syncthreads();
@@ -1357,6 +1381,13 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, int 
     for (int k = t; k < 8 * nbk; k += kBlock) {
       const double* r = rec + (k >> 3) * kRec + 2 * (k & 7);
       kd[k] = d2{r[0], r[1]};
+    }
+  if (predict && !driven)
+    for (int k = d.bvoff[b0] + t; k < d.bvoff[b0 + nbk]; k += kBlock) {
+      const int bb = d.bvbody[k];
+      if (d.soff[bb + 1] == d.soff[bb]) continue;
+      const BodyKin P = rec_load(rec + (bb - b0) * kRec);
+      st3(d.gv + 3 * (size_t)k, glob_vertex(d.sh, P, k - d.bvoff[bb]));
     }
   if (!guard) return;
   // only the threads t < NB (the first wavefront) finish bodies
@@ -1853,6 +1884,22 @@ __device__ __forceinline__ void store_predicted(const Dev& d, int b, const BodyK
   out->wz = P.wz;
 }
 
+// The driven bodies of the next step, where the resultant kernel took the
+// free bodies' predictor: their controls, and their listed vertices (with
+// driven_glob; else k_glob follows).
+__global__ void __launch_bounds__(kBlock) k_drive(Dev d, StepParams sp, int driven_glob) {
+  if (frozen(d)) return;
+  drive_controls_block(d, sp);
+  if (!driven_glob) return;
+  __syncthreads();
+  for (int k = threadIdx.x; k < d.nvdriven; k += blockDim.x) {
+    const int b = d.bvbody[k];
+    if (d.soff[b + 1] == d.soff[b]) continue;
+    const BodyKin& P = d.kin[b];
+    st3(d.gv + 3 * (size_t)k, glob_vertex(d.sh, P, k - d.bvoff[b]));
+  }
+}
+
 // glob: also the global vertices of the free bodies with listed slots, from
 // the new pose (the driven bodies' follow in k_glob)
 __global__ void __launch_bounds__(kBlock) k_predict(Dev d, StepParams sp, int glob) {
@@ -2108,6 +2155,13 @@ void launch_predict(const Dev& d, const StepParams& sp, int glob, hipStream_t s)
   launch_glob(d, listed ? 0 : 1, fused ? d.nvdriven : d.nvtot, s);
 }
 
+void launch_drive(const Dev& d, const StepParams& sp, hipStream_t s) {
+  if (d.nctrl <= 0) return;  // no body moves by a control: poses and vertices stay
+  const int driven_glob = d.nvdriven <= 1024 ? 1 : 0;
+  hipLaunchKernelGGL(k_drive, dim3(1), dim3(kBlock), 0, s, d, sp, driven_glob);
+  if (!driven_glob) launch_glob(d, 0, d.nvdriven, s);
+}
+
 template <int BS>
 void launch_geom(const Dev& d, int write_geom_all, hipStream_t s) {
   const dim3 g = grid_for(d, (d.ne + BS - 1) / BS), bl(BS);
@@ -2202,19 +2256,19 @@ int gather_blocks(const Dev& d) {
 
 int gather_blocks_max(int nb, int nhch) { return nb + (nhch + 3) / 4 + 8; }
 
-void launch_gather(const Dev& d, const StepParams& sp, int kick, int guard, hipStream_t s) {
+void launch_gather(const Dev& d, const StepParams& sp, int kick, int guard, int fuse, hipStream_t s) {
   if (d.nb <= 0) return;
   guard = guard && kick;
   const dim3 blocks(gather_blocks(d));
   const bool bf = d.bf != BF_NONE, large = gather_bodies(d) == 64;
   if (large && bf)
-    hipLaunchKernelGGL((k_gather<64, true>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard);
+    hipLaunchKernelGGL((k_gather<64, true>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard, fuse);
   else if (large)
-    hipLaunchKernelGGL((k_gather<64, false>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard);
+    hipLaunchKernelGGL((k_gather<64, false>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard, fuse);
   else if (bf)
-    hipLaunchKernelGGL((k_gather<32, true>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard);
+    hipLaunchKernelGGL((k_gather<32, true>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard, fuse);
   else
-    hipLaunchKernelGGL((k_gather<32, false>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard);
+    hipLaunchKernelGGL((k_gather<32, false>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard, fuse);
   if (d.nheavy > 0) {
     hipLaunchKernelGGL(k_heavy_finish, grid_for(d, d.nheavy), dim3(kBlock), 0, s, d, sp, kick, guard);
     if (d.nheavy_exact > 0)
