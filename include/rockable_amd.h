@@ -155,9 +155,10 @@ int rk_set_body_force(rk_engine* eng, const char* name, const double* args, int 
  * entries, record_geometry 0, an inactive entry with zero history whose gap
  * is proven positive by the bodies' accumulated motion bounds is not
  * evaluated; its gap is recomputed when the list is read out or rebuilt;
- * 0: every listed entry every step), "skip_segment" (entries a workgroup
- * tests and compacts before evaluating them under skip_far: 512, 1024, 2048,
- * 4096; 256: no compaction; default 1024), "count_skips" (1: the geometry pass
+ * 0: every listed entry every step), "skip_segment" (512, 1024, 2048 or 4096:
+ * under skip_far the steps work from a list of the entries to evaluate, which
+ * the device writes anew when a body outruns its allowance; 256: every entry
+ * is tested at every step; default 1024), "count_skips" (1: the geometry pass
  * counts entries skipped, inactive with zero history, and looked at, read
  * back with rk_get_option as "skipped_entries", "zero_history_entries" and
  * "entries_looked_at"; setting it again clears them; 0 stops counting),

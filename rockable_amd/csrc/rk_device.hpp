@@ -100,6 +100,37 @@ struct DevGuard {
   long long step;              // index of the step the next check ends
 };
 
+// An entry on the evaluation list with what the step reads of it that does
+// not change until the list is rebuilt: its index and bodies, its contact
+// type (bits 0-1) and face's vertex count (from bit 2), the vertices of its
+// geometry in the shapes' table (VV i, j; VE i, j's edge; EE i's edge, j's
+// edge; VF i, the face's first three and last vertices), its bodies' place in
+// a parameter's group table (-1: none), its interface when the list was
+// written, its resultant slots and its damping.  Read densely from the list,
+// they cost 64 bytes and one latency; gathered from the entry arrays and the
+// shapes' tables, nearly every line of the former (one entry in five is
+// listed) and a chain of loads.
+struct alignas(16) ListItem {
+  int32_t e, i, j, kind;
+  int32_t v[4];
+  int32_t v4, gpair, stick, pad;
+  int2 slots;
+  double damp;
+};
+static_assert(sizeof(ListItem) == 64, "ListItem is four 16-byte loads");
+
+// The evaluation list (below, Dev::elist): the sizes of its eight parts in
+// the list in use (gen & 1) and the one a relisting step writes; want[p]: a
+// step of parity p has to test every entry and write the list anew; again:
+// the step after that one too (after a reset of the keys, which at first puts
+// every entry on the list).
+struct ListState {
+  int cnt[2][8];
+  int gen;
+  int want[2];
+  int again;
+};
+
 struct DevControl {
   int32_t type, i;
   double value;
@@ -184,9 +215,12 @@ struct Dev {
   int32_t* estick;
   uint8_t* eact;
   // Far-entry skip.  cbound[b] accumulates a bound on how far any vertex of
-  // body b has moved since the list was built (|dx| + 2 |dQ| rmax[b] per step,
-  // rmax the largest vertex distance from the body's centre; +inf for a
-  // driven body with a control).  An inactive entry with zero history keeps
+  // body b has moved (|dx - D| + 2 |dQ| rmax[b] per step, rmax the largest
+  // vertex distance from the body's centre; +inf for a driven body with a
+  // control) in a frame that moves by D = dt drift each step: two bodies' gap
+  // changes by no more than both their motions in any common frame, and
+  // in a flow most of the motion is common.  drift is the bodies' mean
+  // velocity when the list was built.  An inactive entry with zero history keeps
   // ekey = dn + cbound[i] + cbound[j] of the step it was last evaluated: its
   // gap cannot have fallen by more than the growth of cbound[i] + cbound[j]
   // since, so while ekey - cbound[i] - cbound[j] > kSkipMargin it is still
@@ -194,8 +228,23 @@ struct Dev {
   double* ekey;
   double* cbound;
   const double* rmax;
+  double* drift;          // 3
+  // The evaluation list: the entries that cannot be left alone, so that a
+  // step need not test the others.  When it is written, an entry is left out
+  // if its gap stays positive even with both bodies' bounds at ahead[b]
+  // (cbound[b] plus an allowance of some steps' motion); climit[b] keeps that
+  // value, and the list holds while cbound[b] <= climit[b] for every body.
+  // The predictor checks that and else has the next force phase test every
+  // entry and write the list anew.  Part x of elist (the tiles of XCD x)
+  // starts at the first entry of its tiles.
+  double* ahead;
+  double* climit;
+  double ahead_min;       // the smallest allowance
+  ListState* ls;
+  ListItem* elist;
+  int4* edesc_s;          // per entry: as edesc, with indices into the shapes' vertex table
   int skip_far;           // 1: skip such entries (only when the step writes no geometry of inactive entries)
-  int skip_seg;           // entries a workgroup tests and compacts before evaluating (512 ... 4096; else none)
+  int skip_seg;           // 512 or more: the evaluation list; else entries tested where they are evaluated
   // with the count_skips option: [0] entries skipped, [1] inactive entries
   // with zero history, [2] entries looked at, summed over the steps
   unsigned long long* skip_count;
@@ -322,24 +371,33 @@ inline int persistent_grid(int T, int persist) {
 // the entries' resolved vertex indices, after every change of the list
 void launch_entry_desc(const Dev& d, hipStream_t s);
 // the predictor; then the global vertices of the new poses: of the listed
-// bodies (glob), else of every body
-void launch_predict(const Dev& d, const StepParams& sp, int glob, hipStream_t s);
+// bodies, of every body, or of none.  par: the step's parity (ListState)
+enum { GLOB_ALL, GLOB_LISTED, GLOB_NONE };
+void launch_predict(const Dev& d, const StepParams& sp, int glob, int par, hipStream_t s);
 // all: every body's vertices; else those of the bodies with listed slots
 void launch_glob(const Dev& d, int all, hipStream_t s);
-void launch_interact(const Dev& d, const StepParams& sp, int write_geom_all, hipStream_t s);
+// whether a step takes the evaluation list (it then reads no global vertices)
+bool uses_list(const Dev& d, int write_geom_all);
+void launch_interact(const Dev& d, const StepParams& sp, int write_geom_all, int par, hipStream_t s);
 // The gap of every inactive entry with zero history from the current poses,
 // as the last step computed it (an entry the step skipped keeps an older gap
 // until then); before the list is read out.
 void launch_refresh_gaps(const Dev& d, hipStream_t s);
 // Every entry evaluated at the next step (after the poses were set from outside).
 void launch_reset_keys(const Dev& d, hipStream_t s);
+// The evaluation list written anew at the next step.
+void launch_reset_list(const Dev& d, hipStream_t s);
 // kick: the closing half kick; guard: also the displacement check's
 // accumulation (k_guard_check then follows); fuse: the free bodies also take
 // the next step's predictor, unless a rebuild falls due after this one
-// (launch_drive then follows, after the check)
-void launch_gather(const Dev& d, const StepParams& sp, int kick, int guard, int fuse, hipStream_t s);
+// (launch_drive then follows, after the check), with the global vertices
+// (GLOB_LISTED or GLOB_NONE); listed: this step took the evaluation list
+struct GatherArgs {
+  int kick, guard, fuse, glob, listed, par;
+};
+void launch_gather(const Dev& d, const StepParams& sp, GatherArgs a, hipStream_t s);
 // the driven bodies' part of that predictor
-void launch_drive(const Dev& d, const StepParams& sp, hipStream_t s);
+void launch_drive(const Dev& d, const StepParams& sp, int glob, hipStream_t s);
 // capacity of gpart for any launch shape
 int gather_blocks_max(int nb, int nhch);
 void launch_breakage(const Dev& d, const StepParams& sp, hipStream_t s);

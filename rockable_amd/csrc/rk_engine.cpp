@@ -71,6 +71,10 @@ struct rk_engine {
   double *acc = nullptr, *arot = nullptr, *force = nullptr, *moment = nullptr;
   double *mass = nullptr, *inertia = nullptr, *bf_surface = nullptr;
   double *cbound = nullptr, *rmax = nullptr;  // far-entry skip: per-body motion bounds
+  double *ahead = nullptr, *climit = nullptr;  // and the evaluation list's limits on them
+  double* drift = nullptr;
+  ListState* ls = nullptr;
+  int parity = 0;  // of the next step (ListState)
   int skip_far = 1;
   int skip_seg = 1024;  // entries tested and compacted per workgroup under the skip (256: no compaction)
   unsigned long long* skip_count = nullptr;  // count_skips: the geometry pass's counts
@@ -229,13 +233,14 @@ void free_device(rk_engine* eng) {
                 eng->ifc_key,  eng->ifc_istart, eng->ifc_par,  eng->ifc_inner, eng->ifc_alive, eng->ifc_bond_off, eng->ifc_bond_key,
                 eng->ifc_brk,  eng->ifc_broken, eng->ifc_nbroken, eng->ctrl,      eng->ctrl_off,  eng->ctrl_idx,  eng->flags,    eng->passive,
                 eng->gv,       eng->bvoff,     eng->bvbody,    eng->guard,     eng->gdpos,    eng->gdq,      eng->gpart,
-                eng->beoff,    eng->bfoff,     eng->cbound,    eng->rmax,
+                eng->beoff,    eng->bfoff,     eng->cbound,    eng->rmax,  eng->ahead, eng->climit, eng->drift, eng->ls,
                 eng->feat,     eng->pred,      eng->feat_part, eng->stat_part, eng->stat_out};
   for (void* p : ps)
     if (p) (void)hipFree(p);
   eng->kin = nullptr;
   eng->acc = eng->arot = eng->force = eng->moment = eng->mass = eng->inertia = eng->bf_surface = nullptr;
-  eng->cbound = eng->rmax = nullptr;
+  eng->cbound = eng->rmax = eng->ahead = eng->climit = eng->drift = nullptr;
+  eng->ls = nullptr;
   eng->cluster = nullptr;
   eng->sh_nv = eng->sh_ne = eng->sh_nf = eng->sh_voff = eng->sh_eoff = eng->sh_foff = eng->sh_edge = nullptr;
   eng->sh_fstart = eng->sh_fidx = nullptr;
@@ -397,6 +402,16 @@ void assemble_dev(rk_engine* eng) {
   d.ekey = E.ekey;
   d.cbound = eng->cbound;
   d.rmax = eng->rmax;
+  d.ahead = eng->ahead;
+  d.climit = eng->climit;
+  // a hundredth of the reach of the list's near tests: at 0.1 m/s and the
+  // configurations' steps some hundred steps of motion, for a few per cent
+  // more entries listed
+  d.ahead_min = 0.01 * m.dVerlet;
+  d.drift = eng->drift;
+  d.ls = eng->ls;
+  d.elist = E.elist;
+  d.edesc_s = E.edesc + E.n;
   d.skip_far = eng->skip_far;
   d.skip_count = eng->skip_count;
   d.skip_seg = eng->skip_seg;
@@ -666,7 +681,10 @@ int upload_model(rk_engine* eng) {
       for (const v3& v : m.shapes[m.bodies[b].shape].vertex) r2 = std::max(r2, v.x * v.x + v.y * v.y + v.z * v.z);
       rmax[b] = m.bodies[b].homothety * sqrt(r2);
     }
-    if (upload(eng, eng->rmax, rmax) || upload(eng, eng->cbound, initial_bounds(m))) return -1;
+    const std::vector<double> bounds = initial_bounds(m);
+    if (upload(eng, eng->rmax, rmax) || upload(eng, eng->cbound, bounds) || upload(eng, eng->ahead, bounds) ||
+        upload(eng, eng->climit, bounds) || upload(eng, eng->drift, std::vector<double>(3, 0.0)) || upload(eng, eng->ls, std::vector<ListState>(1, ListState{})))
+      return -1;
   }
   // global-vertex table: body b's vertices from bvoff[b]
   {
@@ -958,10 +976,13 @@ int account_breakage(rk_engine* eng) {
 // fuse: the next step's predictor runs with the resultants.
 int run_accelerations(rk_engine* eng, int kick, int write_geom, bool guard = false, bool fuse = false) {
   const StepParams sp = step_params(eng);
-  ensure_gv(eng, false);
+  const int geom_all = write_geom || eng->record_geometry;
+  // (the evaluation list is kept by the steps of the loop, whose predictor checks it)
+  const bool listed = kick && uses_list(eng->d, geom_all);
+  if (!listed) ensure_gv(eng, false);
   tic(eng, 1);
   tic(eng, 2);
-  launch_interact(eng->d, sp, write_geom || eng->record_geometry, eng->stream);
+  launch_interact(eng->d, sp, geom_all, eng->parity, eng->stream);
   toc(eng, "interact", 2);
   const bool bonds = eng->m.law == LAW_STICKED && eng->live_interfaces > 0;
   if (bonds) {
@@ -972,7 +993,14 @@ int run_accelerations(rk_engine* eng, int kick, int write_geom, bool guard = fal
     toc(eng, "breakage", 2);
   }
   tic(eng, 2);
-  launch_gather(eng->d, sp, kick, guard && eng->d.disp_check ? 1 : 0, fuse ? 1 : 0, eng->stream);
+  GatherArgs ga;
+  ga.kick = kick;
+  ga.guard = guard && eng->d.disp_check ? 1 : 0;
+  ga.fuse = fuse ? 1 : 0;
+  ga.glob = listed ? GLOB_NONE : GLOB_LISTED;
+  ga.listed = listed ? 1 : 0;
+  ga.par = eng->parity;
+  launch_gather(eng->d, sp, ga, eng->stream);
   toc(eng, "gather", 2);
   toc(eng, "force", 1);
   if (bonds && !guard) {
@@ -1036,13 +1064,17 @@ int vv_step(rk_engine* eng, int write_geom, bool guard, bool next) {
   if (guard && !eng->guard) return fail(eng, "device guard: not allocated");
   if (guard && eng->d.disp_check && eng->gpart_cap < gather_blocks_max(eng->d.nb, eng->d.nhch))
     return fail(eng, "device guard: no room for the gather's maxima");
+  // a step on the evaluation list reads no global vertices: the predictor
+  // leaves them stale (the same for the next step's, fused here), else those
+  // of the listed bodies current (every body's while there is no list)
+  const bool list = uses_list(eng->d, write_geom || eng->record_geometry);
+  const int glob = list ? GLOB_NONE : eng->d.soff ? GLOB_LISTED : GLOB_ALL;
+  const auto gv_after = list ? rk_engine::GV_STALE : eng->d.soff ? rk_engine::GV_LISTED : rk_engine::GV_ALL;
   if (!eng->predicted) {
     tic(eng, 2);
-    launch_predict(eng->d, sp, 1, eng->stream);
+    launch_predict(eng->d, sp, glob, eng->parity, eng->stream);
     toc(eng, "predict", 2);
-    // the predictor leaves the listed bodies' global vertices current (every
-    // body's while there is no list)
-    eng->gv_state = eng->d.soff ? rk_engine::GV_LISTED : rk_engine::GV_ALL;
+    eng->gv_state = gv_after;
   }
   const bool fuse = next && can_fuse(eng, guard);
   eng->predicted = fuse;
@@ -1053,9 +1085,10 @@ int vv_step(rk_engine* eng, int write_geom, bool guard, bool next) {
     toc(eng, "guard", 2);
   }
   if (fuse) {
-    launch_drive(eng->d, sp, eng->stream);
-    eng->gv_state = rk_engine::GV_LISTED;
+    launch_drive(eng->d, sp, glob, eng->stream);
+    eng->gv_state = gv_after;
   }
+  eng->parity ^= 1;
   return 0;
 }
 
@@ -1070,7 +1103,7 @@ int launch_one_step(rk_engine* eng, bool with_guard, bool next) {
 std::vector<unsigned char> graph_key(rk_engine* eng, int n, bool with_guard) {
   const StepParams sp = step_params(eng);
   const double spv[6] = {sp.dt, sp.dt_2, sp.dt2_2, sp.gx, sp.gy, sp.gz};
-  const int iv[5] = {n, with_guard ? 1 : 0, sp.law, eng->record_geometry, eng->live_interfaces};
+  const int iv[6] = {n, with_guard ? 1 : 0, sp.law, eng->record_geometry, eng->live_interfaces, eng->parity};
   std::vector<unsigned char> k(sizeof(Dev) + sizeof spv + sizeof iv);
   memcpy(k.data(), &eng->d, sizeof(Dev));
   memcpy(k.data() + sizeof(Dev), spv, sizeof spv);
@@ -1090,12 +1123,13 @@ int step_graph(rk_engine* eng, int n, bool with_guard, hipGraphExec_t* out) {
       *out = g.exec;
       return 0;
     }
+  const int parity = eng->parity;
   HIPCHK(hipStreamBeginCapture(eng->stream, hipStreamCaptureModeThreadLocal));
   int rc = 0;
   for (int k = 0; k < n && rc == 0; k++) rc = launch_one_step(eng, with_guard, k + 1 < n);
   hipGraph_t graph = nullptr;
   const hipError_t ec = hipStreamEndCapture(eng->stream, &graph);
-  eng->gv_state = rk_engine::GV_LISTED;  // each step of the graph ends with the listed bodies' fresh
+  eng->parity = parity;  // capturing runs nothing
   if (rc != 0 || ec != hipSuccess) {
     if (graph) (void)hipGraphDestroy(graph);
     return fail(eng, rc != 0 ? eng->err : std::string("step capture: ") + hipGetErrorString(ec));
@@ -1153,14 +1187,15 @@ int flush_steps(rk_engine* eng) {
   eng->pending = 0;
   const int G = eng->graph_steps;
   if (G > 1 && n >= G && eng->profile == 0) {
-    hipGraphExec_t exec = nullptr;
-    if (step_graph(eng, G, with_guard, &exec) != 0) return -1;
     for (; n >= G; n -= G) {
+      hipGraphExec_t exec = nullptr;
+      if (step_graph(eng, G, with_guard, &exec) != 0) return -1;  // (the step's parity is part of its key)
       HIPCHK(hipGraphLaunch(exec, eng->stream));
       eng->graph_launches++;
+      eng->parity ^= G & 1;
     }
-    // a replayed step leaves only the listed bodies' global vertices current
-    eng->gv_state = rk_engine::GV_LISTED;
+    // what a replayed step leaves of the global vertices (see vv_step)
+    eng->gv_state = uses_list(eng->d, eng->record_geometry) ? rk_engine::GV_STALE : rk_engine::GV_LISTED;
   }
   for (; n > 0; n--)
     if (launch_one_step(eng, with_guard, n > 1) != 0) return -1;
@@ -1944,6 +1979,7 @@ int upload_controls(rk_engine* eng) {
     // is evaluated at the next step
     const std::vector<double> cb = initial_bounds(eng->m);
     HIPCHK(hipMemcpyAsync(eng->cbound, cb.data(), sizeof(double) * nd, hipMemcpyHostToDevice, eng->stream));
+    HIPCHK(hipMemcpyAsync(eng->ahead, cb.data(), sizeof(double) * nd, hipMemcpyHostToDevice, eng->stream));
   }
   launch_reset_keys(eng->d, eng->stream);
   // the heavy bodies' summation paths depend on the passive flags
@@ -2226,7 +2262,7 @@ int rk_autotune(rk_engine* eng, int steps_per_trial, int64_t* steps_done) {
   };
   const Knob knobs[] = {{"fuse_law", {0, 1}},
                         {"type_sort", {1, 0}},
-                        {"skip_segment", {1024, 2048, 512, 4096, 256}},
+                        {"skip_segment", {1024, 256}},
                         {"law_group", {1, 2, 4, 8}},
                         {"geom_block", {64, 128, 256, 512}},
                         {"fuse_glob", {0, 1, 2, 3}},

@@ -1573,7 +1573,7 @@ int nl_build_csr(NLWork& w, int nb, EntryArrays& E, const uint8_t* passive, hipS
   if (ensure(w, E.istart, E.istart_cap, (size_t)nb + 1) || ensure(w, E.jstart, E.jstart_cap, (size_t)nb + 1) ||
       ensure(w, E.jlist, E.jlist_cap, (size_t)(n > 0 ? n : 1)) || ensure(w, w.i32a, w.i32a_cap, (size_t)nb + 1) ||
       ensure(w, w.i32b, w.i32b_cap, (size_t)(n > 0 ? n : 1)) || ensure(w, w.i32c, w.i32c_cap, (size_t)(n > 0 ? n : 1)) ||
-      ensure(w, E.edesc, E.edesc_cap, (size_t)(n > 0 ? n : 1)))
+      ensure(w, E.edesc, E.edesc_cap, 2 * (size_t)(n > 0 ? n : 1)))
     return -1;
   // istart: counts by owner, exclusive scan over nb + 1 (trailing zero)
   RK_CHECK(hipMemsetAsync(w.i32a, 0, sizeof(int32_t) * (nb + 1), s));
@@ -1989,6 +1989,7 @@ int entries_reserve(NLWork& w, EntryArrays& E, int n) {
             hipMalloc(&E.egeo, c * sizeof(EGeom)) == hipSuccess && hipMalloc(&E.edamp, c * sizeof(double)) == hipSuccess &&
             hipMalloc(&E.estick, c * sizeof(int32_t)) == hipSuccess && hipMalloc(&E.eact, c * sizeof(uint8_t)) == hipSuccess &&
             hipMalloc(&E.ekey, c * sizeof(double)) == hipSuccess &&
+            hipMalloc(&E.elist, c * sizeof(ListItem)) == hipSuccess &&
             hipMalloc(&E.spos, c * 2 * sizeof(int32_t)) == hipSuccess &&
             hipMalloc(&E.sact, c * 2 * sizeof(uint8_t) + 64) == hipSuccess  /* read 16 bytes at a time */ &&
             hipMalloc(&E.sval, c * 12 * sizeof(double)) == hipSuccess &&
@@ -2005,10 +2006,11 @@ int entries_reserve(NLWork& w, EntryArrays& E, int n) {
 
 void entries_free(EntryArrays& E) {
   void* ps[] = {E.ei, E.ej, E.esub, E.est, E.edn, E.egeo, E.edamp, E.estick, E.eact, E.ekey, E.spos, E.sact, E.sval,
-                E.akin, E.acount};
+                E.akin, E.acount, E.elist};
   for (void* q : ps)
     if (q) (void)hipFree(q);
   E.ekey = nullptr;
+  E.elist = nullptr;
   E.ei = E.ej = nullptr;
   E.esub = nullptr;
   E.est = nullptr;

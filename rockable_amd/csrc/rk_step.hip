@@ -77,6 +77,28 @@ __device__ __forceinline__ double prm(const DevParams& p, int id, int g1, int g2
   return p.tab[(id * p.G + g1) * p.G + g2];
 }
 
+// The contact parameters of a pair of groups.
+struct ContactPar {
+  double kn, kt, mu, kr, mur, en2;
+};
+__device__ __forceinline__ int group_pair(const DevParams& p, int g1, int g2) {
+  return (g1 < 0 || g2 < 0 || g1 >= p.G || g2 >= p.G) ? -1 : g1 * p.G + g2;
+}
+template <int LAW>
+__device__ __forceinline__ ContactPar contact_par(const DevParams& p, int gpair) {
+  ContactPar c;
+  const int n = p.G * p.G;
+  const double* t = p.tab + (gpair < 0 ? 0 : gpair);
+  c.kn = t[P_KN * n];
+  c.kt = t[P_KT * n];
+  c.mu = t[P_MU * n];
+  c.kr = t[P_KR * n];
+  c.mur = t[P_MUR * n];
+  c.en2 = LAW == LAW_AVALANCHE ? t[P_EN2 * n] : 0.0;
+  if (gpair < 0) c.kn = c.kt = c.mu = c.kr = c.mur = c.en2 = 0.0;
+  return c;
+}
+
 struct Kin {
   v3 n, pos, vel;
   double dn, prev_dn;
@@ -86,25 +108,14 @@ struct Kin {
 // The global vertices of a body, computed once per step by k_glob.
 __device__ __forceinline__ v3 gvtx(const double* g, int v) { return V(g[3 * v], g[3 * v + 1], g[3 * v + 2]); }
 
-// even-odd crossing test of P against a face of body j (Interaction.cpp:236-253):
-// its nbv vertices are gv[bj + fidx[fs + k]]
-__device__ bool face_crossing(const Dev& d, int fs, int nbv, int bj, v3 P, v3 v1, v3 v2) {
-  int odd = 0;
-  double ori1 = vdot(P, v1), ori2 = vdot(P, v2);
-  const int* fv = d.sh.fidx + fs;
-  v3 A = gvtx(d.gv, bj + fv[0]);
-  for (int iva = 0; iva < nbv; iva++) {
-    int ivb = iva + 1;
-    if (ivb == nbv) ivb = 0;
-    v3 B = gvtx(d.gv, bj + fv[ivb]);
-    double pa1 = vdot(A, v1), pb1 = vdot(B, v1);
-    double pa2 = vdot(A, v2), pb2 = vdot(B, v2);
-    if ((pa2 < ori2 && pb2 >= ori2) || (pb2 < ori2 && pa2 >= ori2)) {
-      if (pa1 + (ori2 - pa2) / (pb2 - pa2) * (pb1 - pa1) < ori1) odd = 1 - odd;
-    }
-    A = B;
+// even-odd crossing test of P against a face (Interaction.cpp:236-253), one
+// of its edges: toggles odd
+__device__ __forceinline__ void cross_edge(v3 A, v3 B, v3 v1, v3 v2, double ori1, double ori2, int& odd) {
+  double pa1 = vdot(A, v1), pb1 = vdot(B, v1);
+  double pa2 = vdot(A, v2), pb2 = vdot(B, v2);
+  if ((pa2 < ori2 && pb2 >= ori2) || (pb2 < ori2 && pa2 >= ori2)) {
+    if (pa1 + (ori2 - pa2) / (pb2 - pa2) * (pb1 - pa1) < ori1) odd = 1 - odd;
   }
-  return odd != 0;
 }
 
 // Per entry, the global-vertex indices (and face range) its contact geometry
@@ -112,14 +123,50 @@ __device__ bool face_crossing(const Dev& d, int fs, int nbv, int bj, v3 P, v3 v1
 // shapes at every step (which costs a chain of dependent loads):
 //   VV (vi, vj, -, -); VE (vi, j's edge ends); EE (i's edge ends, j's edge
 //   ends); VF (vi, start of j's face in sh.fidx, its vertex count, bvoff[j]).
+// edesc_s: the same with the indices of the shapes' vertex table (and j's
+// first vertex there for bvoff[j]).
+__device__ __forceinline__ void reset_list(const Dev& d) {
+  for (int k = 0; k < 8; k++) d.ls->cnt[0][k] = d.ls->cnt[1][k] = 0;
+  d.ls->gen = 0;
+  d.ls->want[0] = d.ls->want[1] = 1;
+  d.ls->again = 1;
+}
+__global__ void k_reset_list(Dev d) {
+  if (threadIdx.x == 0) reset_list(d);
+}
 __global__ void __launch_bounds__(kBlock) k_entry_desc(Dev d) {
+  if (blockIdx.x == 0) {
+    // a new list: the evaluation list starts anew, and the motion bounds'
+    // frame takes the mean velocity of up to 2048 free bodies spread over all
+    // (any frame is valid; a mean that is not finite is none)
+    __shared__ double red[3][kBlock];
+    const int t = threadIdx.x, nfree = d.nb - d.nDriven, n = min(nfree, 2048);
+    v3 u = V(0.0, 0.0, 0.0);
+    for (int k = t; k < n; k += kBlock) u = vadd(u, kvel(d.kin[d.nDriven + (int)((long)k * nfree / n)]));
+    red[0][t] = u.x;
+    red[1][t] = u.y;
+    red[2][t] = u.z;
+    for (int h = kBlock / 2; h > 0; h >>= 1) {
+      __syncthreads();
+      if (t < h)
+        for (int k = 0; k < 3; k++) red[k][t] += red[k][t + h];
+    }
+    if (t == 0) {
+      reset_list(d);
+      for (int k = 0; k < 3; k++) {
+        const double m = n > 0 ? red[k][0] / n : 0.0;
+        d.drift[k] = fabs(m) < 1e6 ? m : 0.0;
+      }
+    }
+  }
   for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < d.ne; e += gridDim.x * blockDim.x) {
     const int i = d.ei[e], j = d.ej[e];
     const uint32_t sub = d.esub[e];
     const int type = (int)(sub >> 30), isub = (int)((sub >> 15) & 0x7fffu), jsub = (int)(sub & 0x7fffu);
     const int bi = d.bvoff[i], bj = d.bvoff[j];
     const int shi = d.kin[i].shape, shj = d.kin[j].shape;
-    int4 q = make_int4(bi + isub, 0, 0, 0);
+    const int dvi = d.sh.voff[shi] - bi, dvj = d.sh.voff[shj] - bj;
+    int4 q = make_int4(bi + isub, 0, 0, 0), r;
     if (type == VV) {
       q.y = bj + jsub;
     } else if (type == VE) {
@@ -136,27 +183,33 @@ __global__ void __launch_bounds__(kBlock) k_entry_desc(Dev d) {
       const int* edj = d.sh.edge + 2 * (d.sh.eoff[shj] + jsub);
       q = make_int4(bi + edi[0], bi + edi[1], bj + edj[0], bj + edj[1]);
     }
+    r = type == EE   ? make_int4(q.x + dvi, q.y + dvi, q.z + dvj, q.w + dvj)
+        : type == VF ? make_int4(q.x + dvi, q.y, q.z, q.w + dvj)
+                     : make_int4(q.x + dvi, q.y + dvj, q.z + dvj, 0);
     d.edesc[e] = q;
+    d.edesc_s[e] = r;
   }
 }
 
-// Interaction::UpdateDispatcher (Interaction.cpp:147-326), on the entry's
-// resolved vertex indices q (k_entry_desc).
-// WITH_VEL: also the relative velocity at the contact point (Interaction.cpp:162).
-template <bool WITH_VEL>
-__device__ void update_kinematics(const Dev& d, int type, int4 q, const BodyKin& Pi, const BodyKin& Pj, Kin& k) {
-  const double Ri = Pi.R, Rj = Pj.R;
+// Interaction::UpdateDispatcher (Interaction.cpp:147-326) without the
+// relative velocity (the law computes it), on the positions p of the
+// entry's vertices: VV i, j; VE i, j's edge; EE i's edge, j's edge; VF i, the
+// face's first three and last vertices.  nbv: the face's vertex count; a
+// face of more than four (or fewer than three) takes the others from
+// face(k).
+template <class Face>
+__device__ __forceinline__ void update_kinematics(int type, int nbv, const v3 p[5], double Ri, double Rj, Kin& k,
+                                                  Face face) {
   if (type == VV) {
-    v3 posi = gvtx(d.gv, q.x);
-    v3 posj = gvtx(d.gv, q.y);
+    v3 posi = p[0];
+    v3 posj = p[1];
     k.n = vsub(posi, posj);
     k.dn = vnormalize(&k.n) - (Ri + Rj);
     k.pos = vsub(posi, vsc(Ri + 0.5 * k.dn, k.n));
-    if (WITH_VEL) k.vel = rel_vel(k.pos, Pi, Pj);
   } else if (type == VE) {
-    v3 posj1 = gvtx(d.gv, q.y);
-    v3 posj2 = gvtx(d.gv, q.z);
-    v3 posi = gvtx(d.gv, q.x);
+    v3 posj1 = p[1];
+    v3 posj2 = p[2];
+    v3 posi = p[0];
     v3 E = vsub(posj2, posj1);
     v3 v = vsub(posi, posj1);
     double r = vdot(v, E) / vdot(E, E);
@@ -167,14 +220,11 @@ __device__ void update_kinematics(const Dev& d, int type, int4 q, const BodyKin&
     k.n = vsub(posi, vadd(posj1, vsc(r, E)));
     k.dn = vnormalize(&k.n) - (Ri + Rj);
     k.pos = vsub(posi, vsc(Ri + 0.5 * k.dn, k.n));
-    if (WITH_VEL) k.vel = rel_vel(k.pos, Pi, Pj);
   } else if (type == VF) {
-    const int fs = q.y, nbv = q.z, bj = q.w;
-    const int* fv = d.sh.fidx + fs;
-    v3 A = gvtx(d.gv, bj + fv[0]);
-    v3 B = gvtx(d.gv, bj + fv[1]);
-    v3 C = gvtx(d.gv, bj + fv[nbv - 1]);
-    v3 posi = gvtx(d.gv, q.x);
+    v3 A = p[1];
+    v3 B = p[2];
+    v3 C = p[4];
+    v3 posi = p[0];
     v3 v = vsub(posi, A);
     v3 v1 = vsub(B, A);
     vnormalize(&v1);
@@ -188,18 +238,32 @@ __device__ void update_kinematics(const Dev& d, int type, int4 q, const BodyKin&
     }
     v3 P = vsub(posi, vsc(dist, k.n));
     v2 = vcross(k.n, v1);
-    if (face_crossing(d, fs, nbv, bj, P, v1, v2)) {
+    int odd = 0;
+    const double ori1 = vdot(P, v1), ori2 = vdot(P, v2);
+    if (nbv == 3 || nbv == 4) {
+      cross_edge(A, B, v1, v2, ori1, ori2, odd);
+      cross_edge(B, p[3], v1, v2, ori1, ori2, odd);
+      if (nbv == 4) cross_edge(p[3], C, v1, v2, ori1, ori2, odd);
+      cross_edge(C, A, v1, v2, ori1, ori2, odd);
+    } else {
+      v3 a = A;
+      for (int iva = 0; iva < nbv; iva++) {
+        const v3 b = face(iva + 1 == nbv ? 0 : iva + 1);
+        cross_edge(a, b, v1, v2, ori1, ori2, odd);
+        a = b;
+      }
+    }
+    if (odd != 0) {
       k.dn = dist - (Ri + Rj);
       k.pos = vsub(posi, vsc(Ri + 0.5 * k.dn, k.n));
-      if (WITH_VEL) k.vel = rel_vel(k.pos, Pi, Pj);
     } else {
       k.deact = true;  // n keeps the new face normal, pos and vel stay stale
     }
   } else {
-    v3 posi1 = gvtx(d.gv, q.x);
-    v3 posi2 = gvtx(d.gv, q.y);
-    v3 posj1 = gvtx(d.gv, q.z);
-    v3 posj2 = gvtx(d.gv, q.w);
+    v3 posi1 = p[0];
+    v3 posi2 = p[1];
+    v3 posj1 = p[2];
+    v3 posj2 = p[3];
     v3 Ei = vsub(posi2, posi1);
     v3 Ej = vsub(posj2, posj1);
     v3 v = vsub(posi1, posj1);
@@ -217,11 +281,34 @@ __device__ void update_kinematics(const Dev& d, int type, int4 q, const BodyKin&
       k.n = vsub(vadd(posi1, vsc(s, Ei)), vadd(posj1, vsc(t, Ej)));
       k.dn = vnormalize(&k.n) - (Ri + Rj);
       k.pos = vsub(vadd(posi1, vsc(s, Ei)), vsc(Ri + 0.5 * k.dn, k.n));
-      if (WITH_VEL) k.vel = rel_vel(k.pos, Pi, Pj);
     } else {
       k.deact = true;
     }
   }
+}
+
+// The same on an entry's resolved global vertices q (k_entry_desc), as the
+// steps that evaluate every entry read them.
+__device__ __forceinline__ void update_kinematics_gv(const Dev& d, int type, int4 q, double Ri, double Rj, Kin& k) {
+  v3 p[5];
+  int nbv = 0, fs = 0, bj = 0;
+  p[0] = gvtx(d.gv, q.x);
+  if (type == VF) {
+    fs = q.y;
+    nbv = q.z;
+    bj = q.w;
+    const int* fv = d.sh.fidx + fs;
+    p[1] = gvtx(d.gv, bj + fv[0]);
+    p[2] = gvtx(d.gv, bj + fv[1]);
+    p[3] = gvtx(d.gv, bj + fv[nbv > 2 ? 2 : 0]);
+    p[4] = gvtx(d.gv, bj + fv[nbv - 1]);
+  } else {
+    p[1] = gvtx(d.gv, q.y);
+    p[2] = type == VV ? p[1] : gvtx(d.gv, q.z);
+    p[3] = type == EE ? gvtx(d.gv, q.w) : p[2];
+    p[4] = p[3];
+  }
+  update_kinematics(type, nbv, p, Ri, Rj, k, [&](int a) { return gvtx(d.gv, bj + d.sh.fidx[fs + a]); });
 }
 
 struct Hist {
@@ -230,7 +317,7 @@ struct Hist {
 };
 
 // ForceLaw_Default::computeInteraction (ForceLaw_Default.cpp:57-131), FT_CORR off
-__device__ void law_default(const Dev& d, const StepParams& sp, const Kin& k, double damp, const BodyKin& Pi,
+__device__ void law_default(const ContactPar& cp, const StepParams& sp, const Kin& k, double damp, const BodyKin& Pi,
                             const BodyKin& Pj, Hist& h) {
   if (k.dn > 0.0) {
     h.fn = 0.0;
@@ -238,9 +325,7 @@ __device__ void law_default(const Dev& d, const StepParams& sp, const Kin& k, do
     h.mom = V(0, 0, 0);
     return;
   }
-  const int g1 = Pi.group, g2 = Pj.group;
-  const double kn = prm(d.par, P_KN, g1, g2), kt = prm(d.par, P_KT, g1, g2), mu = prm(d.par, P_MU, g1, g2);
-  const double kr = prm(d.par, P_KR, g1, g2), mur = prm(d.par, P_MUR, g1, g2);
+  const double kn = cp.kn, kt = cp.kt, mu = cp.mu, kr = cp.kr, mur = cp.mur;
   double vn = vdot(k.vel, k.n);
   double fne = -kn * k.dn;
   double fnv = damp * vn;
@@ -261,17 +346,15 @@ __device__ void law_default(const Dev& d, const StepParams& sp, const Kin& k, do
 }
 
 // ForceLaw_Avalanche::computeInteraction (ForceLaw_Avalanche.cpp:57-136)
-__device__ void law_avalanche(const Dev& d, const StepParams& sp, const Kin& k, int i, const BodyKin& Pi,
-                              const BodyKin& Pj, Hist& h) {
+__device__ void law_avalanche(const Dev& d, const ContactPar& cp, const StepParams& sp, const Kin& k, int i,
+                              const BodyKin& Pi, const BodyKin& Pj, Hist& h) {
   if (k.dn > 0.0) {
     h.fn = 0.0;
     h.ft = V(0, 0, 0);
     h.mom = V(0, 0, 0);
     return;
   }
-  const int g1 = Pi.group, g2 = Pj.group;
-  const double kn = prm(d.par, P_KN, g1, g2), en2 = prm(d.par, P_EN2, g1, g2), kt = prm(d.par, P_KT, g1, g2);
-  const double mu = prm(d.par, P_MU, g1, g2), kr = prm(d.par, P_KR, g1, g2), mur = prm(d.par, P_MUR, g1, g2);
+  const double kn = cp.kn, en2 = cp.en2, kt = cp.kt, mu = cp.mu, kr = cp.kr, mur = cp.mur;
   double prev_dn = k.prev_dn;
   if (prev_dn > 0.0) prev_dn = 0.0;
   double delta_Dn = k.dn - prev_dn;
@@ -298,11 +381,12 @@ __device__ void law_avalanche(const Dev& d, const StepParams& sp, const Kin& k, 
 }
 
 // ForceLaw_StickedLinks::computeInteraction (ForceLaw_StickedLinks.cpp:75-215)
-__device__ void law_sticked(const Dev& d, const StepParams& sp, const Kin& k, double damp, int stick, int i, int j,
-                            const BodyKin& Pi, const BodyKin& Pj, Hist& h, bool paramsInInterfaces) {
+// bp: the bond's interface parameters (read for stick >= 0)
+__device__ void law_sticked(const Dev& d, const ContactPar& cp, const double bp[8], const StepParams& sp, const Kin& k,
+                            double damp, int stick, int i, int j, const BodyKin& Pi, const BodyKin& Pj, Hist& h,
+                            bool paramsInInterfaces) {
   if (stick >= 0) {
     double kn = 0.0, kt = 0.0, kr = 0.0, fn0 = 1.0, ft0 = 1.0, mom0 = 1.0, power = 1.0;
-    const double* bp = d.ifc.par + 8 * stick;
     double dn0 = bp[7];
     const int g1 = Pi.group, g2 = Pj.group;
     if (paramsInInterfaces) {
@@ -357,9 +441,7 @@ __device__ void law_sticked(const Dev& d, const StepParams& sp, const Kin& k, do
       h.mom = V(0, 0, 0);
       return;
     }
-    const int g1 = Pi.group, g2 = Pj.group;
-    const double kn = prm(d.par, P_KN, g1, g2), kt = prm(d.par, P_KT, g1, g2), mu = prm(d.par, P_MU, g1, g2);
-    const double kr = prm(d.par, P_KR, g1, g2), mur = prm(d.par, P_MUR, g1, g2);
+    const double kn = cp.kn, kt = cp.kt, mu = cp.mu, kr = cp.kr, mur = cp.mur;
     double vn = vdot(k.vel, k.n);
     double fne = -kn * k.dn;
     double fnv = damp * vn;
@@ -382,14 +464,13 @@ __device__ void law_sticked(const Dev& d, const StepParams& sp, const Kin& k, do
 // Rockable.cpp:2934-2977): its gap, and for an active entry its kinematics in
 // a (returns true); an inactive entry gets its gap and activity byte here,
 // and with skipping its far-entry key.
-template <bool GEOM_ALL>
-__device__ __forceinline__ bool geom_entry(const Dev& d, int e, bool skipping, ActiveKin& a) {
+// kinematics(k): the contact kinematics; old: the entry's activity byte and
+// ci, cj its bodies' motion bounds, which only an inactive entry needs.
+template <bool GEOM_ALL, class Kinematics, class Old, class Bounds>
+__device__ __forceinline__ bool geom_entry(const Dev& d, int e, bool skipping, int i, int j, int stick, const BodyKin& Pi,
+                                           const BodyKin& Pj, ActiveKin& a, Kinematics kinematics, Old old_act,
+                                           Bounds bounds) {
   bool act = false;
-  const int i = d.ei[e], j = d.ej[e];
-  const int type = (int)(d.esub[e] >> 30);
-  const BodyKin& Pi = d.kin[i];
-  const BodyKin& Pj = d.kin[j];
-  const int stick = d.ifc.n > 0 ? d.estick[e] : -1;  // bonds exist only with interfaces
   Kin k;
   k.deact = false;
   k.prev_dn = 0.0;  // the previous dn is read by the law, for active entries only
@@ -398,7 +479,7 @@ __device__ __forceinline__ bool geom_entry(const Dev& d, int e, bool skipping, A
     k.n = V(g.nx, g.ny, g.nz);
     k.pos = V(g.px, g.py, g.pz);
   }
-  update_kinematics<false>(d, type, d.edesc[e], Pi, Pj, k);
+  kinematics(k);
   if (k.deact) k.dn = 0.0;  // Interaction::deactivate (Interaction.cpp:123-128)
   act = (k.dn < 0.0) || (stick >= 0);
   if (act) {
@@ -417,7 +498,7 @@ __device__ __forceinline__ bool geom_entry(const Dev& d, int e, bool skipping, A
   } else {
     // activity byte: bit 0 active, bit 1 history maybe non-zero; the
     // history and the slot flags are written only when they change
-    const uint8_t old = d.eact[e];
+    const uint8_t old = old_act();
     uint8_t now = old & 2;
     if (k.deact) {
       if (old & 2) {
@@ -435,7 +516,8 @@ __device__ __forceinline__ bool geom_entry(const Dev& d, int e, bool skipping, A
       if (skipping && now == 0) {
         // the key of a zero-history entry (a body without a finite bound
         // never lets its entries be skipped)
-        const double ci = d.cbound[i], cj = d.cbound[j];
+        double ci, cj;
+        bounds(ci, cj);
         d.ekey[e] = (ci < INFINITY && cj < INFINITY) ? k.dn + ci + cj : -INFINITY;
       }
       if (GEOM_ALL) {
@@ -528,7 +610,19 @@ __device__ __forceinline__ bool geom_pass(const Dev& d, int blk, int (*wtype)[5]
       atomicAdd(d.skip_count + 2, (unsigned long long)__popcll(ml));
     }
   }
-  if (e < d.ne && !skip) act = geom_entry<GEOM_ALL>(d, e, skipping, a);
+  if (e < d.ne && !skip) {
+    const int i = d.ei[e], j = d.ej[e];
+    const int stick = d.ifc.n > 0 ? d.estick[e] : -1;  // bonds exist only with interfaces
+    const BodyKin &Pi = d.kin[i], &Pj = d.kin[j];
+    act = geom_entry<GEOM_ALL>(
+        d, e, skipping, i, j, stick, Pi, Pj, a,
+        [&](Kin& k) { update_kinematics_gv(d, (int)(d.esub[e] >> 30), d.edesc[e], Pi.R, Pj.R, k); },
+        [&] { return d.eact[e]; },
+        [&](double& ci, double& cj) {
+          ci = d.cbound[i];
+          cj = d.cbound[j];
+        });
+  }
   return act;
 }
 
@@ -569,20 +663,30 @@ __global__ void __launch_bounds__(BS) k_geom(Dev d) {
 
 // The force law of one active entry (kinematics in a): history, both
 // resultant slots, activity flags.
-template <int LAW>
+// What the law reads of an active entry's own state.
+struct EntryState {
+  EState s;
+  double damp, dn;
+  int2 slots;
+  int stick;
+  uint8_t act;
+  ContactPar cp;
+  double bp[8];
+};
+// PRE: the entry's own state is in x (else it is read where it is needed).
+template <int LAW, bool PRE>
 __device__ __forceinline__ void law_item(const Dev& d, const StepParams& sp, int write_geom_all, int pii,
-                                         const ActiveKin& a) {
+                                         const ActiveKin& a, const BodyKin& Pi, const BodyKin& Pj,
+                                         const EntryState& x) {
   const int e = a.e;
   const int i = a.i, j = a.j;
-  const BodyKin Pi = d.kin[i];
-  const BodyKin Pj = d.kin[j];
-  const int stick = d.estick[e];
+  const int stick = PRE ? x.stick : d.estick[e];
   Kin k;
   k.n = V(a.nx, a.ny, a.nz);
   k.pos = V(a.px, a.py, a.pz);
   k.dn = a.dn;
   // the previous step's dn (the Avalanche law's only; a deactivation zeroes it)
-  k.prev_dn = (LAW == LAW_AVALANCHE && !a.deact) ? d.edn[e] : 0.0;
+  k.prev_dn = (LAW == LAW_AVALANCHE && !a.deact) ? (PRE ? x.dn : d.edn[e]) : 0.0;
   k.deact = a.deact != 0;
   Hist h;
   if (k.deact) {  // a bond keeps its stale velocity; the history restarts
@@ -593,18 +697,20 @@ __device__ __forceinline__ void law_item(const Dev& d, const StepParams& sp, int
     h.mom = V(0, 0, 0);
   } else {
     k.vel = rel_vel(k.pos, Pi, Pj);
-    const EState s = d.est[e];
+    const EState s = PRE ? x.s : d.est[e];
     h.fn = s.fn;
     h.ft = V(s.ftx, s.fty, s.ftz);
     h.mom = V(s.momx, s.momy, s.momz);
   }
-  const double damp = d.edamp[e];
+  const double damp = LAW == LAW_AVALANCHE ? 0.0 : PRE ? x.damp : d.edamp[e];  // (the Avalanche law has none)
+  const ContactPar cp = PRE ? x.cp : contact_par<LAW>(d.par, group_pair(d.par, Pi.group, Pj.group));
   if (LAW == LAW_AVALANCHE)
-    law_avalanche(d, sp, k, i, Pi, Pj, h);
+    law_avalanche(d, cp, sp, k, i, Pi, Pj, h);
   else if (LAW == LAW_STICKED)
-    law_sticked(d, sp, k, damp, stick, i, j, Pi, Pj, h, pii != 0);
+    law_sticked(d, cp, PRE ? x.bp : d.ifc.par + 8 * (size_t)(stick >= 0 ? stick : 0), sp, k, damp, stick, i, j, Pi, Pj, h,
+                pii != 0);
   else
-    law_default(d, sp, k, damp, Pi, Pj, h);
+    law_default(cp, sp, k, damp, Pi, Pj, h);
   EState o;
   o.fn = h.fn;
   o.ftx = h.ft.x;
@@ -623,7 +729,7 @@ __device__ __forceinline__ void law_item(const Dev& d, const StepParams& sp, int
   v3 mj = vsub(vcross(Cj, vneg(f)), h.mom);
   // the two resultant slots: body i adds (f, mi), body j adds (-f, mj);
   // x + (-y) is x - y exactly, so the serial sums are unchanged
-  const int2 slots = reinterpret_cast<const int2*>(d.spos)[e];
+  const int2 slots = PRE ? x.slots : reinterpret_cast<const int2*>(d.spos)[e];
   double* ci = d.sval + 6 * (size_t)slots.x;
   double* cj = d.sval + 6 * (size_t)slots.y;
   st3(ci, f);
@@ -645,7 +751,7 @@ __device__ __forceinline__ void law_item(const Dev& d, const StepParams& sp, int
     g.vz = k.vel.z;
     d.egeo[e] = g;
   }
-  const uint8_t old = d.eact[e];
+  const uint8_t old = PRE ? x.act : d.eact[e];
   if (old != 3) {
     d.eact[e] = 3;
     if (!(old & 1)) {
@@ -653,6 +759,15 @@ __device__ __forceinline__ void law_item(const Dev& d, const StepParams& sp, int
       d.sact[slots.y] = 1;
     }
   }
+}
+
+// The law of an active entry apart from its geometry pass.
+template <int LAW>
+__device__ __forceinline__ void law_entry(const Dev& d, const StepParams& sp, int write_geom_all, int pii,
+                                          const ActiveKin& a) {
+  const BodyKin Pi = d.kin[a.i];
+  const BodyKin Pj = d.kin[a.j];
+  law_item<LAW, false>(d, sp, write_geom_all, pii, a, Pi, Pj, EntryState{});
 }
 
 // Each wavefront takes W (at most kLawGroup) consecutive geometry blocks
@@ -687,7 +802,7 @@ __global__ void __launch_bounds__(kBlock, LAW == LAW_STICKED ? 2 : 4) k_law(Dev 
         before = pre[m];
       }
     const ActiveKin a = d.akin[(size_t)(g0 + gb) * d.geom_block + (t - before)];
-    law_item<LAW>(d, sp, write_geom_all, pii, a);
+    law_entry<LAW>(d, sp, write_geom_all, pii, a);
   }
   }
 }
@@ -710,97 +825,215 @@ __global__ void __launch_bounds__(kBlock, LAW == LAW_STICKED ? 2 : 4) k_interact
     const int r = active_rank<kBlock>(act, wcount, &total);
     if (act) sa[r] = a;
     __syncthreads();
-    if ((int)threadIdx.x < total) law_item<LAW>(d, sp, write_geom_all, pii, sa[threadIdx.x]);
+    if ((int)threadIdx.x < total) law_entry<LAW>(d, sp, write_geom_all, pii, sa[threadIdx.x]);
     __syncthreads();
   }
 }
 
-// The far-entry skip with compaction: a workgroup takes SEG consecutive
-// entries, tests each against the motion bounds (coalesced reads of the
-// activity byte, the key and the pair; the bounds are per body and stay in
-// L2), gathers the entries still to evaluate into an LDS list, and runs the
-// geometry and the force law on that list, each lane taking the law of its
-// own entry.  In a settled packing about one entry in ten is evaluated and
-// most of those are active: the list fills whole wavefronts, where the
-// per-entry test of k_interact leaves most lanes of every wavefront idle for
-// the length of the busiest lane's chain.  The
-// entries are independent (each writes its own state and its own two
-// resultant slots), so the order of the list changes no result.
-template <int LAW, int SEG>
-__global__ void __launch_bounds__(kBlock, LAW == LAW_STICKED ? 2 : 4) k_interact_seg(Dev d, StepParams sp, int pii) {
-  constexpr int M = SEG / kBlock;
-  __shared__ int wcnt[M][kBlock / 64];
-  __shared__ int list[SEG];
-  if (frozen(d)) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  unsigned long long cnt[3] = {0ull, 0ull, 0ull};  // the wavefront's counts (count_skips)
-  for (TileLoop L = xcd_tiles((d.ne + SEG - 1) / SEG); L.t < L.end; L.t += L.step) {
-    const int e0 = L.t * SEG + (int)threadIdx.x;
-    bool need[M];
+// Geometry and force law of one entry of the evaluation list.  Everything it
+// may read is read at once, before the geometry: its own state (an entry on
+// the list is more often active than not), the bodies, the vertices in their
+// shapes' frames, the law's parameters, the motion bounds; the reads then
+// share one latency.  The vertices are moved by the bodies' poses here
+// (glob_vertex's expression): a listed entry reads few of them, and computing
+// them saves the round trip of every vertex through memory (264 bytes per
+// hull and step).
+template <int LAW>
+__device__ __forceinline__ void eval_item(const Dev& d, const StepParams& sp, int pii, const ListItem& it) {
+  const int e = it.e, i = it.i, j = it.j, type = it.kind & 3;
+  EntryState x;
+  x.s = d.est[e];
+  x.dn = LAW == LAW_AVALANCHE ? d.edn[e] : 0.0;
+  x.act = d.eact[e];
+  x.stick = d.ifc.n > 0 ? d.estick[e] : -1;  // bonds exist only with interfaces; one may have broken since
+  x.slots = it.slots;
+  x.damp = it.damp;
+  x.cp = contact_par<LAW>(d.par, it.gpair);
+  if (LAW == LAW_STICKED && it.stick >= 0) {
+    const double* bp = d.ifc.par + 8 * (size_t)it.stick;
 #pragma unroll
-    for (int r = 0; r < M; r++) {
-      // the activity byte, key and pair together (one round trip), then the bounds
-      const int e = e0 + r * kBlock;
-      bool nd = e < d.ne;
-      if (nd) {
-        const uint8_t ea = d.eact[e];
-        const double key = d.ekey[e];
-        const int bi = d.ei[e], bj = d.ej[e];
-        nd = !(ea == 0 && key - d.cbound[bi] - d.cbound[bj] > kSkipMargin);
-      }
-      need[r] = nd;
-    }
-    if (d.skip_count) {  // counts for the measurement of the skip (off in production)
-#pragma unroll
-      for (int r = 0; r < M; r++) {
-        const int e = e0 + r * kBlock;
-        cnt[0] += __popcll(__ballot(e < d.ne && !need[r]));
-        cnt[1] += __popcll(__ballot(e < d.ne && d.eact[e] == 0));
-        cnt[2] += __popcll(__ballot(e < d.ne));
-      }
-    }
-    // rank the entries to evaluate, in entry order: every wavefront's counts
-    // for the M rows first, one barrier, then each thread its own places
-    unsigned long long mask[M];
-#pragma unroll
-    for (int r = 0; r < M; r++) {
-      mask[r] = __ballot(need[r]);
-      if (lane == 0) wcnt[r][wave] = __popcll(mask[r]);
-    }
-    __syncthreads();
-    int n = 0;
-#pragma unroll
-    for (int r = 0; r < M; r++) {
-      int before = 0, tot = 0;
-#pragma unroll
-      for (int w = 0; w < kBlock / 64; w++) {
-        const int c = wcnt[r][w];
-        before += w < wave ? c : 0;
-        tot += c;
-      }
-      if (need[r]) list[n + before + __popcll(mask[r] & ((1ull << lane) - 1ull))] = e0 + r * kBlock;
-      n += tot;
-    }
-    __syncthreads();
-    // the evaluated entries are dense in the list and most of them are
-    // active: each lane applies the law to its own entry right after its
-    // geometry (the body records still in registers), no second ranking
-    for (int c = (int)threadIdx.x; c < n; c += kBlock) {
-      ActiveKin a;
-      if (geom_entry<false>(d, list[c], true, a)) law_item<LAW>(d, sp, 0, pii, a);
-    }
-    __syncthreads();  // the next tile's ranking rewrites wcnt and list
+    for (int q = 0; q < 8; q++) x.bp[q] = bp[q];
   }
-  if (d.skip_count) {  // one atomic per workgroup and count (the counts summed in LDS first)
-    __shared__ unsigned long long wsum[3][kBlock / 64];
-    if (lane == 0)
-      for (int k = 0; k < 3; k++) wsum[k][wave] = cnt[k];
-    __syncthreads();
-    if (threadIdx.x < 3) {
-      unsigned long long t = 0ull;
-      for (int w = 0; w < kBlock / 64; w++) t += wsum[threadIdx.x][w];
-      atomicAdd(d.skip_count + threadIdx.x, t);
+  const BodyKin &Pi = d.kin[i], &Pj = d.kin[j];
+  const double cbi = d.cbound[i], cbj = d.cbound[j];
+  v3 r[5];
+#pragma unroll
+  for (int q = 0; q < 4; q++) r[q] = gvtx(d.sh.vtx, it.v[q]);
+  r[4] = gvtx(d.sh.vtx, it.v4);
+  const v3 ci = kpos(Pi), cj = kpos(Pj);
+  const qt Qi = kq(Pi), Qj = kq(Pj);
+  const double Hi = Pi.h, Hj = Pj.h, Ri = Pi.R, Rj = Pj.R;
+  auto of_j = [&](v3 u) { return vadd(cj, qrot(Qj, vsc(Hj, u))); };
+  ActiveKin a;
+  if (geom_entry<false>(
+          d, e, true, i, j, x.stick, Pi, Pj, a,
+          [&](Kin& k) {
+            v3 p[5];
+            p[0] = vadd(ci, qrot(Qi, vsc(Hi, r[0])));
+            // the second vertex is i's for two edges, else j's
+            const bool ee = type == EE;
+            p[1] = vadd(ee ? ci : cj, qrot(ee ? Qi : Qj, vsc(ee ? Hi : Hj, r[1])));
+            if (type != VV) p[2] = of_j(r[2]);
+            if (type == EE || type == VF) p[3] = of_j(r[3]);
+            if (type == VF) p[4] = of_j(r[4]);
+            update_kinematics(type, it.kind >> 2, p, Ri, Rj, k, [&](int n) {
+              const int4 q = d.edesc_s[e];
+              return of_j(gvtx(d.sh.vtx, q.w + d.sh.fidx[q.y + n]));
+            });
+          },
+          [&] { return x.act; },
+          [&](double& bi, double& bj) {
+            bi = cbi;
+            bj = cbj;
+          }))
+    law_item<LAW, true>(d, sp, 0, pii, a, Pi, Pj, x);
+}
+
+constexpr int kListTile = 1024;
+// One tile's test (entries e0, e0 + 256, ... per thread): the entries that
+// may need evaluation while the new list holds go to part, at places taken
+// from count; their range there is returned.
+__device__ __forceinline__ int2 list_tile(const Dev& d, int e0, ListItem* part, int* count) {
+  constexpr int M = kListTile / kBlock;
+  __shared__ int wcnt[M][kBlock / 64];
+  __shared__ int at;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  unsigned keep = 0u;  // bit r: entry e0 + 256 r
+#pragma unroll
+  for (int r = 0; r < M; r++) {
+    // the activity byte, key and pair together (one round trip), then the bounds
+    const int e = e0 + r * kBlock;
+    if (e < d.ne) {
+      const uint8_t ea = d.eact[e];
+      const double key = d.ekey[e];
+      const int bi = d.ei[e], bj = d.ej[e];
+      keep |= (ea == 0 && key - d.ahead[bi] - d.ahead[bj] > kSkipMargin) ? 0u : 1u << r;
     }
+  }
+  // rank the entries, in entry order: every wavefront's counts for the M
+  // rows first, one barrier, then each thread its own places
+  unsigned long long mask[M];
+#pragma unroll
+  for (int r = 0; r < M; r++) {
+    mask[r] = __ballot(keep >> r & 1u);
+    if (lane == 0) wcnt[r][wave] = __popcll(mask[r]);
+  }
+  __syncthreads();
+  int n = 0;
+#pragma unroll
+  for (int r = 0; r < M; r++)
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; w++) n += wcnt[r][w];
+  if (t == 0) at = atomicAdd(count, n);
+  __syncthreads();
+  int k = at;
+  const int first = k;
+#pragma unroll
+  for (int r = 0; r < M; r++) {
+    int before = 0, tot = 0;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; w++) {
+      const int c = wcnt[r][w];
+      before += w < wave ? c : 0;
+      tot += c;
+    }
+    if (keep >> r & 1u) {
+      const int e = e0 + r * kBlock;
+      ListItem it;
+      it.e = e;
+      it.i = d.ei[e];
+      it.j = d.ej[e];
+      const int type = (int)(d.esub[e] >> 30);
+      const int4 q = d.edesc_s[e];
+      it.kind = type;
+      it.v[0] = it.v[1] = it.v[2] = it.v[3] = it.v4 = q.x;
+      if (type == VF) {
+        const int* fv = d.sh.fidx + q.y;
+        it.kind |= q.z << 2;
+        it.v[1] = q.w + fv[0];
+        it.v[2] = q.w + fv[1];
+        it.v[3] = q.w + fv[q.z > 2 ? 2 : 0];
+        it.v4 = q.w + fv[q.z - 1];
+      } else {
+        it.v[1] = q.y;
+        if (type != VV) it.v[2] = q.z;
+        if (type == EE) it.v[3] = q.w;
+      }
+      it.gpair = group_pair(d.par, d.kin[it.i].group, d.kin[it.j].group);
+      it.stick = d.ifc.n > 0 ? d.estick[e] : -1;
+      it.pad = 0;
+      it.slots = reinterpret_cast<const int2*>(d.spos)[e];
+      it.damp = d.edamp[e];
+      part[k + before + __popcll(mask[r] & ((1ull << lane) - 1ull))] = it;
+    }
+    k += tot;
+  }
+  __syncthreads();  // the items are read by other threads; wcnt and at are free again
+  return make_int2(first, k);
+}
+
+// The measurement of the skip (count_skips): entries whose gap the current
+// bounds prove positive, inactive entries with zero history, entries.
+__global__ void __launch_bounds__(kBlock) k_count_skips(Dev d) {
+  if (frozen(d)) return;
+  unsigned long long cnt[3] = {0ull, 0ull, 0ull};
+  for (int e0 = blockIdx.x * blockDim.x; e0 < d.ne; e0 += gridDim.x * blockDim.x) {
+    const int e = e0 + (int)threadIdx.x;
+    const bool in = e < d.ne, zero = in && d.eact[e] == 0;
+    const bool far = zero && d.ekey[e] - d.cbound[d.ei[e]] - d.cbound[d.ej[e]] > kSkipMargin;
+    cnt[0] += __popcll(__ballot(far));
+    cnt[1] += __popcll(__ballot(zero));
+    cnt[2] += __popcll(__ballot(in));
+  }
+  if ((threadIdx.x & 63) == 0)
+    for (int k = 0; k < 3; k++) atomicAdd(d.skip_count + k, cnt[k]);
+}
+
+// The force phase on the evaluation list (Dev::elist).  Most steps take the
+// list as it stands: a lane per listed entry, geometry then law, nothing
+// read of the others (four in five in a settled packing).  A step whose
+// predictor found the list outdated takes the entries in tiles of 1024: each
+// is tested against the motion bounds (coalesced reads of the activity byte,
+// the key and the pair; the bounds are per body and stay in L2), those that
+// may need evaluation while the bodies stay within their allowances are
+// appended to the tile's XCD part of the new list (one atomic per tile), and
+// evaluated.  The entries are independent (each writes its own state and its
+// own two resultant slots), so neither the list's order nor an entry on it
+// without need changes a result.
+// What bounds it is the chain of an entry's dependent loads (the list's
+// words, the item, its state with its bodies and vertices) and, from some
+// 10^5 items, the entry states gathered one in five.  Testing every entry at
+// every step, 1024 to a workgroup, ran a workgroup's evaluations in up to
+// four rounds of a longer chain, however few workgroups a small packing has:
+// 15.4 us for 517 spheres, 34.6 us for the 50 005-body pour (205 000 of its
+// 1.12 M entries listed), 38.5 us for the 90 006-body slope, 24.4 and 34.2 us
+// for 1 201 and 13 001 bonded cubes; on the list 14.0, 30.1, 36.8, 12.5 and
+// 27.5 us, of which a new list every 17 steps or so is 2 to 4 us, and the
+// predictor writes no vertices (22.4 -> 17.4 us at 50 005 bodies).
+// XCD parts: the workgroups on XCD x (block mod 8) take that XCD's tiles and
+// its part of the list, so that its L2 holds the bodies they read.
+template <int LAW>
+__global__ void __launch_bounds__(kBlock, LAW == LAW_STICKED ? 2 : 3) k_interact_list(Dev d, StepParams sp, int pii, int par) {
+  const int t = threadIdx.x;
+  const int x = (int)blockIdx.x & 7, kx = (int)blockIdx.x >> 3, nx = ((int)gridDim.x - x + 7) >> 3;
+  // every control word in one round of loads
+  const bool stop = frozen(d);
+  const ListState* ls = d.ls;
+  const int want = *(volatile const int*)&ls->want[par], gen = ls->gen, n0 = ls->cnt[0][x], n1 = ls->cnt[1][x];
+  if (stop) return;
+  if (blockIdx.x == 0 && t == 0) d.ls->want[1 - par] = 0;  // the next predictor sets it, nothing reads it now
+  // XCD x's tiles, as xcd_block shares them out
+  const int ntile = (d.ne + kListTile - 1) / kListTile, q8 = ntile >> 3, r8 = ntile & 7;
+  const int tile0 = x < r8 ? x * (q8 + 1) : r8 * (q8 + 1) + (x - r8) * q8;
+  const int tile1 = tile0 + q8 + (x < r8 ? 1 : 0);
+  ListItem* part = d.elist + (size_t)tile0 * kListTile;
+  // one round over the whole part, the workgroup's lanes taking every
+  // (nx 256)-th place; or a round per tile over the tile's own items
+  for (int tile = tile0 + kx; want ? tile < tile1 : tile == tile0 + kx; tile += nx) {
+    int2 r = make_int2(kx * kBlock, gen & 1 ? n1 : n0);
+    if (want) r = list_tile(d, tile * kListTile + t, part, &d.ls->cnt[(gen + 1) & 1][x]);
+    const int stride = want ? kBlock : nx * kBlock;
+    for (int k = r.x + t; k < r.y; k += stride) eval_item<LAW>(d, sp, pii, part[k]);
   }
 }
 
@@ -816,12 +1049,13 @@ __global__ void __launch_bounds__(kBlock) k_refresh_gaps(Dev d) {
     Kin k;
     k.deact = false;
     k.prev_dn = 0.0;
-    update_kinematics<false>(d, (int)(d.esub[e] >> 30), d.edesc[e], d.kin[d.ei[e]], d.kin[d.ej[e]], k);
+    update_kinematics_gv(d, (int)(d.esub[e] >> 30), d.edesc[e], d.kin[d.ei[e]].R, d.kin[d.ej[e]].R, k);
     d.edn[e] = k.deact ? 0.0 : k.dn;
   }
 }
 
 __global__ void __launch_bounds__(kBlock) k_reset_keys(Dev d) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) reset_list(d);
   for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < d.ne; e += gridDim.x * blockDim.x) d.ekey[e] = -INFINITY;
 }
 
@@ -1077,18 +1311,43 @@ __device__ __forceinline__ void predict_free(const Dev& d, const StepParams& sp,
 // The far-entry skip's motion bound of one predicted body: no vertex of it
 // moved by more than |dx| + 2 |dQ| rmax in this step (for unit quaternions
 // |Q' v Q'* - Q v Q*| <= 2 |Q' - Q| |v|), plus a rounding allowance.
-__device__ __forceinline__ void add_motion_bound_with(const Dev& d, int b, const BodyKin& old, const BodyKin& P,
-                                                      double cb, double rmax) {
+// It also sets the allowance ahead of it (24 steps of this motion, at least
+// ahead_min) and asks for a new evaluation list when the bound passes limit,
+// what the list in use was written for (a NaN does too).
+constexpr double kAheadSteps = 24.0;
+__device__ __forceinline__ void set_bound(const Dev& d, int b, double bound, double step, double limit, int par) {
+  d.cbound[b] = bound;
+  d.ahead[b] = bound + fmax(kAheadSteps * step, d.ahead_min);
+  if (!(bound <= limit)) d.ls->want[par] = 1;
+}
+__device__ __forceinline__ void add_motion_bound_with(const Dev& d, const StepParams& sp, int b, const BodyKin& old,
+                                                      const BodyKin& P, double cb, double rmax, double limit, int par) {
   if (!d.skip_far) return;
-  const double dx = P.px - old.px, dy = P.py - old.py, dz = P.pz - old.pz;
+  const double dx = P.px - old.px - sp.dt * d.drift[0], dy = P.py - old.py - sp.dt * d.drift[1],
+               dz = P.pz - old.pz - sp.dt * d.drift[2];
   const double qw = P.qw - old.qw, qx = P.qx - old.qx, qy = P.qy - old.qy, qz = P.qz - old.qz;
   const double step = sqrt(dx * dx + dy * dy + dz * dz) + 2.0 * sqrt(qw * qw + qx * qx + qy * qy + qz * qz) * rmax;
   const double mag = fabs(P.px) + fabs(P.py) + fabs(P.pz);
-  d.cbound[b] = cb + (step + 1e-15 * (1.0 + mag));
+  set_bound(d, b, cb + (step + 1e-15 * (1.0 + mag)), step, limit, par);
 }
-__device__ __forceinline__ void add_motion_bound(const Dev& d, int b, const BodyKin& old, const BodyKin& P) {
+// The driven bodies' bounds (by one workgroup): those without a control stay
+// where they are, which in the moving frame is a motion of |D|.  predict: the
+// step is taken now; relisted: the list in use was written in this step.
+__device__ __forceinline__ void driven_bounds(const Dev& d, const StepParams& sp, bool predict, bool relisted, int par) {
   if (!d.skip_far) return;
-  add_motion_bound_with(d, b, old, P, d.cbound[b], d.rmax[b]);
+  const double ux = sp.dt * d.drift[0], uy = sp.dt * d.drift[1], uz = sp.dt * d.drift[2];
+  const double step = sqrt(ux * ux + uy * uy + uz * uz);
+  for (int b = threadIdx.x; b < d.nDriven; b += blockDim.x) {
+    const double limit = relisted ? d.ahead[b] : d.climit[b];
+    if (relisted) d.climit[b] = limit;
+    const double cb = d.cbound[b];
+    if (predict && cb < INFINITY) set_bound(d, b, cb + (step + 1e-15), step, limit, par);
+  }
+}
+__device__ __forceinline__ void add_motion_bound(const Dev& d, const StepParams& sp, int b, const BodyKin& old,
+                                                 const BodyKin& P, int par) {
+  if (!d.skip_far) return;
+  add_motion_bound_with(d, sp, b, old, P, d.cbound[b], d.rmax[b], d.climit[b], par);
 }
 
 typedef double d2 __attribute__((ext_vector_type(2)));  // one 16-byte access
@@ -1201,7 +1460,7 @@ __device__ __forceinline__ double sum_chunk(const Dev& d, int k0, int k1, int la
 }
 
 template <int NB, bool BF>  // BF: the deck has a body force
-__global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, int kick, int guard, int fuse) {
+__global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, GatherArgs A) {
   constexpr int kLanes = kBlock / NB;      // lanes per body in the sums (8 or 4)
   constexpr int kComp = kLanes >= 6 ? 1 : 2;  // components per lane
   __shared__ double rec[NB * kRec];
@@ -1213,9 +1472,22 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, int 
   __shared__ double fm[NB][6];
   if (frozen(d)) return;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int kick = A.kick, guard = A.guard;
   const bool rst = guard && guard_reset(d);
   // (the check that follows this step freezes the later ones on the same words)
-  const bool predict = fuse && !rebuild_due(d);
+  const bool predict = A.fuse && !rebuild_due(d);
+  // this step's force phase wrote a new evaluation list
+  const bool relisted = A.listed && *(volatile const int*)&d.ls->want[A.par] != 0;
+  if (relisted && blockIdx.x == 0 && t == 0) {
+    const int g = d.ls->gen + 1;
+    for (int k = 0; k < 8; k++) d.ls->cnt[(g + 1) & 1][k] = 0;
+    d.ls->gen = g;
+    if (d.ls->again) {
+      d.ls->again = 0;
+      d.ls->want[1 - A.par] = 1;
+    }
+  }
+  if (blockIdx.x == 0 && (predict || relisted)) driven_bounds(d, sp, predict, relisted, 1 - A.par);
   GuardAcc ga;
   ga.kp = 0ull;
   ga.kw = ~0ull;
@@ -1252,7 +1524,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, int 
     r[1] = x.y;
   }
   const int b = b0 + t;
-  double mb = 1.0, cb = 0.0, rmx = 0.0;
+  double mb = 1.0, cb = 0.0, rmx = 0.0, lim = 0.0;
   v3 Ib = V(1.0, 1.0, 1.0);
   bool run = false;
   if (t < nbk) {
@@ -1262,7 +1534,9 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, int 
     if (predict && d.skip_far) {
       cb = d.cbound[b];
       rmx = d.rmax[b];
+      lim = relisted ? d.ahead[b] : d.climit[b];
     }
+    if (relisted) d.climit[b] = d.ahead[b];
   }
   // the summing lanes' bodies and slot ranges
   const int lb = t / kLanes, lc = t % kLanes;
@@ -1370,7 +1644,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, int 
     if (predict && !driven) {
       const BodyKin old = P;
       predict_free_with(sp, P, acc, arot);
-      add_motion_bound_with(d, b, old, P, cb, rmx);
+      add_motion_bound_with(d, sp, b, old, P, cb, rmx, lim, 1 - A.par);
     } else {
       store_resultants(d, b, F, M, acc, arot);
     }
@@ -1382,7 +1656,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, int 
       const double* r = rec + (k >> 3) * kRec + 2 * (k & 7);
       kd[k] = d2{r[0], r[1]};
     }
-  if (predict && !driven)
+  if (predict && !driven && A.glob != GLOB_NONE)
     for (int k = d.bvoff[b0] + t; k < d.bvoff[b0 + nbk]; k += kBlock) {
       const int bb = d.bvbody[k];
       if (d.soff[bb + 1] == d.soff[bb]) continue;
@@ -1902,10 +2176,13 @@ __global__ void __launch_bounds__(kBlock) k_drive(Dev d, StepParams sp, int driv
 
 // glob: also the global vertices of the free bodies with listed slots, from
 // the new pose (the driven bodies' follow in k_glob)
-__global__ void __launch_bounds__(kBlock) k_predict(Dev d, StepParams sp, int glob) {
+__global__ void __launch_bounds__(kBlock) k_predict(Dev d, StepParams sp, int glob, int par) {
   if (frozen(d)) return;
   const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  if (blockIdx.x == 0) drive_controls_block(d, sp);
+  if (blockIdx.x == 0) {
+    drive_controls_block(d, sp);
+    driven_bounds(d, sp, true, false, par);
+  }
   // free bodies (Rockable.cpp:2036-2055), a grid-stride loop
   for (int b = gid; b < d.nb; b += gridDim.x * blockDim.x) {
     if (b < d.nDriven) continue;
@@ -1913,7 +2190,7 @@ __global__ void __launch_bounds__(kBlock) k_predict(Dev d, StepParams sp, int gl
     const BodyKin old = P;
     predict_free(d, sp, b, P);
     store_predicted(d, b, P);
-    add_motion_bound(d, b, old, P);
+    add_motion_bound(d, sp, b, old, P, par);
     if (glob && d.soff[b + 1] != d.soff[b]) {
       const int v0 = d.bvoff[b], nv = d.bvoff[b + 1] - v0;
       for (int v = 0; v < nv; v++) st3(d.gv + 3 * (size_t)(v0 + v), glob_vertex(d.sh, P, v));
@@ -1931,7 +2208,7 @@ __global__ void __launch_bounds__(kBlock) k_predict(Dev d, StepParams sp, int gl
 // The driven bodies are moved by thread 0 of workgroup 0 (controls); with
 // driven_glob, workgroup 0 then writes their listed global vertices (else
 // k_glob does after this kernel).
-__global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, int driven_glob) {
+__global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, int driven_glob, int par) {
   __shared__ double rec[64 * kRec];
   __shared__ double pose[64][8];    // px py pz qw qx qy qz h
   __shared__ int shp[64];           // shape, or -1 if the body is not listed
@@ -1939,6 +2216,7 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
   const int t = threadIdx.x;
   if (blockIdx.x == 0) {
     drive_controls_block(d, sp);
+    driven_bounds(d, sp, true, false, par);
     if (driven_glob) {
       __syncthreads();  // the driven poses, written by thread 0, are visible to the workgroup
       for (int k = t; k < d.nvdriven; k += blockDim.x) {
@@ -1959,7 +2237,7 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
     // the body's other inputs loaded with the records, so that their
     // latencies overlap
     v3 acc = V(0.0, 0.0, 0.0), arot = acc;
-    double cb = 0.0, rmx = 0.0;
+    double cb = 0.0, rmx = 0.0, lim = 0.0;
     bool listed = false;
     if (t < 64 && b0 + t < bend) {
       const int b = b0 + t;
@@ -1968,6 +2246,7 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
       if (d.skip_far) {
         cb = d.cbound[b];
         rmx = d.rmax[b];
+        lim = d.climit[b];
       }
       listed = d.soff[b + 1] != d.soff[b];
     }
@@ -1981,7 +2260,7 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
         const BodyKin old = P;
         predict_free_with(sp, P, acc, arot);
         rec_store_motion(r, P);
-        add_motion_bound_with(d, b, old, P, cb, rmx);
+        add_motion_bound_with(d, sp, b, old, P, cb, rmx, lim, par);
         if (listed) {
           pose[t][0] = P.px;
           pose[t][1] = P.py;
@@ -2024,9 +2303,12 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
 // any of them stores, so the body is read whole before it is overwritten.
 // The driven bodies (controls by thread 0) and their vertices are left to
 // k_glob after it.
-__global__ void __launch_bounds__(kBlock) k_predict_vtx(Dev d, StepParams sp) {
+__global__ void __launch_bounds__(kBlock) k_predict_vtx(Dev d, StepParams sp, int par) {
   if (frozen(d)) return;
-  if (blockIdx.x == 0) drive_controls_block(d, sp);
+  if (blockIdx.x == 0) {
+    drive_controls_block(d, sp);
+    driven_bounds(d, sp, true, false, par);
+  }
   const int lane = threadIdx.x & 63;
   for (int wv = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6); wv < d.nwv;
        wv += (int)((gridDim.x * blockDim.x) >> 6)) {
@@ -2041,7 +2323,7 @@ __global__ void __launch_bounds__(kBlock) k_predict_vtx(Dev d, StepParams sp) {
     predict_free(d, sp, b, P);
     if (v == 0) {
       store_predicted(d, b, P);
-      add_motion_bound(d, b, old, P);
+      add_motion_bound(d, sp, b, old, P, par);
     }
     if (listed) st3(d.gv + 3 * (size_t)k, glob_vertex(d.sh, P, v));
   }
@@ -2121,6 +2403,10 @@ void launch_refresh_gaps(const Dev& d, hipStream_t s) {
   hipLaunchKernelGGL(k_refresh_gaps, dim3(std::min((d.ne + kBlock - 1) / kBlock, 65536)), dim3(kBlock), 0, s, d);
 }
 
+void launch_reset_list(const Dev& d, hipStream_t s) {
+  hipLaunchKernelGGL(k_reset_list, dim3(1), dim3(64), 0, s, d);
+}
+
 void launch_reset_keys(const Dev& d, hipStream_t s) {
   if (d.ne <= 0 || !d.ekey) return;
   hipLaunchKernelGGL(k_reset_keys, dim3(std::min((d.ne + kBlock - 1) / kBlock, 65536)), dim3(kBlock), 0, s, d);
@@ -2131,35 +2417,39 @@ void launch_entry_desc(const Dev& d, hipStream_t s) {
   hipLaunchKernelGGL(k_entry_desc, dim3((d.ne + kBlock - 1) / kBlock), dim3(kBlock), 0, s, d);
 }
 
-void launch_predict(const Dev& d, const StepParams& sp, int glob, hipStream_t s) {
+void launch_predict(const Dev& d, const StepParams& sp, int glob, int par, hipStream_t s) {
   const int n = d.nb > 0 ? d.nb : 1, bs = body_block(d);
-  const bool listed = glob && d.soff;  // else every body's vertices
+  if (glob == GLOB_NONE) {
+    hipLaunchKernelGGL(k_predict, grid_for(d, (n + bs - 1) / bs), dim3(bs), 0, s, d, sp, 0, par);
+    return;
+  }
+  const bool listed = glob == GLOB_LISTED && d.soff;  // else every body's vertices
   if (listed && d.fuse_glob == 3 && d.nb > d.nDriven) {
     // workgroups of 64 free bodies, their vertices from the poses in LDS; a
     // few driven bodies' vertices by workgroup 0 after the controls
     const int tiles = (d.nb - d.nDriven + 63) / 64;
     const int driven_glob = d.nvdriven <= 1024 ? 1 : 0;
-    hipLaunchKernelGGL(k_predict_blk, grid_for(d, tiles), dim3(kBlock), 0, s, d, sp, driven_glob);
+    hipLaunchKernelGGL(k_predict_blk, grid_for(d, tiles), dim3(kBlock), 0, s, d, sp, driven_glob, par);
     if (!driven_glob) launch_glob(d, 0, d.nvdriven, s);
     return;
   }
   if (listed && d.fuse_glob == 2 && d.nwv > 0) {
     // one thread per vertex of the free bodies, wavefronts of whole bodies
     const int wpb = kBlock / 64;
-    hipLaunchKernelGGL(k_predict_vtx, grid_for(d, (d.nwv + wpb - 1) / wpb), dim3(kBlock), 0, s, d, sp);
+    hipLaunchKernelGGL(k_predict_vtx, grid_for(d, (d.nwv + wpb - 1) / wpb), dim3(kBlock), 0, s, d, sp, par);
     launch_glob(d, 0, d.nvdriven, s);
     return;
   }
   const int fused = listed && d.fuse_glob != 0;  // the free bodies' in k_predict
-  hipLaunchKernelGGL(k_predict, grid_for(d, (n + bs - 1) / bs), dim3(bs), 0, s, d, sp, fused);
+  hipLaunchKernelGGL(k_predict, grid_for(d, (n + bs - 1) / bs), dim3(bs), 0, s, d, sp, fused, par);
   launch_glob(d, listed ? 0 : 1, fused ? d.nvdriven : d.nvtot, s);
 }
 
-void launch_drive(const Dev& d, const StepParams& sp, hipStream_t s) {
+void launch_drive(const Dev& d, const StepParams& sp, int glob, hipStream_t s) {
   if (d.nctrl <= 0) return;  // no body moves by a control: poses and vertices stay
-  const int driven_glob = d.nvdriven <= 1024 ? 1 : 0;
+  const int driven_glob = glob != GLOB_NONE && d.nvdriven <= 1024 ? 1 : 0;
   hipLaunchKernelGGL(k_drive, dim3(1), dim3(kBlock), 0, s, d, sp, driven_glob);
-  if (!driven_glob) launch_glob(d, 0, d.nvdriven, s);
+  if (glob != GLOB_NONE && !driven_glob) launch_glob(d, 0, d.nvdriven, s);
 }
 
 template <int BS>
@@ -2183,35 +2473,41 @@ void launch_fused_sorted(const Dev& d, const StepParams& sp, int write_geom_all,
     hipLaunchKernelGGL((k_interact<LAW_DEFAULT, GEOM_ALL, SORT>), g, bl, 0, s, d, sp, write_geom_all, 0);
 }
 
-template <int SEG>
-void launch_seg(const Dev& d, const StepParams& sp, hipStream_t s) {
-  const dim3 g = grid_for(d, (d.ne + SEG - 1) / SEG), bl(kBlock);
+bool uses_list(const Dev& d, int write_geom_all) {
+  return !write_geom_all && d.fuse_law && d.skip_far && d.skip_seg >= 512;
+}
+
+// The grid of the list kernel: a lane for each second entry (a list holds a
+// tenth to a third of them, bonds more), up to 2048 workgroups, twice what
+// the chip holds of it; a multiple of 8, so that every XCD part has its
+// workgroups.
+void launch_list(const Dev& d, const StepParams& sp, int par, hipStream_t s) {
+  const long want = ((long)d.ne + 2 * kBlock - 1) / (2 * kBlock);
+  const int g = (int)std::min(2048L, (want + 7) & ~7L);
+  const dim3 grid(std::max(8, persistent_grid(g, d.persist))), bl(kBlock);
+  if (d.skip_count) hipLaunchKernelGGL(k_count_skips, dim3(std::min((d.ne + kBlock - 1) / kBlock, 2048)), bl, 0, s, d);
   if (sp.law == LAW_AVALANCHE)
-    hipLaunchKernelGGL((k_interact_seg<LAW_AVALANCHE, SEG>), g, bl, 0, s, d, sp, 0);
+    hipLaunchKernelGGL((k_interact_list<LAW_AVALANCHE>), grid, bl, 0, s, d, sp, 0, par);
   else if (sp.law == LAW_STICKED)
-    hipLaunchKernelGGL((k_interact_seg<LAW_STICKED, SEG>), g, bl, 0, s, d, sp, d.paramsInInterfaces);
+    hipLaunchKernelGGL((k_interact_list<LAW_STICKED>), grid, bl, 0, s, d, sp, d.paramsInInterfaces, par);
   else
-    hipLaunchKernelGGL((k_interact_seg<LAW_DEFAULT, SEG>), g, bl, 0, s, d, sp, 0);
+    hipLaunchKernelGGL((k_interact_list<LAW_DEFAULT>), grid, bl, 0, s, d, sp, 0, par);
 }
 
 template <bool GEOM_ALL>
 void launch_fused(const Dev& d, const StepParams& sp, int write_geom_all, hipStream_t s) {
-  if (!GEOM_ALL && d.skip_far && d.skip_seg >= 512) {
-    switch (d.skip_seg) {
-      case 512: launch_seg<512>(d, sp, s); return;
-      case 2048: launch_seg<2048>(d, sp, s); return;
-      case 4096: launch_seg<4096>(d, sp, s); return;
-      default: launch_seg<1024>(d, sp, s); return;
-    }
-  }
   if (d.type_sort)
     launch_fused_sorted<GEOM_ALL, true>(d, sp, write_geom_all, s);
   else
     launch_fused_sorted<GEOM_ALL, false>(d, sp, write_geom_all, s);
 }
 
-void launch_interact(const Dev& d, const StepParams& sp, int write_geom_all, hipStream_t s) {
+void launch_interact(const Dev& d, const StepParams& sp, int write_geom_all, int par, hipStream_t s) {
   if (d.ne <= 0) return;
+  if (uses_list(d, write_geom_all)) {
+    launch_list(d, sp, par, s);
+    return;
+  }
   if (d.fuse_law) {
     if (write_geom_all)
       launch_fused<true>(d, sp, write_geom_all, s);
@@ -2256,19 +2552,20 @@ int gather_blocks(const Dev& d) {
 
 int gather_blocks_max(int nb, int nhch) { return nb + (nhch + 3) / 4 + 8; }
 
-void launch_gather(const Dev& d, const StepParams& sp, int kick, int guard, int fuse, hipStream_t s) {
+void launch_gather(const Dev& d, const StepParams& sp, GatherArgs A, hipStream_t s) {
   if (d.nb <= 0) return;
-  guard = guard && kick;
+  A.guard = A.guard && A.kick;
+  const int kick = A.kick, guard = A.guard;
   const dim3 blocks(gather_blocks(d));
   const bool bf = d.bf != BF_NONE, large = gather_bodies(d) == 64;
   if (large && bf)
-    hipLaunchKernelGGL((k_gather<64, true>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard, fuse);
+    hipLaunchKernelGGL((k_gather<64, true>), blocks, dim3(kBlock), 0, s, d, sp, A);
   else if (large)
-    hipLaunchKernelGGL((k_gather<64, false>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard, fuse);
+    hipLaunchKernelGGL((k_gather<64, false>), blocks, dim3(kBlock), 0, s, d, sp, A);
   else if (bf)
-    hipLaunchKernelGGL((k_gather<32, true>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard, fuse);
+    hipLaunchKernelGGL((k_gather<32, true>), blocks, dim3(kBlock), 0, s, d, sp, A);
   else
-    hipLaunchKernelGGL((k_gather<32, false>), blocks, dim3(kBlock), 0, s, d, sp, kick, guard, fuse);
+    hipLaunchKernelGGL((k_gather<32, false>), blocks, dim3(kBlock), 0, s, d, sp, A);
   if (d.nheavy > 0) {
     hipLaunchKernelGGL(k_heavy_finish, grid_for(d, d.nheavy), dim3(kBlock), 0, s, d, sp, kick, guard);
     if (d.nheavy_exact > 0)

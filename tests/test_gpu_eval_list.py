@@ -1,0 +1,55 @@
+"""The evaluation list of the steps that write no geometry records: counts
+around its tiles of 1024 entries and its eight parts, faces of three, four
+and more vertices, a flow whose motion is mostly common, against steps that
+evaluate every entry (skip_far 0): same bits, gaps and rebuild steps."""
+import numpy as np
+import pytest
+
+from rockable_amd import decks as D
+from tests.test_gpu_parity import assert_bodies_equal, assert_interactions_equal
+
+pytestmark = pytest.mark.gpu
+
+
+def _prism(n, h, r):
+    """A prism over a regular n-gon: two faces of n vertices."""
+    a = 2 * np.pi * np.arange(n) / n
+    v = np.array([(np.cos(x), np.sin(x), z) for z in (-0.5 * h, 0.5 * h) for x in a])
+    edge = [(k, (k + 1) % n) for k in range(n)] + [(n + k, n + (k + 1) % n) for k in range(n)] + \
+        [(k, n + k) for k in range(n)]
+    face = [list(range(n)), list(range(n, 2 * n))] + [[k, (k + 1) % n, n + (k + 1) % n, n + k] for k in range(n)]
+    return D.Shape("PRISM%d" % n, r, v, edge, face, volume=0.5 * n * np.sin(2 * np.pi / n) * h,
+                   inertia_mass=(0.3, 0.3, 0.4))
+
+
+@pytest.mark.parametrize("n,flow", [(1, 0.0), (30, 0.0), (200, 0.0), (200, 3.0), (700, -5.0)])
+def test_list_equals_full_evaluation(tmp_path, n, flow):
+    from rockable_amd.engine import Engine
+    rng = np.random.default_rng(n)
+    walls, wb = D.box_walls((-0.2, -0.03, 0.0), (0.4, 0.08, 0.2), 2e-4)
+    pool = [_prism(k, 0.8, 0.05) for k in (3, 4, 5, 7)] + [D.sphere_shape("BALL", 0.6)]
+    deck = D.Deck(dt=1e-6, tmax=1.0, interVerlet=3e-5, DVerlet=6e-4, dVerlet=3e-4, density={0: 2700.0, 1: 2700.0},
+                  gravity=(20.0, 0.0, -90.0), update_nl="linkCells", nDriven=len(wb), force_law="Avalanche",
+                  params=D.contact_params(1e6, 8e5, 0.25, 0.4, groups=((0, 0), (0, 1))))
+    deck.cell_min_sizes = (0.012, 0.012, 0.012)
+    deck.box_for_linkcells_opt = 1
+    deck.bodies = list(wb)
+    for k in range(n):
+        p = (0.006 + 0.0097 * (k % 6), 0.006 + 0.0097 * (k // 6 % 5), 0.0046 + 0.0091 * (k // 30))
+        v = rng.uniform(-1.0, 1.0, 3) + (flow, 0.0, -1.0)
+        deck.bodies.append(D.Body(pool[k % len(pool)].name, homothety=0.0042, pos=p, vel=tuple(v),
+                                  Q=tuple(D.small_rotations(rng, 1, 0.1)[0]), vrot=tuple(rng.uniform(-50, 50, 3))))
+    path = D.write_deck(str(tmp_path), walls + pool, deck)
+    a, b = Engine(path), Engine(path)
+    for e, skip in ((a, 1), (b, 0)):
+        e.set_option("record_geometry", 0)
+        e.set_option("skip_far", skip)
+        e.update_nl()
+    contacts = 0
+    for steps in (1, 40, 300, 400):
+        a.step(steps)
+        b.step(steps)
+        assert_bodies_equal(a.bodies(), b.bodies())
+        assert_interactions_equal(a.interactions(), b.interactions(), fields=("dn", "fn", "ft", "mom", "damp", "stick"))
+        contacts += a.counts()["nactive"]
+    assert contacts > 0 or n < 200  # the bodies met
