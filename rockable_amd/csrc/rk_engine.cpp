@@ -985,9 +985,7 @@ int run_accelerations(rk_engine* eng, int kick, int write_geom, bool guard = fal
   launch_interact(eng->d, sp, geom_all, eng->parity, eng->stream);
   toc(eng, "interact", 2);
   const bool bonds = eng->m.law == LAW_STICKED && eng->live_interfaces > 0;
-  if (bonds) {
-    // before the resultants (it touches the bonds' state, which they do not
-    // read), so that their fused predictor knows of a breakage
+  if (bonds && !guard) {  // (a guarded step breaks its bonds at its end)
     tic(eng, 2);
     launch_breakage(eng->d, sp, eng->stream);
     toc(eng, "breakage", 2);
@@ -1081,7 +1079,7 @@ int vv_step(rk_engine* eng, int write_geom, bool guard, bool next) {
   if (run_accelerations(eng, 1, write_geom, guard, fuse) != 0) return -1;
   if (guard) {
     tic(eng, 2);
-    launch_guard(eng->d, eng->stream);
+    launch_guard(eng->d, sp, fuse ? 1 : 0, eng->stream);
     toc(eng, "guard", 2);
   }
   if (fuse) {

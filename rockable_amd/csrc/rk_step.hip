@@ -18,7 +18,9 @@
 //               serial order of the reference, + compute_accelerations_from_
 //               resultants (3419-3552) + the closing kick (2120-2155)
 //   k_gather_heavy  the same for bodies with many slots, one workgroup each
-//   k_breakage  breakage_of_interfaces (3350-3413)
+//   k_guard_check  the end of a guarded step: breakage_of_interfaces
+//               (3350-3413; k_breakage in steps without the guard) and the
+//               displacement check
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -433,7 +435,10 @@ __device__ void law_sticked(const Dev& d, const ContactPar& cp, const double bp[
     const double pt = power == 2.0 ? rt * rt : pow(rt, power);
     const double pm = power == 2.0 ? rm * rm : pow(rm, power);
     double yield = pt + pm - h.fn / fn0 - 1.0;
-    if (yield > 0.0) d.ifc.brk[stick] = 1;  // idempotent byte store, consumed after the resultants
+    if (yield > 0.0) {  // idempotent stores, consumed at the end of the step
+      d.ifc.brk[stick] = 1;
+      d.flags[0] = 1;
+    }
   } else {
     if (k.dn > 0.0) {
       h.fn = 0.0;
@@ -1491,7 +1496,8 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, Gath
   GuardAcc ga;
   ga.kp = 0ull;
   ga.kw = ~0ull;
-  const int nchunk = (d.nhch + kBlock / 64 - 1) / (kBlock / 64);
+  // (gather_blocks sizes the grid by the same rule)
+  const int nchunk = A.fuse && !d.guard_on ? 0 : (d.nhch + kBlock / 64 - 1) / (kBlock / 64);
   const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
   const bool driven = tile < d.nDriven, chunks = !driven && tile < d.nDriven + nchunk;
   const int b0 = driven ? tile : d.nDriven + (tile - d.nDriven - nchunk) * NB;
@@ -1499,7 +1505,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, Gath
   int k0 = 0, kend = 0;
   if (chunks) {
     const int c = (tile - d.nDriven) * (kBlock / 64) + wv;
-    if (c < d.nhch) {
+    if (c < d.nhch && !predict) {
       const int2 r = d.hch[c];
       const double s = sum_chunk(d, r.x, r.y, lane, vals + 64 * 6 * wv);
       if (lane < 6) d.hpart[6 * (size_t)c + lane] = s;
@@ -1510,6 +1516,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, Gath
   }
   if (chunks || (driven && kend - k0 > d.heavy_min)) {  // no body to finish
     if (guard && t == 0) {
+      if (A.fuse && !chunks) guard_body(d, sp, b0, d.kin[b0], rst, ga);  // (else k_heavy_finish does)
       d.gpart[2 * (size_t)blockIdx.x] = ga.kp;
       d.gpart[2 * (size_t)blockIdx.x + 1] = ga.kw;
     }
@@ -1692,15 +1699,14 @@ __device__ __forceinline__ void guard_heavy(const Dev& d, const StepParams& sp, 
   if (a.kw != ~0ull) atomicMin(&d.guard->minw, a.kw);
 }
 
-static_assert(kBlock == 256, "k_heavy_finish combines four wavefronts");
-__global__ void __launch_bounds__(kBlock) k_heavy_finish(Dev d, StepParams sp, int kick, int guard) {
+static_assert(kBlock == 256, "heavy_finish combines four wavefronts");
+// heavy body h, by the first 256 threads of a workgroup (every thread calls it)
+__device__ __forceinline__ void heavy_finish(const Dev& d, const StepParams& sp, int kick, int guard, int h) {
   __shared__ double red[kBlock / 64][6];
-  if (frozen(d)) return;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  for (TileLoop T = xcd_tiles(d.nheavy); T.t < T.end; T.t += T.step) {
-    const int h = T.t;
-    const int b = d.heavy[h];
-    if (!d.passive[b] || d.exact_sums) continue;  // the same for the whole workgroup
+  const int b = d.heavy[h];
+  if (!d.passive[b] || d.exact_sums) return;  // the same for the whole workgroup
+  if (t < kBlock) {
     double a[6] = {-0.0, -0.0, -0.0, -0.0, -0.0, -0.0};
     for (int c = d.hch_off[h] + t; c < d.hch_off[h + 1]; c += kBlock) {
       const double* p = d.hpart + 6 * (size_t)c;
@@ -1714,21 +1720,26 @@ __global__ void __launch_bounds__(kBlock) k_heavy_finish(Dev d, StepParams sp, i
     if (lane == 0)
 #pragma unroll
       for (int q = 0; q < 6; q++) red[wv][q] = a[q];
-    __syncthreads();
-    if (t == 0) {
-#pragma unroll
-      for (int q = 0; q < 6; q++) a[q] = (red[0][q] + red[1][q]) + (red[2][q] + red[3][q]);
-      BodyKin P = d.kin[b];
-      const bool driven = b < d.nDriven;
-      v3 F, M;
-      int c0, c1;
-      init_resultants(d, b, P, driven, F, M, c0, c1);
-      finish_body(d, sp, kick, b, P, driven, vadd(F, V(a[0], a[1], a[2])), vadd(M, V(a[3], a[4], a[5])), c0, c1,
-                  d.mass[b], ld3(d.inertia + 3 * (size_t)b));
-      if (guard) guard_heavy(d, sp, b, P);
-    }
-    __syncthreads();
   }
+  __syncthreads();
+  if (t == 0) {
+    double a[6];
+#pragma unroll
+    for (int q = 0; q < 6; q++) a[q] = (red[0][q] + red[1][q]) + (red[2][q] + red[3][q]);
+    BodyKin P = d.kin[b];
+    const bool driven = b < d.nDriven;
+    v3 F, M;
+    int c0, c1;
+    init_resultants(d, b, P, driven, F, M, c0, c1);
+    finish_body(d, sp, kick, b, P, driven, vadd(F, V(a[0], a[1], a[2])), vadd(M, V(a[3], a[4], a[5])), c0, c1,
+                d.mass[b], ld3(d.inertia + 3 * (size_t)b));
+    if (guard) guard_heavy(d, sp, b, P);
+  }
+  __syncthreads();
+}
+__global__ void __launch_bounds__(kBlock) k_heavy_finish(Dev d, StepParams sp, int kick, int guard) {
+  if (frozen(d)) return;
+  for (TileLoop T = xcd_tiles(d.nheavy); T.t < T.end; T.t += T.step) heavy_finish(d, sp, kick, guard, T.t);
 }
 
 // compute_resultants for a heavy body that is not passive (or any heavy
@@ -1791,6 +1802,64 @@ __global__ void __launch_bounds__(kBlock) k_gather_heavy(Dev d, StepParams sp, i
   }
 }
 
+// locate entry (owner, other, sub) in the owner's sorted run
+__device__ int find_entry(const Dev& d, int owner, int other, uint32_t sub) {
+  int lo = d.istart[owner], hi = d.istart[owner + 1];
+  while (lo < hi) {
+    int mid = (lo + hi) >> 1;
+    bool less = (d.ej[mid] < other) || (d.ej[mid] == other && d.esub[mid] < sub);
+    if (less)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  if (lo < d.istart[owner + 1] && d.ej[lo] == other && d.esub[lo] == sub) return lo;
+  return -1;
+}
+
+// breakage_of_interfaces (Rockable.cpp:3350-3413) for interface k
+__device__ void break_interface(const Dev& d, int k) {
+  if (!d.ifc.brk[k]) return;
+  d.ifc.brk[k] = 0;
+  if (!d.ifc.alive[k]) return;
+  const uint64_t key = d.ifc.key[k];
+  const int bi = (int)(key >> 32), bj = (int)(key & 0xffffffffu);
+  const int g1 = d.kin[bi].group, g2 = d.kin[bj].group;
+  for (int q = d.ifc.bond_off[k]; q < d.ifc.bond_off[k + 1]; q++) {
+    const int* bk = d.ifc.bond_key + 3 * q;
+    const int e = find_entry(d, bi, bj, pack_sub(bk[0], bk[1], bk[2]));
+    if (e < 0) continue;
+    d.estick[e] = -1;
+    EState s = d.est[e];
+    if (d.edn[e] >= 0.0) {
+      s.fn = 0.0;
+      s.ftx = s.fty = s.ftz = 0.0;
+    } else {
+      v3 T = V(s.ftx, s.fty, s.ftz);
+      double FT = vnormalize(&T);
+      double mu = prm(d.par, P_MU, g1, g2);
+      double thr = fabs(mu * s.fn);
+      if (FT > thr) {
+        v3 ft = vsc(thr, T);
+        s.ftx = ft.x;
+        s.fty = ft.y;
+        s.ftz = ft.z;
+      }
+    }
+    d.est[e] = s;
+  }
+  d.ifc.alive[k] = 0;
+  // for the host's accounting (it sorts them: interface order); an interface
+  // breaks once, so the list holds at most n
+  d.ifc.broken[atomicAdd(d.ifc.nbroken, 1)] = k;
+  d.flags[0] = 1;  // needUpdate
+}
+__global__ void k_breakage(Dev d) {
+  if (frozen(d)) return;
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < d.ifc.n) break_interface(d, k);
+}
+
 // the end of a step of the integrate() loop (Rockable.cpp:2690-2740): a
 // needUpdate left by the previous check makes the rebuild due now (the step
 // kernels then wait for the host); then the check itself, on the maxima of
@@ -1798,9 +1867,20 @@ __global__ void __launch_bounds__(kBlock) k_gather_heavy(Dev d, StepParams sp, i
 // on the order).  The step index lives on the device, so that a captured
 // sequence of steps replays as is.
 constexpr int kCheckBlock = 1024;
-__global__ void __launch_bounds__(kCheckBlock) k_guard_check(Dev d, int nparts) {
+// One launch ends the step: where the law marked a bond (flags), the interfaces
+// are broken here, and where a fused step turns out to be the last before a
+// rebuild, the passive heavy bodies are finished here (fused steps that go on
+// leave them: nothing reads their sums).  Apart, the breakage kernel and
+// k_heavy_finish took a launch each at every step, 4 to 6 us of nothing.
+__global__ void __launch_bounds__(kCheckBlock) k_guard_check(Dev d, StepParams sp, int nparts, int fuse) {
   __shared__ unsigned long long red[2][kCheckBlock / 64];
   if (frozen(d)) return;
+  if (*(volatile const int*)d.flags != 0 && d.ifc.n > 0) {
+    for (int k = threadIdx.x; k < d.ifc.n; k += kCheckBlock) break_interface(d, k);
+    __syncthreads();
+  }
+  if (fuse && rebuild_due(d))
+    for (int h = 0; h < d.nheavy; h++) heavy_finish(d, sp, 1, 0, h);
   unsigned long long kp = 0ull, kw = ~0ull;
   for (int k = threadIdx.x; k < nparts; k += kCheckBlock) {
     const unsigned long long p = d.gpart[2 * (size_t)k], w = d.gpart[2 * (size_t)k + 1];
@@ -2329,60 +2409,6 @@ __global__ void __launch_bounds__(kBlock) k_predict_vtx(Dev d, StepParams sp, in
   }
 }
 
-// locate entry (owner, other, sub) in the owner's sorted run
-__device__ int find_entry(const Dev& d, int owner, int other, uint32_t sub) {
-  int lo = d.istart[owner], hi = d.istart[owner + 1];
-  while (lo < hi) {
-    int mid = (lo + hi) >> 1;
-    bool less = (d.ej[mid] < other) || (d.ej[mid] == other && d.esub[mid] < sub);
-    if (less)
-      lo = mid + 1;
-    else
-      hi = mid;
-  }
-  if (lo < d.istart[owner + 1] && d.ej[lo] == other && d.esub[lo] == sub) return lo;
-  return -1;
-}
-
-__global__ void k_breakage(Dev d) {
-  if (frozen(d)) return;
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= d.ifc.n || !d.ifc.brk[k]) return;
-  d.ifc.brk[k] = 0;
-  if (!d.ifc.alive[k]) return;
-  const uint64_t key = d.ifc.key[k];
-  const int bi = (int)(key >> 32), bj = (int)(key & 0xffffffffu);
-  const int g1 = d.kin[bi].group, g2 = d.kin[bj].group;
-  for (int q = d.ifc.bond_off[k]; q < d.ifc.bond_off[k + 1]; q++) {
-    const int* bk = d.ifc.bond_key + 3 * q;
-    const int e = find_entry(d, bi, bj, pack_sub(bk[0], bk[1], bk[2]));
-    if (e < 0) continue;
-    d.estick[e] = -1;
-    EState s = d.est[e];
-    if (d.edn[e] >= 0.0) {
-      s.fn = 0.0;
-      s.ftx = s.fty = s.ftz = 0.0;
-    } else {
-      v3 T = V(s.ftx, s.fty, s.ftz);
-      double FT = vnormalize(&T);
-      double mu = prm(d.par, P_MU, g1, g2);
-      double thr = fabs(mu * s.fn);
-      if (FT > thr) {
-        v3 ft = vsc(thr, T);
-        s.ftx = ft.x;
-        s.fty = ft.y;
-        s.ftz = ft.z;
-      }
-    }
-    d.est[e] = s;
-  }
-  d.ifc.alive[k] = 0;
-  // for the host's accounting (it sorts them: interface order); an interface
-  // breaks once, so the list holds at most n
-  d.ifc.broken[atomicAdd(d.ifc.nbroken, 1)] = k;
-  d.flags[0] = 1;  // needUpdate
-}
-
 }  // namespace
 
 int body_block(const Dev& d) { return d.body_block == 64 || d.body_block == 128 ? d.body_block : 256; }
@@ -2545,9 +2571,9 @@ int gather_bodies(const Dev& d) { return d.nb - d.nDriven >= kGatherLarge ? 64 :
 
 // k_gather's workgroups: one per driven body, the heavy chunks four to one,
 // the free bodies
-int gather_blocks(const Dev& d) {
+int gather_blocks(const Dev& d, int fuse) {
   const int nb = gather_bodies(d);
-  return d.nDriven + (d.nhch + 3) / 4 + (d.nb - d.nDriven + nb - 1) / nb;
+  return d.nDriven + (fuse && !d.guard_on ? 0 : (d.nhch + 3) / 4) + (d.nb - d.nDriven + nb - 1) / nb;
 }
 
 int gather_blocks_max(int nb, int nhch) { return nb + (nhch + 3) / 4 + 8; }
@@ -2556,7 +2582,7 @@ void launch_gather(const Dev& d, const StepParams& sp, GatherArgs A, hipStream_t
   if (d.nb <= 0) return;
   A.guard = A.guard && A.kick;
   const int kick = A.kick, guard = A.guard;
-  const dim3 blocks(gather_blocks(d));
+  const dim3 blocks(gather_blocks(d, A.fuse));
   const bool bf = d.bf != BF_NONE, large = gather_bodies(d) == 64;
   if (large && bf)
     hipLaunchKernelGGL((k_gather<64, true>), blocks, dim3(kBlock), 0, s, d, sp, A);
@@ -2566,7 +2592,7 @@ void launch_gather(const Dev& d, const StepParams& sp, GatherArgs A, hipStream_t
     hipLaunchKernelGGL((k_gather<32, true>), blocks, dim3(kBlock), 0, s, d, sp, A);
   else
     hipLaunchKernelGGL((k_gather<32, false>), blocks, dim3(kBlock), 0, s, d, sp, A);
-  if (d.nheavy > 0) {
+  if (d.nheavy > 0 && !A.fuse) {
     hipLaunchKernelGGL(k_heavy_finish, grid_for(d, d.nheavy), dim3(kBlock), 0, s, d, sp, kick, guard);
     if (d.nheavy_exact > 0)
       hipLaunchKernelGGL(k_gather_heavy, dim3(d.nheavy), dim3(kBlock), 0, s, d, sp, kick, guard);
@@ -2725,9 +2751,9 @@ __global__ void k_guard_set_step(Dev d, long long step) {
   if (threadIdx.x == 0) d.guard->step = step;
 }
 
-void launch_guard(const Dev& d, hipStream_t s) {
-  const int nparts = (d.disp_check && d.nb > 0) ? gather_blocks(d) : 0;
-  hipLaunchKernelGGL(k_guard_check, dim3(1), dim3(kCheckBlock), 0, s, d, nparts);
+void launch_guard(const Dev& d, const StepParams& sp, int fuse, hipStream_t s) {
+  const int nparts = (d.disp_check && d.nb > 0) ? gather_blocks(d, fuse) : 0;
+  hipLaunchKernelGGL(k_guard_check, dim3(1), dim3(kCheckBlock), 0, s, d, sp, nparts, fuse);
 }
 
 void launch_guard_set_step(const Dev& d, long long step, hipStream_t s) {
