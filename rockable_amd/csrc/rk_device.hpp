@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <cstdint>
 
+#include "../../include/rockable_amd.h"
 #include "rk_math.hpp"
 
 namespace rk {
@@ -404,6 +405,14 @@ void launch_drive(const Dev& d, const StepParams& sp, int glob, hipStream_t s);
 // capacity of gpart for any launch shape
 int gather_blocks_max(int nb, int nhch);
 void launch_breakage(const Dev& d, const StepParams& sp, hipStream_t s);
+// Read-outs packed on the device.  The bodies' kinematics as four arrays (3,
+// 4, 3 and 3 doubles per body: pos, Q, vel, vrot), out holding 13 nb doubles;
+void launch_pack_bodies(const Dev& d, double* out, hipStream_t s);
+// the active entries' count (block: active_blocks(d) + 1 integers, the last
+// one the count) and their records in entry order, at most cap of them.
+int active_blocks(const Dev& d);
+void launch_active_count(const Dev& d, int32_t* block, hipStream_t s);
+void launch_active_records(const Dev& d, const int32_t* block, rk_interaction* out, int cap, hipStream_t s);
 // statistics: part holds stat_parts(d) doubles, out 9 doubles (KE translation,
 // KE rotation, max |v|, free bodies, active, contacts, active pairs, sum dn,
 // min dn over contacts)

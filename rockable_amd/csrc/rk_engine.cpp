@@ -53,6 +53,14 @@ struct rk_engine {
   int persist = 0;
   // host wall time of the rebuilds while the autotuner runs (it synchronises
   // after each rebuild then)
+  // read-outs packed on the device: the bodies' kinematics, the active
+  // entries' block counts and records (kept, grown as needed, freed with the deck)
+  double* pack_bodies = nullptr;
+  size_t pack_bodies_cap = 0;
+  int32_t* active_block = nullptr;
+  size_t active_block_cap = 0;
+  rk_interaction* active_rec = nullptr;
+  size_t active_rec_cap = 0;
   double* stat_part = nullptr;
   double* stat_out = nullptr;
   size_t stat_cap = 0;
@@ -218,6 +226,19 @@ int upload(rk_engine* eng, T*& dst, const std::vector<T>& src) {
   return 0;
 }
 
+// A buffer kept between calls, at least n elements.
+template <class T>
+int grow(rk_engine* eng, T*& p, size_t& cap, size_t n) {
+  if (n <= cap) return 0;
+  if (p) (void)hipFree(p);
+  p = nullptr;
+  cap = 0;
+  const size_t c = n + n / 4 + 64;
+  HIPCHK(hipMalloc(&p, c * sizeof(T)));
+  cap = c;
+  return 0;
+}
+
 void free_graphs(rk_engine* eng) {
   for (auto& g : eng->graphs)
     if (g.exec) (void)hipGraphExecDestroy(g.exec);
@@ -234,6 +255,7 @@ void free_device(rk_engine* eng) {
                 eng->ifc_brk,  eng->ifc_broken, eng->ifc_nbroken, eng->ctrl,      eng->ctrl_off,  eng->ctrl_idx,  eng->flags,    eng->passive,
                 eng->gv,       eng->bvoff,     eng->bvbody,    eng->guard,     eng->gdpos,    eng->gdq,      eng->gpart,
                 eng->beoff,    eng->bfoff,     eng->cbound,    eng->rmax,  eng->ahead, eng->climit, eng->drift, eng->ls,
+                eng->pack_bodies, eng->active_block, eng->active_rec,
                 eng->feat,     eng->pred,      eng->feat_part, eng->stat_part, eng->stat_out};
   for (void* p : ps)
     if (p) (void)hipFree(p);
@@ -241,6 +263,10 @@ void free_device(rk_engine* eng) {
   eng->acc = eng->arot = eng->force = eng->moment = eng->mass = eng->inertia = eng->bf_surface = nullptr;
   eng->cbound = eng->rmax = eng->ahead = eng->climit = eng->drift = nullptr;
   eng->ls = nullptr;
+  eng->pack_bodies = nullptr;
+  eng->active_block = nullptr;
+  eng->active_rec = nullptr;
+  eng->pack_bodies_cap = eng->active_block_cap = eng->active_rec_cap = 0;
   eng->cluster = nullptr;
   eng->sh_nv = eng->sh_ne = eng->sh_nf = eng->sh_voff = eng->sh_eoff = eng->sh_foff = eng->sh_edge = nullptr;
   eng->sh_fstart = eng->sh_fidx = nullptr;
@@ -2550,12 +2576,15 @@ int rk_get_counts(rk_engine* eng, rk_counts* out) {
   out->nbodies = (int64_t)eng->m.bodies.size();
   out->ndriven = eng->m.nDriven;
   out->nlisted = E.n;
-  int64_t na = 0;
+  int32_t na = 0;
   if (E.n > 0) {
-    std::vector<uint8_t> act(E.n);
+    (void)hipSetDevice(eng->device);
+    const int nblk = active_blocks(eng->d);
+    if (grow(eng, eng->active_block, eng->active_block_cap, (size_t)nblk + 1) != 0) return -1;
+    launch_active_count(eng->d, eng->active_block, eng->stream);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(&na, eng->active_block + nblk, sizeof na, hipMemcpyDeviceToHost, eng->stream));
     HIPCHK(hipStreamSynchronize(eng->stream));
-    HIPCHK(hipMemcpy(act.data(), E.eact, E.n, hipMemcpyDeviceToHost));
-    for (uint8_t a : act) na += a & 1;
   }
   out->nactive = na;
   out->ninterfaces = eng->live_interfaces;
@@ -2576,31 +2605,24 @@ int rk_get_counts(rk_engine* eng, rk_counts* out) {
 int rk_get_bodies(rk_engine* eng, double* pos, double* Q, double* vel, double* vrot, double* acc, double* arot,
                   double* force, double* moment, size_t nbodies) {
   if (check_loaded(eng)) return -1;
-  if (nbodies < eng->m.bodies.size()) return fail(eng, "output arrays too small");
-  if (download_bodies(eng) != 0) return -1;
-  for (size_t b = 0; b < eng->m.bodies.size(); b++) {
-    const Body& p = eng->m.bodies[b];
-    auto put = [&](double* a, v3 v) {
-      if (a) {
-        a[3 * b] = v.x;
-        a[3 * b + 1] = v.y;
-        a[3 * b + 2] = v.z;
-      }
-    };
-    put(pos, p.pos);
-    put(vel, p.vel);
-    put(vrot, p.vrot);
-    put(acc, p.acc);
-    put(arot, p.arot);
-    put(force, p.force);
-    put(moment, p.moment);
-    if (Q) {
-      Q[4 * b] = p.Q.w;
-      Q[4 * b + 1] = p.Q.x;
-      Q[4 * b + 2] = p.Q.y;
-      Q[4 * b + 3] = p.Q.z;
-    }
-  }
+  (void)hipSetDevice(eng->device);
+  const size_t nb = eng->m.bodies.size();
+  if (nbodies < nb) return fail(eng, "output arrays too small");
+  if (nb == 0) return 0;
+  if (flush_steps(eng) != 0) return -1;
+  if (grow(eng, eng->pack_bodies, eng->pack_bodies_cap, 13 * nb) != 0) return -1;
+  const double* k = eng->pack_bodies;
+  if (pos || Q || vel || vrot) launch_pack_bodies(eng->d, eng->pack_bodies, eng->stream);
+  HIPCHK(hipGetLastError());
+  const struct {
+    double* to;
+    const double* from;
+    size_t per;
+  } copies[] = {{pos, k, 3},         {Q, k + 3 * nb, 4},     {vel, k + 7 * nb, 3},     {vrot, k + 10 * nb, 3},
+                {acc, eng->acc, 3}, {arot, eng->arot, 3}, {force, eng->force, 3}, {moment, eng->moment, 3}};
+  for (const auto& c : copies)
+    if (c.to) HIPCHK(hipMemcpyAsync(c.to, c.from, c.per * nb * sizeof(double), hipMemcpyDeviceToHost, eng->stream));
+  HIPCHK(hipStreamSynchronize(eng->stream));
   return 0;
 }
 
@@ -2645,6 +2667,28 @@ int rk_set_bodies(rk_engine* eng, const double* pos, const double* Q, const doub
 
 int rk_get_interactions(rk_engine* eng, int active_only, rk_interaction* out, size_t cap, size_t* n) {
   if (check_loaded(eng)) return -1;
+  (void)hipSetDevice(eng->device);
+  if (!active_only && !out) {
+    if (n) *n = (size_t)eng->E[eng->cur].n;
+    return 0;
+  }
+  if (active_only) {
+    if (flush_steps(eng) != 0) return -1;
+    const int nblk = active_blocks(eng->d);
+    const int room = (int)std::min<size_t>(out ? cap : 0, (size_t)std::max(0, eng->d.ne));
+    if (grow(eng, eng->active_block, eng->active_block_cap, (size_t)nblk + 1) != 0) return -1;
+    if (room > 0 && grow(eng, eng->active_rec, eng->active_rec_cap, (size_t)room) != 0) return -1;
+    launch_active_count(eng->d, eng->active_block, eng->stream);
+    launch_active_records(eng->d, eng->active_block, eng->active_rec, room, eng->stream);
+    HIPCHK(hipGetLastError());
+    int32_t total = 0;
+    HIPCHK(hipMemcpyAsync(&total, eng->active_block + nblk, sizeof total, hipMemcpyDeviceToHost, eng->stream));
+    HIPCHK(hipStreamSynchronize(eng->stream));
+    const size_t k = std::min<size_t>((size_t)room, (size_t)total);
+    if (k > 0) HIPCHK(hipMemcpy(out, eng->active_rec, k * sizeof(rk_interaction), hipMemcpyDeviceToHost));
+    if (n) *n = (size_t)total;
+    return 0;
+  }
   std::vector<Inter> v;
   if (download_interactions(eng, active_only, v) != 0) return -1;
   if (n) *n = v.size();

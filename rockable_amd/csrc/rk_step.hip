@@ -2409,6 +2409,115 @@ __global__ void __launch_bounds__(kBlock) k_predict_vtx(Dev d, StepParams sp, in
   }
 }
 
+// The bodies' kinematics as the arrays the caller reads (pos, Q, vel, vrot):
+// one thread per double of the 13, so that the records are read and the arrays
+// written in near-contiguous runs.
+__global__ void __launch_bounds__(kBlock) k_pack_bodies(Dev d, double* out) {
+  const long n = 13l * d.nb;
+  const double* kin = reinterpret_cast<const double*>(d.kin);
+  for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (long)gridDim.x * blockDim.x) {
+    const long b = k / 13;
+    const int c = (int)(k - 13 * b);
+    const double x = kin[16 * b + c];
+    const long nb = d.nb;
+    const long at = c < 3 ? 3 * b + c : c < 7 ? 3 * nb + 4 * b + (c - 3) : c < 10 ? 7 * nb + 3 * b + (c - 7)
+                                                                       : 10 * nb + 3 * b + (c - 10);
+    out[at] = x;
+  }
+}
+
+// The active entries' records for a read-out, in entry order: counts per
+// block of 1024 entries, their scan by one workgroup, the records.  The host
+// copies only those (176 bytes each) instead of every listed entry's arrays
+// (206 bytes, one in ten active in a settled packing).
+constexpr int kActiveTile = 1024;
+__global__ void __launch_bounds__(kBlock) k_active_count(Dev d, int32_t* block) {
+  __shared__ int w[kBlock / 64];
+  int n = 0;
+  for (int r = 0; r < kActiveTile / kBlock; r++) {
+    const int e = blockIdx.x * kActiveTile + r * kBlock + (int)threadIdx.x;
+    n += __popcll(__ballot(e < d.ne && (d.eact[e] & 1)));
+  }
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) block[blockIdx.x] = w[0] + w[1] + w[2] + w[3];
+}
+// exclusive, in place; the total after the last block's
+__global__ void __launch_bounds__(kBlock) k_active_scan(int n, int32_t* block) {
+  __shared__ int sc[kBlock];
+  const int t = threadIdx.x;
+  int carry = 0;
+  for (int b0 = 0; b0 < n; b0 += kBlock) {
+    const int v = b0 + t < n ? block[b0 + t] : 0;
+    sc[t] = v;
+    for (int o = 1; o < kBlock; o <<= 1) {
+      __syncthreads();
+      const int x = t >= o ? sc[t - o] : 0;
+      __syncthreads();
+      sc[t] += x;
+    }
+    __syncthreads();
+    if (b0 + t < n) block[b0 + t] = carry + sc[t] - v;
+    carry += sc[kBlock - 1];
+    __syncthreads();
+  }
+  if (t == 0) block[n] = carry;
+}
+__global__ void __launch_bounds__(kBlock) k_active_records(Dev d, const int32_t* block, rk_interaction* out, int cap) {
+  __shared__ int w[kActiveTile / kBlock][kBlock / 64];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  unsigned long long mask[kActiveTile / kBlock];
+#pragma unroll
+  for (int r = 0; r < kActiveTile / kBlock; r++) {
+    const int e = blockIdx.x * kActiveTile + r * kBlock + t;
+    mask[r] = __ballot(e < d.ne && (d.eact[e] & 1));
+    if (lane == 0) w[r][wv] = __popcll(mask[r]);
+  }
+  __syncthreads();
+  int base = block[blockIdx.x];
+#pragma unroll
+  for (int r = 0; r < kActiveTile / kBlock; r++) {
+    int before = 0, tot = 0;
+    for (int q = 0; q < kBlock / 64; q++) {
+      before += q < wv ? w[r][q] : 0;
+      tot += w[r][q];
+    }
+    const int e = blockIdx.x * kActiveTile + r * kBlock + t;
+    const int k = base + before + __popcll(mask[r] & ((1ull << lane) - 1ull));
+    base += tot;
+    if (!(mask[r] >> lane & 1ull) || k >= cap) continue;
+    rk_interaction o;
+    const uint32_t sub = d.esub[e];
+    const EState s = d.est[e];
+    const EGeom g = d.egeo[e];
+    o.i = d.ei[e];
+    o.j = d.ej[e];
+    o.type = (int32_t)(sub >> 30);
+    o.isub = (int32_t)((sub >> 15) & 0x7fffu);
+    o.jsub = (int32_t)(sub & 0x7fffu);
+    o.stick = d.estick[e];
+    o.n[0] = g.nx;
+    o.n[1] = g.ny;
+    o.n[2] = g.nz;
+    o.dn = d.edn[e];
+    o.pos[0] = g.px;
+    o.pos[1] = g.py;
+    o.pos[2] = g.pz;
+    o.vel[0] = g.vx;
+    o.vel[1] = g.vy;
+    o.vel[2] = g.vz;
+    o.fn = s.fn;
+    o.ft[0] = s.ftx;
+    o.ft[1] = s.fty;
+    o.ft[2] = s.ftz;
+    o.mom[0] = s.momx;
+    o.mom[1] = s.momy;
+    o.mom[2] = s.momz;
+    o.damp = d.edamp[e];
+    out[k] = o;
+  }
+}
+
 }  // namespace
 
 int body_block(const Dev& d) { return d.body_block == 64 || d.body_block == 128 ? d.body_block : 256; }
@@ -2469,6 +2578,24 @@ void launch_predict(const Dev& d, const StepParams& sp, int glob, int par, hipSt
   const int fused = listed && d.fuse_glob != 0;  // the free bodies' in k_predict
   hipLaunchKernelGGL(k_predict, grid_for(d, (n + bs - 1) / bs), dim3(bs), 0, s, d, sp, fused, par);
   launch_glob(d, listed ? 0 : 1, fused ? d.nvdriven : d.nvtot, s);
+}
+
+void launch_pack_bodies(const Dev& d, double* out, hipStream_t s) {
+  const long n = (13l * d.nb + kBlock - 1) / kBlock;
+  hipLaunchKernelGGL(k_pack_bodies, dim3((int)std::min(n, 65536L)), dim3(kBlock), 0, s, d, out);
+}
+
+int active_blocks(const Dev& d) { return (d.ne + kActiveTile - 1) / kActiveTile; }
+
+void launch_active_count(const Dev& d, int32_t* block, hipStream_t s) {
+  const int n = active_blocks(d);
+  if (n > 0) hipLaunchKernelGGL(k_active_count, dim3(n), dim3(kBlock), 0, s, d, block);
+  hipLaunchKernelGGL(k_active_scan, dim3(1), dim3(kBlock), 0, s, n, block);
+}
+
+void launch_active_records(const Dev& d, const int32_t* block, rk_interaction* out, int cap, hipStream_t s) {
+  const int n = active_blocks(d);
+  if (n > 0 && cap > 0) hipLaunchKernelGGL(k_active_records, dim3(n), dim3(kBlock), 0, s, d, block, out, cap);
 }
 
 void launch_drive(const Dev& d, const StepParams& sp, int glob, hipStream_t s) {
