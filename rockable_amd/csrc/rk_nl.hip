@@ -777,56 +777,117 @@ __device__ __forceinline__ double group_min(double x) {
   return x;
 }
 
-// Candidate pairs of two point shapes (one vertex, no edge or face: the
-// spheres), one pair per lane.  Their only test is vertex-vertex, so their
-// result is k_narrow's computed directly: the key (VV, 0, 0) when i's vertex
-// passes the reference's gate against j's OBB, j's vertex lies within sum of
-// i's box and VertexIsNearVertex holds.  A wavefront's near keys go to one
-// stripe (one atomic); rest[c] flags the other candidates for k_narrow.
-__global__ void __launch_bounds__(kBlock) k_narrow_points(Dev d, const double* bobb, const double* baabb,
-                                                          NarrowCfg cfg, int nc, const uint64_t* cand,
-                                                          uint32_t* nearbuf, int* near_cnt, int near_rcap,
-                                                          int32_t* cbase, int32_t* cnf, int32_t* cnb, int32_t* rest) {
+// Every near test of a pair is false when a plane separates the two
+// bodies' vertices by more than the tests reach: a vertex-vertex or edge-edge
+// test compares the distance of two points of the vertices' convex hulls with
+// sum; a vertex-edge test takes a foot on the edge's line up to dVerlet edge
+// lengths past its ends; a vertex-face test takes a foot in the face's outline
+// projected on a plane the face's vertices lie within reach[1] of.  The planes
+// tried are those normal to the line of centres, whose projection is
+// 1-Lipschitz, so a gap along it above sum + those allowances + margin
+// (rounding) leaves no test true.  A NaN coordinate turns the test off.
+__device__ __forceinline__ double apart_slack(const Dev& d, const BodyKin& Ki, const BodyKin& Kj, int shi, int shj,
+                                              double sum, double margin, double dmax) {
+  const double* ri = d.sh.reach + 2 * shi;
+  const double* rj = d.sh.reach + 2 * shj;
+  const double reach = dmax * fmax(Ki.h * ri[0], Kj.h * rj[0]) + fmax(Ki.h * ri[1], Kj.h * rj[1]);
+  return sum + reach + margin;
+}
+
+// The candidate pairs that need no wavefront of their own, one pair per lane.
+//  * Two point shapes (one vertex, no edge or face: the spheres).  Their only
+//    test is vertex-vertex, so their result is k_narrow's computed directly:
+//    the key (VV, 0, 0) when i's vertex passes the reference's gate against
+//    j's OBB, j's vertex lies within sum of i's box and VertexIsNearVertex
+//    holds.  A wavefront's near keys go to one stripe (one atomic).
+//  * Bodies apart (above): zero counts.  They are more than half of a settled
+//    packing's pairs; a wavefront each, which found it out after staging both
+//    bodies in LDS, cost a launch slot and idle lanes: k_narrow took 928 us
+//    for the 50 005-body pour's 434 000 pairs and 174 us for 13 001 bonded
+//    cubes, with this pass 59 + 845 us and 14 + 144 us.
+// The others go to list for k_narrow, their count in nrest (one atomic per
+// workgroup; their order changes no result).
+__global__ void __launch_bounds__(kBlock) k_narrow_lanes(Dev d, const double* bobb, const double* baabb, NarrowCfg cfg,
+                                                         int nc, const uint64_t* cand, uint32_t* nearbuf, int* near_cnt,
+                                                         int near_rcap, int32_t* cbase, int32_t* cnf, int32_t* cnb,
+                                                         int32_t* list, int* nrest) {
+  __shared__ int wcnt[kBlock / 64], at;
   const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  const int lane = threadIdx.x & 63;
-  bool point = false, near = false;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  bool point = false, near = false, rest = false;
   if (c < nc) {
     const uint64_t key = cand[c];
     const int i = (int)(key >> 32), j = (int)(key & 0xffffffffu);
-    const int shi = d.kin[i].shape, shj = d.kin[j].shape;
-    point = d.sh.nv[shi] == 1 && d.sh.ne[shi] == 0 && d.sh.nf[shi] == 0 && d.sh.nv[shj] == 1 && d.sh.ne[shj] == 0 &&
-            d.sh.nf[shj] == 0;
-    rest[c] = point ? 0 : 1;
+    const BodyKin &Ki = d.kin[i], &Kj = d.kin[j];
+    const int shi = Ki.shape, shj = Kj.shape;
+    const double Ri = Ki.R, Rj = Kj.R;
+    const int nvi = d.sh.nv[shi], nvj = d.sh.nv[shj];
+    const double* gvi = d.gv + 3 * (size_t)d.bvoff[i];
+    const double* gvj = d.gv + 3 * (size_t)d.bvoff[j];
+    const double *bxi = baabb + 6 * (size_t)i, *bxj = baabb + 6 * (size_t)j;
+    double xmax = 0.0;
+    for (int k = 0; k < 6; k++) xmax = fmax(fmax(xmax, fabs(bxi[k])), fabs(bxj[k]));
+    const double dmax = cfg.dmax;
+    const double sum = Ri + Rj + dmax;
+    const double margin = 1e-9 * (1.0 + xmax + sum);
+    point = nvi == 1 && d.sh.ne[shi] == 0 && d.sh.nf[shi] == 0 && nvj == 1 && d.sh.ne[shj] == 0 && d.sh.nf[shj] == 0;
     if (point) {
-      const double Ri = d.kin[i].R, Rj = d.kin[j].R;
-      const double *bxi = baabb + 6 * (size_t)i, *bxj = baabb + 6 * (size_t)j;
-      double xmax = 0.0;
-      for (int k = 0; k < 6; k++) xmax = fmax(fmax(xmax, fabs(bxi[k])), fabs(bxj[k]));
-      const double dmax = cfg.dmax;
-      const double sum = Ri + Rj + dmax;
-      const double margin = 1e-9 * (1.0 + xmax + sum);
-      const double* gvi = d.gv + 3 * (size_t)d.bvoff[i];
-      const double* gvj = d.gv + 3 * (size_t)d.bvoff[j];
       const double gvv = sum + margin;
       const v3 pj = lds_v(gvj, 0);
       const bool jnear = pj.x >= bxi[0] - gvv && pj.x <= bxi[3] + gvv && pj.y >= bxi[1] - gvv &&
                          pj.y <= bxi[4] + gvv && pj.z >= bxi[2] - gvv && pj.z <= bxi[5] + gvv;
       near = jnear && vertex_gate(lds_v(gvi, 0), Ri, load_obb(bobb + 15 * (size_t)j), dmax) &&
              near_vv(gvi, gvj, Ri, Rj, 0, 0, dmax);
+    } else {
+      v3 ax = V(Kj.px - Ki.px, Kj.py - Ki.py, Kj.pz - Ki.pz);
+      const double a2 = vdot(ax, ax);
+      bool apart = false;
+      if (a2 > 0.0) {
+        ax = vsc(1.0 / sqrt(a2), ax);
+        double hi_i = -INFINITY, lo_j = INFINITY;
+        for (int v = 0; v < nvi; v++) {
+          const double q = vdot(ax, lds_v(gvi, v));
+          hi_i = q == q ? fmax(hi_i, q) : INFINITY;
+        }
+        for (int v = 0; v < nvj; v++) {
+          const double q = vdot(ax, lds_v(gvj, v));
+          lo_j = q == q ? fmin(lo_j, q) : -INFINITY;
+        }
+        apart = lo_j - hi_i > apart_slack(d, Ki, Kj, shi, shj, sum, margin, dmax);
+      }
+      rest = !apart;
+      // (k_narrow rewrites the others'; the merge's count may run before it)
+      cbase[c] = 0;
+      cnf[c] = 0;
+      cnb[c] = 0;
     }
   }
-  const unsigned long long m = __ballot(near);
+  const unsigned long long m = __ballot(near), mr = __ballot(rest);
+  if (lane == 0) wcnt[wv] = __popcll(mr);
   const int stripe = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6) & (kStripes - 1);
   int base = 0;
   if (lane == 0 && m) base = atomicAdd(near_cnt + stripe * kStripeStride, __popcll(m));
   base = __shfl(base, 0, 64);
+  const unsigned long long below = (1ull << lane) - 1ull;
   if (point) {
-    const int local = base + __popcll(m & ((1ull << lane) - 1ull));
-    cbase[c] = stripe * near_rcap + local;
-    cnf[c] = near ? 1 : 0;
+    const int local = base + __popcll(m & below);
+    // over capacity: no key, and the host re-runs with a larger buffer
+    const bool room = local < near_rcap;
+    cbase[c] = room ? stripe * near_rcap + local : 0;
+    cnf[c] = near && room ? 1 : 0;
     cnb[c] = 0;
-    // over capacity: the host re-runs with a larger buffer
-    if (near && local < near_rcap) nearbuf[stripe * near_rcap + local] = pack_sub(VV, 0, 0);
+    if (near && room) nearbuf[stripe * near_rcap + local] = pack_sub(VV, 0, 0);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int n = wcnt[0] + wcnt[1] + wcnt[2] + wcnt[3];
+    at = n ? atomicAdd(nrest, n) : 0;
+  }
+  __syncthreads();
+  if (rest) {
+    int k = at + __popcll(mr & below);
+    for (int w = 0; w < wv; w++) k += wcnt[w];
+    list[k] = c;
   }
 }
 
@@ -837,22 +898,22 @@ __global__ void __launch_bounds__(kBlock) k_narrow_points(Dev d, const double* b
 // of the compiler: 6 wavefronts per SIMD with one pair (80 VGPRs, no
 // spill), 3 with two.
 template <int P>
-__global__ void __launch_bounds__(64, P == 1 ? 6 : 3) k_narrow(Dev d, const double* bobb, const double* baabb, NarrowCfg cfg, int nc,
+__global__ void __launch_bounds__(64, P == 1 ? 6 : 3) k_narrow(Dev d, const double* bobb, const double* baabb, NarrowCfg cfg,
                                                const uint64_t* cand, uint32_t* nearbuf, int* near_cnt,
                                                int near_rcap, int32_t* cbase, int32_t* cnf, int32_t* cnb,
-                                               int stride, const int32_t* clist) {
+                                               int stride, const int32_t* clist, const int* nrest, int first) {
   constexpr int SW = 64 / P;
   extern __shared__ double lds_all[];
   const int lane = threadIdx.x;
   // (with one pair per wavefront the pair's values stay wavefront-uniform,
   // in scalar registers)
   const int g = P == 1 ? 0 : lane / SW, sl = P == 1 ? lane : lane % SW;
-  // the idx-th pair to test: candidate clist[idx] (all candidates in order
-  // without a list)
-  const int idx = xcd_block((int)blockIdx.x, (int)gridDim.x) * P + g;
-  const bool valid = idx < nc;
-  if (P == 1 && !valid) return;
-  const int c = valid ? (clist ? clist[idx] : idx) : 0;
+  // the idx-th pair to test: candidate clist[idx], of *nrest (the grid is
+  // sized from the last rebuild's count, before this one's is known)
+  const int idx = first + xcd_block((int)blockIdx.x, (int)gridDim.x) * P + g;
+  const bool valid = idx < *nrest;
+  if (P == 1 ? !valid : !__any(valid)) return;
+  const int c = valid ? clist[idx] : 0;
   double* lds = lds_all + (size_t)g * (stride / 8);
   uint64_t key = 0;
   if (valid) key = cand[c];
@@ -908,22 +969,11 @@ __global__ void __launch_bounds__(64, P == 1 ? 6 : 3) k_narrow(Dev d, const doub
   const double sum = Ri + Rj + dmax;
   const double margin = 1e-9 * (1.0 + xmax + sum);
 
-  // Every near test of the pair is false when a plane separates the two
-  // bodies' vertices by more than the tests reach: a vertex-vertex or
-  // edge-edge test compares the distance of two points of the vertices'
-  // convex hulls with sum; a vertex-edge test takes a foot on the edge's line
-  // up to dVerlet edge lengths past its ends; a vertex-face test takes a
-  // foot in the face's outline projected on a plane the face's vertices lie
-  // within reach[1] of.  The planes tried are those normal to the line of
-  // centres, whose projection is 1-Lipschitz, so a gap along it above sum +
-  // those allowances + margin (rounding) leaves no test true.  Such pairs are
-  // most candidates in a settled packing; they get zero counts without a
-  // gate or test.  A NaN coordinate (or a zero axis) turns the test off.
-  // The same bound culls single elements of the other pairs: a test of an
-  // element of i needs its hull's projection to reach lo_j - slack (lim_i),
-  // one of j's to reach down to hi_i + slack (lim_j); the culls apply it to
-  // the vertices and to the edges' and faces' boxes, which hold them.
-  bool apart = false;
+  // Slab culls: the bound that sends pairs apart away (k_narrow_lanes) culls
+  // single elements of the others: a test of an element of i needs its hull's
+  // projection on the line of centres to reach lo_j - slack (lim_i), one of
+  // j's to reach down to hi_i + slack (lim_j); the culls apply it to the
+  // vertices and to the edges' and faces' boxes, which hold them.
   v3 ax = V(0.0, 0.0, 0.0);
   double lim_i = -INFINITY, lim_j = INFINITY;
   // bit v: vertex v within the limit (all set where not computed, shapes of
@@ -947,11 +997,7 @@ __global__ void __launch_bounds__(64, P == 1 ? 6 : 3) k_narrow(Dev d, const doub
       }
       hi_i = group_max<SW>(hi_i);
       lo_j = group_min<SW>(lo_j);
-      const double* ri = d.sh.reach + 2 * shi;
-      const double* rj = d.sh.reach + 2 * shj;
-      const double reach = dmax * fmax(Ki.h * ri[0], Kj.h * rj[0]) + fmax(Ki.h * ri[1], Kj.h * rj[1]);
-      const double slack = sum + reach + margin;
-      apart = lo_j - hi_i > slack;
+      const double slack = apart_slack(d, Ki, Kj, shi, shj, sum, margin, dmax);
       const double li = lo_j - slack, lj = hi_i + slack;
       if (li == li) lim_i = li;
       if (lj == lj) lim_j = lj;
@@ -969,17 +1015,6 @@ __global__ void __launch_bounds__(64, P == 1 ? 6 : 3) k_narrow(Dev d, const doub
       ax = V(0.0, 0.0, 0.0);
     }
   }
-  // (with several pairs per wavefront, when every pair of it is apart; the
-  // workgroup is this one wavefront)
-  if (P == 1 ? apart : __all(apart || !valid)) {
-    if (valid && sl == 0) {
-      cbase[c] = 0;
-      cnf[c] = 0;
-      cnb[c] = 0;
-    }
-    return;
-  }
-
   // edges and faces of both bodies in one pass, index q over i's edges, j's
   // edges, i's faces, j's faces (before the vertices, so that ax and the
   // limits are dead in the vertex gates' registers)
@@ -989,7 +1024,6 @@ __global__ void __launch_bounds__(64, P == 1 ? 6 : 3) k_narrow(Dev d, const doub
   const float* gfi = cfg.gface + kGate * (size_t)d.bfoff[i];
   const float* gfj = cfg.gface + kGate * (size_t)d.bfoff[j];
   const int nefg = group_compact<SW>(nef, sl, g, ef_l, [&](int q) {
-    if (apart) return false;
     if (q < nei) {
       const float* gb = gei + kGate * q;
       return gate_box_reach(gb, ax, true) >= lim_i && edge_gate_pre(gb, sum, dmax, margin, bxj, bxj + 3);
@@ -1008,7 +1042,6 @@ __global__ void __launch_bounds__(64, P == 1 ? 6 : 3) k_narrow(Dev d, const doub
   // reference vertex gates of both bodies in one pass: i's vertices against
   // j's OBB, j's against i's
   const int nvg = group_compact<SW>(nvi + nvj, sl, g, vg_l, [&](int v) {
-    if (apart) return false;
     if (v < nvi) return (v >= 64 || ((keep_i >> v) & 1ull)) && vertex_gate(lds_v(gvi, v), Ri, load_obb(obj), dmax);
     const int u = v - nvi;
     return (u >= 64 || ((keep_j >> u) & 1ull)) && vertex_gate(lds_v(gvj, u), Rj, load_obb(obi), dmax);
@@ -1122,13 +1155,13 @@ __global__ void __launch_bounds__(64, P == 1 ? 6 : 3) k_narrow(Dev d, const doub
   if (valid && sl == 0) local = atomicAdd(near_cnt + stripe * kStripeStride, cf + cb);
   local = __shfl(local, 0, SW);
   const int base_out = stripe * near_rcap + local;
-  if (valid && sl == 0) {
-    cbase[c] = base_out;
-    cnf[c] = cf;
-    cnb[c] = cb;
-  }
-  // over capacity: the host re-runs with a larger buffer
+  // over capacity: no keys, and the host re-runs with a larger buffer
   const bool room = valid && local + cf + cb <= near_rcap;
+  if (valid && sl == 0) {
+    cbase[c] = room ? base_out : 0;
+    cnf[c] = room ? cf : 0;
+    cnb[c] = room ? cb : 0;
+  }
   // write the keys in test order (output slot = rank of the set bit), one
   // key per lane: the exclusive prefix of the words' bit counts in LDS, then
   // key q's word by a binary search over it and its bit as the
@@ -1780,7 +1813,8 @@ int nl_rebuild(NLWork& w, Dev& d, const NLParams& p, EntryArrays& cur, EntryArra
       ensure(w, w.cnb, w.cnb_cap, (size_t)std::max(nc, 1)))
     return -1;
   std::function<int(int)> launch_narrow;
-  int narrow_rcap = 0;
+  std::function<void(int, int, int)> launch_rest;
+  int narrow_rcap = 0, narrow_done = 0;  // pairs the narrow phase's grid has covered
   if (nc > 0) {
     NarrowCfg cfg;
     cfg.maxv = p.maxv;
@@ -1809,34 +1843,27 @@ int nl_rebuild(NLWork& w, Dev& d, const NLParams& p, EntryArrays& cur, EntryArra
     const size_t lds = (size_t)P * stride;
     // one run of the narrow phase into stripes of rcap keys; the stripe
     // totals (all, largest) land in counter[2..3]
-    launch_narrow = [&, cfg, P, stride, lds](int rcap) -> int {
+    // (the stripes' counters use the first word of every 32; the pairs left go to word 1)
+    launch_rest = [&, cfg, P, stride, lds](int rcap, int first, int count) {
+      const dim3 grid((count + P - 1) / P);
+      if (P == 2)
+        hipLaunchKernelGGL(k_narrow<2>, grid, dim3(64), lds, s, d, w.bobb, w.baabb, cfg, w.cand, w.nearbuf, w.scnt, rcap,
+                           w.cbase, w.cnf, w.cnb, (int)stride, w.plist, w.scnt + 1, first);
+      else
+        hipLaunchKernelGGL(k_narrow<1>, grid, dim3(64), lds, s, d, w.bobb, w.baabb, cfg, w.cand, w.nearbuf, w.scnt, rcap,
+                           w.cbase, w.cnf, w.cnb, (int)stride, w.plist, w.scnt + 1, first);
+    };
+    launch_narrow = [&, cfg](int rcap) -> int {
       if (ensure(w, w.nearbuf, w.nearbuf_cap, (size_t)kStripes * rcap)) return -1;
       RK_CHECK(hipMemsetAsync(w.scnt, 0, sizeof(int) * kStripes * kStripeStride, s));
-      // pairs of point shapes one per lane; the others (all of them without
-      // point shapes) one or two per wavefront
-      int nrest = nc;
-      const int32_t* clist = nullptr;
-      if (p.has_points) {
-        if (ensure(w, w.pflag, w.pflag_cap, (size_t)nc) || ensure(w, w.ppos, w.ppos_cap, (size_t)nc) ||
-            ensure(w, w.plist, w.plist_cap, (size_t)nc))
-          return -1;
-        hipLaunchKernelGGL(k_narrow_points, dim3(nblk(nc)), dim3(kBlock), 0, s, d, w.bobb, w.baabb, cfg, nc, w.cand,
-                           w.nearbuf, w.scnt, rcap, w.cbase, w.cnf, w.cnb, w.pflag);
-        if (scan_exclusive(w, w.pflag, w.ppos, nc, s)) return -1;
-        hipLaunchKernelGGL(k_heavy_list, dim3(nblk(nc)), dim3(kBlock), 0, s, nc, w.pflag, w.ppos, w.plist);
-        int last[2] = {0, 0};
-        if (read_small(w, s, {{&last[0], {w.ppos + nc - 1, sizeof(int)}}, {&last[1], {w.pflag + nc - 1, sizeof(int)}}}))
-          return -1;
-        nrest = last[0] + last[1];
-        clist = w.plist;
-      }
-      const dim3 grid((nrest + P - 1) / P);
-      if (nrest > 0 && P == 2)
-        hipLaunchKernelGGL(k_narrow<2>, grid, dim3(64), lds, s, d, w.bobb, w.baabb, cfg, nrest, w.cand, w.nearbuf,
-                           w.scnt, rcap, w.cbase, w.cnf, w.cnb, (int)stride, clist);
-      else if (nrest > 0)
-        hipLaunchKernelGGL(k_narrow<1>, grid, dim3(64), lds, s, d, w.bobb, w.baabb, cfg, nrest, w.cand, w.nearbuf,
-                           w.scnt, rcap, w.cbase, w.cnf, w.cnb, (int)stride, clist);
+      // the pairs of point shapes and those apart one per lane, the others one
+      // or two per wavefront; their count is not known yet, so the grid takes
+      // the last rebuild's and the rest follows if it was short (below)
+      if (ensure(w, w.plist, w.plist_cap, (size_t)nc)) return -1;
+      hipLaunchKernelGGL(k_narrow_lanes, dim3(nblk(nc)), dim3(kBlock), 0, s, d, w.bobb, w.baabb, cfg, nc, w.cand,
+                         w.nearbuf, w.scnt, rcap, w.cbase, w.cnf, w.cnb, w.plist, w.scnt + 1);
+      narrow_done = w.rest_hint >= 0 ? std::min(nc, w.rest_hint + w.rest_hint / 8 + 256) : nc;
+      launch_rest(rcap, 0, narrow_done);
       RK_CHECK(hipGetLastError());
       hipLaunchKernelGGL(k_stripe_scan, dim3(1), dim3(kStripes), 0, s, w.scnt, w.soff, w.counter + 2);
       return 0;
@@ -1931,8 +1958,20 @@ int nl_rebuild(NLWork& w, Dev& d, const NLParams& p, EntryArrays& cur, EntryArra
       return 0;
     };
     if (count_pass()) return -1;
-    int rd[4] = {0, 0, 0, 0};
-    if (read_small(w, s, {{rd, {w.counter, 4 * sizeof(int)}}})) return -1;
+    int rd[4] = {0, 0, 0, 0}, nrest = 0;
+    if (launch_narrow) {
+      if (read_small(w, s, {{rd, {w.counter, 4 * sizeof(int)}}, {&nrest, {w.scnt + 1, sizeof(int)}}})) return -1;
+    } else {
+      if (read_small(w, s, {{rd, {w.counter, 2 * sizeof(int)}}})) return -1;
+    }
+    bool again = false;
+    if (launch_narrow && nrest > narrow_done) {  // more pairs than the grid covered
+      launch_rest(narrow_rcap, narrow_done, nrest - narrow_done);
+      hipLaunchKernelGGL(k_stripe_scan, dim3(1), dim3(kStripes), 0, s, w.scnt, w.soff, w.counter + 2);
+      if (read_small(w, s, {{rd + 2, {w.counter + 2, 2 * sizeof(int)}}})) return -1;
+      again = true;
+    }
+    if (launch_narrow) w.rest_hint = nrest;
     if (launch_narrow && rd[3] > narrow_rcap) {
       for (int attempt = 0;; attempt++) {
         if (attempt == 2) {
@@ -1946,6 +1985,9 @@ int nl_rebuild(NLWork& w, Dev& d, const NLParams& p, EntryArrays& cur, EntryArra
         if (rd[3] <= narrow_rcap) break;
       }
       in.nearbuf = w.nearbuf;
+      again = true;
+    }
+    if (again) {
       if (count_pass()) return -1;
       if (read_small(w, s, {{rd, {w.counter, 2 * sizeof(int)}}})) return -1;
     }
@@ -2028,7 +2070,7 @@ void entries_free(EntryArrays& E) {
 }
 
 void nl_work_free(NLWork& w) {
-  void* ps[] = {w.pflag, w.ppos, w.plist,
+  void* ps[] = {w.plist,
                 w.cstripe, w.scnt, w.soff, w.bobb,  w.baabb, w.counter, w.cand,  w.cbase, w.cnf,   w.cnb,   w.nearbuf, w.okey,  w.ostart,
                 w.gk,    w.gk2,   w.gv,      w.gv2,   w.gflag, w.gpos,  w.ukey,  w.ucand,   w.uold,  w.gcount,
                 w.goff,  w.tmp,   w.i32a,    w.i32b,  w.i32c,  w.f64a,  w.cell_of, w.ccount, w.cstart, w.cfill,

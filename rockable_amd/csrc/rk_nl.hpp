@@ -65,7 +65,6 @@ struct NLParams {
   int maxe = 0;      // max edges per shape
   int maxf = 0;      // max faces per shape
   int maxwords = 1;  // max 64-bit words of predicate bits per body pair
-  int has_points = 0;  // some shape is a point (one vertex, no edge or face)
 };
 
 // LDS of one narrow-phase pair: both bodies' OBBs and boxes, the global
@@ -82,6 +81,7 @@ struct NLWork {
   // partials): a pageable destination makes the runtime stage each copy
   char* pin = nullptr;
   int cand_hint = 0, near_hint = 0, last_candidates = 0;
+  int rest_hint = -1;  // pairs left to the narrow phase's wavefronts in the last rebuild (-1: none yet)
   int heavy_min = 256;  // slot count above which a body's sum runs block-wide
   int narrow_pairs = 0;  // candidate pairs per narrow-phase wavefront (1, 2; 0: by shape size)
 #define RK_BUF(T, name) \
@@ -89,9 +89,7 @@ struct NLWork {
   size_t name##_cap = 0;
   RK_BUF(double, bobb)
   RK_BUF(double, baabb)
-  RK_BUF(int32_t, pflag)  // narrow phase: candidates that are not point pairs, their prefix, their list
-  RK_BUF(int32_t, ppos)
-  RK_BUF(int32_t, plist)
+  RK_BUF(int32_t, plist)  // narrow phase: the candidates left to the wavefronts (their count in scnt[1])
   RK_BUF(float, gedge)
   RK_BUF(float, gface)
   RK_BUF(int32_t, kout)
