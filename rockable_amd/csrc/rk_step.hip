@@ -1404,11 +1404,11 @@ __device__ __forceinline__ unsigned byte_bits(unsigned x) { return ((x & 0x01010
 // order, with initialise_particle_forces_and_moments, the accelerations and
 // the closing kick.  A workgroup takes NB free bodies, whose slots are
 // consecutive, or one driven body:
-//   1. the 256 threads read all the slots' activity bytes (16 each, up to
-//      4 096 slots at a time) and rank the active ones into an LDS list;
-//   2. they read the active slots' terms (48 bytes each), 512 slots at a
+//   1. the T threads read all the slots' activity bytes (16 each, up to
+//      16 T slots at a time) and rank the active ones into an LDS list;
+//   2. they read the active slots' terms (48 bytes each), 2 T slots at a
 //      time, into LDS;
-//   3. lanes of each body, one per component of (F, M), add its terms in
+//   3. lanes of each body, one to three components of (F, M) each, add its terms in
 //      slot order, so every component is the reference's bit for bit;
 //   4. one thread per body finishes it.  The records (128 bytes) are read at
 //      the start and written back whole, in contiguous doubles, through LDS.
@@ -1418,8 +1418,8 @@ __device__ __forceinline__ unsigned byte_bits(unsigned x) { return ((x & 0x01010
 // so a wall with 200 slots or a bonded cube with 18 active ones waited for
 // many loads in turn, and 4 of a wavefront's lanes finished its bodies:
 // 15.7 us for 706 bodies, 22.6 us for 50 005, 40.3 us for 90 006 with the
-// displacement check, 13.7 us for 13 001 bonded cubes; now 6.6, 14.8, 23.4 and
-// 10.3 us.
+// displacement check, 13.7 us for 13 001 bonded cubes; at first 6.6, 14.8, 23.4
+// and 10.3 us, before the predictor joined (below).
 // With fuse the step after this one follows at once, and the free bodies take
 // its predictor (and their listed vertices) here, while their records and
 // accelerations are at hand: one launch and one pass over the records less,
@@ -1435,8 +1435,6 @@ __device__ __forceinline__ unsigned byte_bits(unsigned x) { return ((x & 0x01010
 // workgroup stores its maxima in gpart[2 blockIdx.x].  One tile per workgroup
 // whatever the persistent option: in a loop over tiles the compiler keeps the
 // loop's invariants in 196 registers (102 without).
-constexpr int kGatherCap = 512;   // slots' terms in LDS
-constexpr int kGatherWin = 4096;  // slots scanned at a time: 16 per thread
 
 // The sum of one component (lanes gl < 6) over the slots [k0, k1) of one
 // chunk of at most 64 slots by one wavefront, from -0.0, in slot order
@@ -1464,25 +1462,37 @@ __device__ __forceinline__ double sum_chunk(const Dev& d, int k0, int k1, int la
   return s;
 }
 
-template <int NB, bool BF>  // BF: the deck has a body force
-__global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, GatherArgs A) {
-  constexpr int kLanes = kBlock / NB;      // lanes per body in the sums (8 or 4)
-  constexpr int kComp = kLanes >= 6 ? 1 : 2;  // components per lane
+template <int T, int NB, bool BF>  // T threads; BF: the deck has a body force
+__global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArgs A) {
+  constexpr int kLanes = T / NB;  // lanes per body in the sums (8, 4 or 2)
+  constexpr int kComp = kLanes >= 6 ? 1 : kLanes >= 3 ? 2 : 3;  // components per lane
+  constexpr int kCap = 2 * T;   // slots' terms in LDS
+  constexpr int kWin = 16 * T;  // slots scanned at a time
   __shared__ double rec[NB * kRec];
-  __shared__ __align__(16) double vals[kGatherCap * 6];
-  __shared__ unsigned short list[kGatherWin];
-  __shared__ int pre[kBlock + 1];
-  __shared__ unsigned short act[kBlock];
-  __shared__ int wsum[kBlock / 64];
+  __shared__ __align__(16) double vals[kCap * 6];
+  __shared__ unsigned short list[kWin];
+  __shared__ int pre[T + 1];
+  __shared__ unsigned short act[T];
+  __shared__ int wsum[T / 64];
   __shared__ double fm[NB][6];
-  if (frozen(d)) return;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int kick = A.kick, guard = A.guard;
-  const bool rst = guard && guard_reset(d);
+  // every control word in one round of loads
+  int stop = 0, due = 0, again = 0;
+  if (d.guard_on) {
+    const volatile DevGuard* G = d.guard;
+    const int fr = G->frozen, nu = G->nu, re = G->reset, fl = *(volatile const int*)d.flags;
+    stop = fr;
+    due = nu | fl;
+    again = re;
+  }
+  const int want = *(volatile const int*)&d.ls->want[A.par];
+  if (stop) return;
+  const bool rst = guard && again;
   // (the check that follows this step freezes the later ones on the same words)
-  const bool predict = A.fuse && !rebuild_due(d);
+  const bool predict = A.fuse && !due;
   // this step's force phase wrote a new evaluation list
-  const bool relisted = A.listed && *(volatile const int*)&d.ls->want[A.par] != 0;
+  const bool relisted = A.listed && want != 0;
   if (relisted && blockIdx.x == 0 && t == 0) {
     const int g = d.ls->gen + 1;
     for (int k = 0; k < 8; k++) d.ls->cnt[(g + 1) & 1][k] = 0;
@@ -1497,14 +1507,14 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, Gath
   ga.kp = 0ull;
   ga.kw = ~0ull;
   // (gather_blocks sizes the grid by the same rule)
-  const int nchunk = A.fuse && !d.guard_on ? 0 : (d.nhch + kBlock / 64 - 1) / (kBlock / 64);
+  const int nchunk = A.fuse && !d.guard_on ? 0 : (d.nhch + T / 64 - 1) / (T / 64);
   const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
   const bool driven = tile < d.nDriven, chunks = !driven && tile < d.nDriven + nchunk;
   const int b0 = driven ? tile : d.nDriven + (tile - d.nDriven - nchunk) * NB;
   const int nbk = driven ? 1 : min(NB, d.nb - b0);
   int k0 = 0, kend = 0;
   if (chunks) {
-    const int c = (tile - d.nDriven) * (kBlock / 64) + wv;
+    const int c = (tile - d.nDriven) * (T / 64) + wv;
     if (c < d.nhch && !predict) {
       const int2 r = d.hch[c];
       const double s = sum_chunk(d, r.x, r.y, lane, vals + 64 * 6 * wv);
@@ -1524,7 +1534,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, Gath
   }
   // the records, and what finishing a body needs, ahead of the sums
   d2* kd = reinterpret_cast<d2*>(d.kin + b0);
-  for (int k = t; k < 8 * nbk; k += kBlock) {
+  for (int k = t; k < 8 * nbk; k += T) {
     const d2 x = kd[k];
     double* r = rec + (k >> 3) * kRec + 2 * (k & 7);
     r[0] = x.x;
@@ -1563,7 +1573,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, Gath
   }
   double s[kComp];
   bool first = true;
-  for (int w0 = k0 & ~15; w0 < kend; w0 += kGatherWin) {
+  for (int w0 = k0 & ~15; w0 < kend; w0 += kWin) {
     const int pos = w0 + 16 * t;
     unsigned m = 0u;
     if (pos < kend) {
@@ -1583,20 +1593,20 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, Gath
     __syncthreads();
     int base = 0, total = 0;
 #pragma unroll
-    for (int w = 0; w < kBlock / 64; w++) {
+    for (int w = 0; w < T / 64; w++) {
       base += w < wv ? wsum[w] : 0;
       total += wsum[w];
     }
     int r = base + incl - mine;
     pre[t] = r;
     act[t] = (unsigned short)m;
-    if (t == 0) pre[kBlock] = total;
+    if (t == 0) pre[T] = total;
     for (unsigned rest = m; rest; rest &= rest - 1u) list[r++] = (unsigned short)(16 * t + __ffs((int)rest) - 1);
     __syncthreads();
     // ranks of a body's slots within the window's list
     auto rank = [&](int k) -> int {
-      const int q = min(max(k - w0, 0), kGatherWin);
-      if (q == kGatherWin) return pre[kBlock];
+      const int q = min(max(k - w0, 0), kWin);
+      if (q == kWin) return pre[T];
       return pre[q >> 4] + __popc((unsigned)act[q >> 4] & ((1u << (q & 15)) - 1u));
     };
     int lo = 0, hi = 0;
@@ -1608,21 +1618,21 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, Gath
       hi = rank(sb1);
     }
     first = false;
-    for (int p0 = 0; p0 < total; p0 += kGatherCap) {
-      const int n = min(kGatherCap, total - p0);
+    for (int p0 = 0; p0 < total; p0 += kCap) {
+      const int n = min(kCap, total - p0);
       d2 v[2][3];
 #pragma unroll
       for (int h = 0; h < 2; h++)
-        if (t + h * kBlock < n) {
+        if (t + h * T < n) {
           const d2* x =
-              reinterpret_cast<const d2*>(d.sval + 6 * (size_t)(w0 + (int)list[p0 + t + h * kBlock]));
+              reinterpret_cast<const d2*>(d.sval + 6 * (size_t)(w0 + (int)list[p0 + t + h * T]));
 #pragma unroll
           for (int q = 0; q < 3; q++) v[h][q] = x[q];
         }
 #pragma unroll
       for (int h = 0; h < 2; h++)
-        if (t + h * kBlock < n) {
-          d2* x = reinterpret_cast<d2*>(vals + 6 * (t + h * kBlock));
+        if (t + h * T < n) {
+          d2* x = reinterpret_cast<d2*>(vals + 6 * (t + h * T));
 #pragma unroll
           for (int q = 0; q < 3; q++) x[q] = v[h][q];
         }
@@ -1659,12 +1669,12 @@ __global__ void __launch_bounds__(kBlock, 4) k_gather(Dev d, StepParams sp, Gath
   }
   __syncthreads();
   if (kick)
-    for (int k = t; k < 8 * nbk; k += kBlock) {
+    for (int k = t; k < 8 * nbk; k += T) {
       const double* r = rec + (k >> 3) * kRec + 2 * (k & 7);
       kd[k] = d2{r[0], r[1]};
     }
   if (predict && !driven && A.glob != GLOB_NONE)
-    for (int k = d.bvoff[b0] + t; k < d.bvoff[b0 + nbk]; k += kBlock) {
+    for (int k = d.bvoff[b0] + t; k < d.bvoff[b0 + nbk]; k += T) {
       const int bb = d.bvbody[k];
       if (d.soff[bb + 1] == d.soff[bb]) continue;
       const BodyKin P = rec_load(rec + (bb - b0) * kRec);
@@ -2696,29 +2706,46 @@ void launch_interact(const Dev& d, const StepParams& sp, int write_geom_all, int
 constexpr int kGatherLarge = 1 << 17;
 int gather_bodies(const Dev& d) { return d.nb - d.nDriven >= kGatherLarge ? 64 : 32; }
 
-// k_gather's workgroups: one per driven body, the heavy chunks four to one,
-// the free bodies
-int gather_blocks(const Dev& d, int fuse) {
-  const int nb = gather_bodies(d);
-  return d.nDriven + (fuse && !d.guard_on ? 0 : (d.nhch + 3) / 4) + (d.nb - d.nDriven + nb - 1) / nb;
+// and its threads: 256 where all workgroups are resident at once anyway (up to
+// 1024 of them) or bodies have many slots, whose terms then take fewer passes;
+// 128 where workgroups queue, since only one wavefront finishes the bodies and
+// the others' places are worth more to a second workgroup.  256 against 128:
+// 12.9 and 16.2 us for 13 001 bonded cubes (65 slots each), 9.7 and 10.5 us
+// for 706 hulls, but 28.7 and 22.7 us for the 90 006-body slope, 12.3 and 9.2
+// us for 47 000 spheres.
+int gather_threads(const Dev& d) {
+  if (gather_bodies(d) == 64) return 128;
+  const bool few = (d.nb - d.nDriven + 31) / 32 <= 1024, many_slots = 2.0 * d.ne > 56.0 * d.nb;
+  return few || many_slots ? 256 : 128;
 }
 
-int gather_blocks_max(int nb, int nhch) { return nb + (nhch + 3) / 4 + 8; }
+// k_gather's workgroups: one per driven body, the heavy chunks one to a
+// wavefront, the free bodies
+int gather_blocks(const Dev& d, int fuse) {
+  const int nb = gather_bodies(d), wv = gather_threads(d) / 64;
+  return d.nDriven + (fuse && !d.guard_on ? 0 : (d.nhch + wv - 1) / wv) + (d.nb - d.nDriven + nb - 1) / nb;
+}
+
+int gather_blocks_max(int nb, int nhch) { return nb + (nhch + 1) / 2 + 8; }
 
 void launch_gather(const Dev& d, const StepParams& sp, GatherArgs A, hipStream_t s) {
   if (d.nb <= 0) return;
   A.guard = A.guard && A.kick;
   const int kick = A.kick, guard = A.guard;
   const dim3 blocks(gather_blocks(d, A.fuse));
-  const bool bf = d.bf != BF_NONE, large = gather_bodies(d) == 64;
+  const bool bf = d.bf != BF_NONE, large = gather_bodies(d) == 64, wide = gather_threads(d) == 256;
   if (large && bf)
-    hipLaunchKernelGGL((k_gather<64, true>), blocks, dim3(kBlock), 0, s, d, sp, A);
+    hipLaunchKernelGGL((k_gather<128, 64, true>), blocks, dim3(128), 0, s, d, sp, A);
   else if (large)
-    hipLaunchKernelGGL((k_gather<64, false>), blocks, dim3(kBlock), 0, s, d, sp, A);
+    hipLaunchKernelGGL((k_gather<128, 64, false>), blocks, dim3(128), 0, s, d, sp, A);
+  else if (wide && bf)
+    hipLaunchKernelGGL((k_gather<256, 32, true>), blocks, dim3(256), 0, s, d, sp, A);
+  else if (wide)
+    hipLaunchKernelGGL((k_gather<256, 32, false>), blocks, dim3(256), 0, s, d, sp, A);
   else if (bf)
-    hipLaunchKernelGGL((k_gather<32, true>), blocks, dim3(kBlock), 0, s, d, sp, A);
+    hipLaunchKernelGGL((k_gather<128, 32, true>), blocks, dim3(128), 0, s, d, sp, A);
   else
-    hipLaunchKernelGGL((k_gather<32, false>), blocks, dim3(kBlock), 0, s, d, sp, A);
+    hipLaunchKernelGGL((k_gather<128, 32, false>), blocks, dim3(128), 0, s, d, sp, A);
   if (d.nheavy > 0 && !A.fuse) {
     hipLaunchKernelGGL(k_heavy_finish, grid_for(d, d.nheavy), dim3(kBlock), 0, s, d, sp, kick, guard);
     if (d.nheavy_exact > 0)
