@@ -19,7 +19,7 @@
 //            active at the last force phase, bit 1 history maybe non-zero)
 //            spos[2n]     the entry's two resultant slots (i side, j side)
 //   CSR      istart[N+1]  entries owned by body b are [istart[b], istart[b+1])
-//            jstart[N+1], jlist[]  entries whose j == b, ascending index
+//            jstart[N+1]  the counts of the entries whose j == b, summed
 //   slots    body b's incident entries in the serial order of the reference's
 //            resultant loop (entries with j == b below b's own range, b's own
 //            range, entries with j == b above it) are the slots
@@ -250,8 +250,6 @@ struct Dev {
   // with zero history, [2] entries looked at, summed over the steps
   unsigned long long* skip_count;
   const int32_t* istart;
-  const int32_t* jstart;
-  const int32_t* jlist;
   // resultant slots
   const int32_t* spos;
   const int32_t* soff;

@@ -477,8 +477,6 @@ void assemble_dev(rk_engine* eng) {
   }
   d.persist = eng->persist;
   d.istart = E.istart;
-  d.jstart = E.jstart;
-  d.jlist = E.jlist;
   d.nctrl = (int)m.ctrl.size();
   d.ctrl = eng->ctrl;
   d.ctrl_off = eng->ctrl_off;

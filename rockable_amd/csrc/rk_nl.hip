@@ -28,7 +28,6 @@
 //   CSR              istart by owner; jlist = entries sorted (stably) by j
 #include <hip/hip_runtime.h>
 
-#include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 
 #include <algorithm>
@@ -447,54 +446,218 @@ __global__ void k_old_heads(int n, const int32_t* ei, const int32_t* ej, int32_t
 __global__ void k_old_compact(int n, const int32_t* ei, const int32_t* ej, const int32_t* flag, const int32_t* pos,
                               uint64_t* okey, int32_t* ostart) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e == n - 1) ostart[pos[e] + flag[e]] = n;
   if (e >= n || !flag[e]) return;
   okey[pos[e]] = ((uint64_t)(uint32_t)ei[e] << 32) | (uint32_t)ej[e];
   ostart[pos[e]] = e;
 }
-// combined key list: candidates in both directions, then old groups
-constexpr uint32_t kOldTag = 0x80000000u;
-// The group keys (owner, other) packed as owner << bb | other, bb the bits
-// of a body index, so that the radix sort runs over 2 bb bits instead of 64
-// (the order is the same: owner first, then other).
-__device__ __forceinline__ uint64_t pack_pair(uint32_t i, uint32_t j, int bb) { return ((uint64_t)i << bb) | j; }
-__global__ void k_fill_groups(int nc, const uint64_t* cand, int ng_old, const uint64_t* okey, uint64_t* gk,
-                              uint32_t* gv, int bb) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < nc) {
-    const uint64_t k = cand[t];
-    const uint32_t i = (uint32_t)(k >> 32), j = (uint32_t)(k & 0xffffffffu);
-    gk[2 * t] = pack_pair(i, j, bb);
-    gv[2 * t] = (uint32_t)t << 1;
-    gk[2 * t + 1] = pack_pair(j, i, bb);
-    gv[2 * t + 1] = ((uint32_t)t << 1) | 1u;
-  } else if (t < nc + ng_old) {
-    const int g = t - nc;
-    const uint64_t k = okey[g];
-    gk[2 * nc + g] = pack_pair((uint32_t)(k >> 32), (uint32_t)(k & 0xffffffffu), bb);
-    gv[2 * nc + g] = kOldTag | (uint32_t)g;
+
+// Placing by counts.  The directed groups ordered by (owner, other) and every
+// body's entries as second body ordered by index are both segments of small
+// integers that are all different, some tens of them for most bodies, and
+// thousands for a wall.  A device-wide radix or merge sort runs its full
+// sequence of passes for them and is launch bound below a million keys
+// (15 007 spheres: 205 us of a rebuild in the two sorts).  Here a count per
+// body, one scan and a fill in any order give the segments, and a member's
+// place is the number of smaller members: a loop over the segment, contiguous
+// and shared by the neighbouring lanes, up to kSegMax members; above that the
+// loop's square would tell, and workgroups mark the members of a window of
+// values in an LDS bitmap and count bits.
+constexpr int kSegMax = 512;
+constexpr int kWinBits = 18;  // values per bitmap window: 32 KB of bits, 16 KB of prefixes
+constexpr int kWinWords = 1 << (kWinBits - 6);
+constexpr int kWinThreads = 512;
+constexpr int kBigGrid = 64;  // workgroups across the list of long segments
+
+// One atomic per run of equal keys in neighbouring lanes (all lanes of the
+// wavefront call it): a wall's members come in runs and would queue on its
+// counter one by one.  `weight` counts a member in the low 32 bits,
+// and may count it in the high ones too (`kind` tells
+// the weights apart: a run has one); returns the member's position
+// among its key's, runs in lane order.  The counting pass keeps the positions,
+// so that the fill needs no atomics (337 000 entries: 27 us with its own,
+// under 13 without).  What bounds the count is the queue on the walls'
+// counters, one atomic per body that touches the wall (38 us).
+template <class T>
+__device__ __forceinline__ int run_add(T* count, int key, bool valid, T weight, int kind = 0) {
+  const int lane = (int)(threadIdx.x & 63);
+  const int k = valid ? key : -1;
+  const int prev = __shfl_up(k, 1, 64), pkind = __shfl_up(kind, 1, 64);
+  const unsigned long long heads = __ballot(lane == 0 || prev != k || pkind != kind);
+  const unsigned long long upto = heads & (~0ull >> (63 - lane));
+  const int head = 63 - __clzll((long long)upto);
+  const unsigned long long above = lane == 63 ? 0ull : heads >> (lane + 1) << (lane + 1);
+  int base = 0;
+  if (lane == head && valid) base = (int)atomicAdd(count + key, weight * (T)((above ? __ffsll(above) - 1 : 64) - lane));
+  return __shfl(base, head, 64) + lane - head;
+}
+
+// The members of [s0, s1) whose values lie in window `win`, as bits with
+// exclusive prefixes; returns the number of members below the window.  All
+// threads of the workgroup call it; it starts and ends with a barrier.
+struct WinLds {
+  unsigned long long bits[kWinWords];
+  int32_t pre[kWinWords];
+  int32_t wsum[kWinThreads / 64];
+  int32_t below;
+};
+__device__ int win_mark(WinLds& L, const int32_t* val, int s0, int s1, int win) {
+  const int t = (int)threadIdx.x, lane = t & 63;
+  __syncthreads();
+  for (int q = t; q < kWinWords; q += kWinThreads) L.bits[q] = 0ull;
+  if (t == 0) L.below = 0;
+  __syncthreads();
+  int under = 0;
+  for (int q = s0 + t; q < s1; q += kWinThreads) {
+    const int v = val[q];
+    const int vw = v >> kWinBits;
+    if (vw < win)
+      under++;
+    else if (vw == win)
+      atomicOr(&L.bits[(v & ((1 << kWinBits) - 1)) >> 6], 1ull << (v & 63));
   }
+  if (under) atomicAdd(&L.below, under);
+  __syncthreads();
+  constexpr int per = kWinWords / kWinThreads;
+  int sum = 0;
+  for (int q = 0; q < per; q++) sum += __popcll(L.bits[t * per + q]);
+  int inc = sum;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int x = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += x;
+  }
+  if (lane == 63) L.wsum[t >> 6] = inc;
+  __syncthreads();
+  int run = inc - sum;
+  for (int q = 0; q < (t >> 6); q++) run += L.wsum[q];
+  for (int q = 0; q < per; q++) {
+    L.pre[t * per + q] = run;
+    run += __popcll(L.bits[t * per + q]);
+  }
+  __syncthreads();
+  return L.below;
 }
-__global__ void k_group_heads(int n, const uint64_t* gk, int32_t* flag) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  flag[t] = (t == 0 || gk[t] != gk[t - 1]) ? 1 : 0;
+// members of the window below value v of the window
+__device__ __forceinline__ int win_rank(const WinLds& L, int v) {
+  const int x = v & ((1 << kWinBits) - 1);
+  return L.pre[x >> 6] + __popcll(L.bits[x >> 6] & ((1ull << (x & 63)) - 1ull));
 }
-__global__ void k_group_compact(int n, const uint64_t* gk, const uint32_t* gv, const int32_t* flag,
-                                const int32_t* pos, uint64_t* ukey, int32_t* ucand, int32_t* uold, int bb) {
+
+// The directed groups: both directions of every candidate and the groups of
+// the current list.  Owner b's part of the group arrays has a slot per member,
+// the slot of a group being the number of candidates plus the number of old
+// groups below it: a pair that is both takes one slot, the same from either
+// side, and leaves the next one empty (no candidate, no old group).
+__global__ void k_group_count(int nc, const uint64_t* cand, int32_t* cnt, int2* at) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n || !flag[t]) return;
-  const int u = pos[t];
-  // back to (owner << 32) | other
-  ukey[u] = ((gk[t] >> bb) << 32) | (gk[t] & ((1ull << bb) - 1ull));
-  int32_t c = -1, o = -1;
-  for (int q = t; q < n && q < t + 2 && gk[q] == gk[t]; q++) {
-    if (gv[q] & kOldTag)
-      o = (int32_t)(gv[q] & ~kOldTag);
+  const bool valid = t < nc;
+  const uint64_t k = valid ? cand[t] : 0;
+  const int qi = run_add(cnt, (int)(k >> 32), valid, 1);
+  const int qj = run_add(cnt, (int)(k & 0xffffffffu), valid, 1);
+  if (valid) at[t] = make_int2(qi, qj);
+}
+__global__ void k_group_fill(int nc, const uint64_t* cand, const int2* at, const int32_t* gstart, int32_t* gowner,
+                             int32_t* gother, int32_t* gref) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= nc) return;
+  const uint64_t k = cand[t];
+  const int i = (int)(k >> 32), j = (int)(k & 0xffffffffu);
+  const int2 q = at[t];
+  const int a = gstart[i] + q.x, b = gstart[j] + q.y;
+  gowner[a] = i;
+  gother[a] = j;
+  gref[a] = t << 1;
+  gowner[b] = j;
+  gother[b] = i;
+  gref[b] = (t << 1) | 1;
+}
+struct GroupIn {
+  int nc2, ng_old, nold;  // directed candidates, old groups, old entries
+  const int32_t* gstart;      // per body: its first directed candidate
+  const int32_t* gowner;
+  const int32_t* gother;
+  const int32_t* gref;
+  const int32_t* istart;  // old entries by owner (null without any)
+  const int32_t* opos;    // old entries: the groups headed before it
+  const uint64_t* okey;
+  uint64_t* ukey;
+  int32_t* ucand;
+  int32_t* uold;
+  int32_t* nbig;  // long segments' owners
+  int32_t* big;
+};
+// the first old group of owner b (b up to nb)
+__device__ __forceinline__ int old_first(const GroupIn& G, int b) {
+  if (!G.ng_old) return 0;
+  const int e = G.istart[b];
+  return e < G.nold ? G.opos[e] : G.ng_old;
+}
+// old groups of [o0, o1) whose other body is below v
+__device__ __forceinline__ int old_below(const GroupIn& G, int o0, int o1, int v) {
+  int lo = o0, hi = o1;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if ((int)(G.okey[mid] & 0xffffffffu) < v)
+      lo = mid + 1;
     else
-      c = (int32_t)gv[q];
+      hi = mid;
   }
-  ucand[u] = c;
-  uold[u] = o;
+  return lo - o0;
+}
+__device__ __forceinline__ void put_cand(const GroupIn& G, int slot, int owner, int other, int ref) {
+  G.ukey[slot] = ((uint64_t)(uint32_t)owner << 32) | (uint32_t)other;
+  G.ucand[slot] = ref;
+}
+__device__ __forceinline__ void put_old(const GroupIn& G, int slot, uint64_t key, int g) {
+  G.ukey[slot] = key;
+  G.uold[slot] = g;
+}
+__device__ __forceinline__ int seg_below(const int32_t* val, int s0, int s1, int v) {
+  int n = 0;
+#pragma unroll 8
+  for (int q = s0; q < s1; q++) n += val[q] < v ? 1 : 0;
+  return n;
+}
+__global__ void k_group_place(GroupIn G) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < G.nc2) {
+    const int b = G.gowner[t];
+    const int s0 = G.gstart[b], s1 = G.gstart[b + 1];
+    if (s1 - s0 > kSegMax) {
+      if (t == s0) G.big[atomicAdd(G.nbig, 1)] = b;
+      return;
+    }
+    const int v = G.gother[t];
+    const int o0 = old_first(G, b), o1 = old_first(G, b + 1);
+    put_cand(G, s0 + o0 + seg_below(G.gother, s0, s1, v) + old_below(G, o0, o1, v), b, v, G.gref[t]);
+  } else if (t < G.nc2 + G.ng_old) {
+    const int g = t - G.nc2;
+    const uint64_t key = G.okey[g];
+    const int b = (int)(key >> 32), v = (int)(key & 0xffffffffu);
+    const int s0 = G.gstart[b], s1 = G.gstart[b + 1];
+    if (s1 - s0 > kSegMax) return;
+    put_old(G, s0 + g + seg_below(G.gother, s0, s1, v), key, g);
+  }
+}
+__global__ void __launch_bounds__(kWinThreads) k_group_place_big(GroupIn G) {
+  __shared__ WinLds L;
+  const int nbig = *G.nbig, win = (int)blockIdx.y;
+  for (int q = (int)blockIdx.x; q < nbig; q += (int)gridDim.x) {
+    const int b = G.big[q];
+    const int s0 = G.gstart[b], s1 = G.gstart[b + 1];
+    const int o0 = old_first(G, b), o1 = old_first(G, b + 1);
+    const int below = win_mark(L, G.gother, s0, s1, win);
+    for (int t = s0 + (int)threadIdx.x; t < s1; t += kWinThreads) {
+      const int v = G.gother[t];
+      if ((v >> kWinBits) == win)
+        put_cand(G, s0 + o0 + below + win_rank(L, v) + old_below(G, o0, o1, v), b, v, G.gref[t]);
+    }
+    for (int g = o0 + (int)threadIdx.x; g < o1; g += kWinThreads) {
+      const uint64_t key = G.okey[g];
+      const int v = (int)(key & 0xffffffffu);
+      if ((v >> kWinBits) == win) put_old(G, s0 + g + below + win_rank(L, v), key, g);
+    }
+  }
 }
 
 // --- narrow phase ------------------------------------------------------
@@ -1225,9 +1388,7 @@ __global__ void __launch_bounds__(64, P == 1 ? 6 : 3) k_narrow(Dev d, const doub
 
 // --- merge ---------------------------------------------------------------
 struct MergeIn {
-  int ng;                    // groups (count pass with ng_pos: the groups' upper bound)
-  const int32_t* ng_pos;     // count pass: the group count is *ng_pos + *ng_flag (the
-  const int32_t* ng_flag;    // heads' scan and flag at the last key), else null
+  int ng;  // group slots
   const uint64_t* ukey;
   const int32_t* ucand;
   const int32_t* uold;
@@ -1285,27 +1446,17 @@ __device__ double pair_damp(const Dev& d, int i, int j) {
   return 2.0 * sqrt(kn * meff);
 }
 
-// The group count and the merged list's length (the count scan at it), for
-// one read with the narrow phase's totals.
-__global__ void k_merge_total(const int32_t* pos_last, const int32_t* flag_last, const int32_t* goff, int32_t* out) {
-  const int ng = *pos_last + *flag_last;
-  out[0] = ng;
-  out[1] = goff[ng];
-}
-
 template <bool WRITE>
 __global__ void k_merge(Dev d, MergeIn in, MergeOut out) {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  // the count pass runs over the groups' upper bound (+1, the scan's
-  // trailing zero) and zeroes the counts past the last group
-  const int ng = (!WRITE && in.ng_pos) ? *in.ng_pos + *in.ng_flag : in.ng;
-  if (g >= ng) {
-    if (!WRITE && g <= in.ng) out.count[g] = 0;
+  if (g > in.ng) return;
+  const int cref = g < in.ng ? in.ucand[g] : -1, oref = g < in.ng ? in.uold[g] : -1;
+  if (cref < 0 && oref < 0) {  // an empty slot, or the scan's trailing zero
+    if (!WRITE) out.count[g] = 0;
     return;
   }
   const uint64_t key = in.ukey[g];
   const int owner = (int)(key >> 32), other = (int)(key & 0xffffffffu);
-  const int cref = in.ucand[g], oref = in.uold[g];
   int os = 0, on = 0;
   if (oref >= 0) {
     os = in.ostart[oref];
@@ -1416,57 +1567,6 @@ __global__ void k_merge_fill(Dev d, int n, MergeIn in, MergeOut out) {
 }
 
 // --- CSR -----------------------------------------------------------------
-// Counts of a sorted key array without atomics (a wall owning thousands of
-// entries would serialise them): the last entry of each run writes the run's
-// length.  Its first index is found by 8-way searches, each round's 8 loads
-// independent: probes 1..8 spans back from the end, the span growing 8-fold
-// until a probe leaves the run, then the interval holding the run's start
-// cut into 8 per round (a few rounds of load latency for a run of tens of
-// entries, against a binary search's chain of log2(n) dependent loads).
-__global__ void k_count_sorted(int n, const int32_t* key, int32_t* cnt) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  const int k = key[e];
-  if (e + 1 < n && key[e + 1] == k) return;
-  // invariant: key[hi] == k, and lo < hi is -1 or an index whose key is not k
-  int hi = e, lo = -1;
-  for (long span = 1;; span *= 8) {
-    int out = 9;
-#pragma unroll
-    for (int q = 8; q >= 1; q--) {
-      const long x = (long)e - span * q;
-      if (x < 0 || key[x] != k) out = q;
-    }
-    if (out <= 8) {
-      hi = (int)((long)e - span * (out - 1));
-      const long l = (long)e - span * out;
-      lo = l < -1 ? -1 : (int)l;
-      break;
-    }
-  }
-  while (hi - lo > 1) {
-    const int st = (hi - lo + 7) / 8;
-    int nlo = lo, nhi = hi;
-#pragma unroll
-    for (int q = 1; q < 8; q++) {
-      const int x = lo + st * q;
-      if (x < hi) {
-        if (key[x] == k)
-          nhi = x < nhi ? x : nhi;
-        else
-          nlo = x > nlo ? x : nlo;
-      }
-    }
-    lo = nlo;
-    hi = nhi;
-  }
-  cnt[k] = e - hi + 1;
-}
-__global__ void k_iota(int n, int32_t* v) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n) v[e] = e;
-}
-
 // --- resultant slots -------------------------------------------------------
 // compute_resultants (Rockable.cpp:3267-3272) walks the bodies in index order
 // and each body's interactions in key order, adding to Particles[i] and
@@ -1474,86 +1574,127 @@ __global__ void k_iota(int n, int32_t* v) {
 // entries (a, b) with a < b, then its own entries (b, c), then the entries
 // (a, b) with a > b.  Body b's slots are [soff[b], soff[b+1]) with
 // soff[b] = istart[b] + jstart[b]; nlow[b] counts b's j-side entries whose
-// index is below b's own range.
-__global__ void k_slot_body(int nb, const int32_t* istart, const int32_t* jstart, const int32_t* jlist,
-                            int32_t* soff, int32_t* nlow) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b > nb) return;
-  soff[b] = istart[b] + jstart[b];
-  if (b == nb) return;
-  int lo = jstart[b], hi = jstart[b + 1];
-  const int is = istart[b];
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (jlist[mid] < is)
-      lo = mid + 1;
-    else
-      hi = mid;
-  }
-  nlow[b] = lo - jstart[b];
-}
-__global__ void k_slot_i(int n, const int32_t* ei, const int32_t* istart, const int32_t* soff, const int32_t* nlow,
-                         int32_t* spos) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  const int b = ei[e];
-  spos[2 * e] = soff[b] + nlow[b] + (e - istart[b]);
-}
-__global__ void k_slot_j(int n, const int32_t* ej, const int32_t* jlist, const int32_t* jstart,
-                         const int32_t* istart, const int32_t* soff, int32_t* spos) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const int e = jlist[q];
-  const int b = ej[e];
-  const int above = e >= istart[b] ? istart[b + 1] - istart[b] : 0;
-  spos[2 * e + 1] = soff[b] + (q - jstart[b]) + above;
-}
-// slot activity of a fresh list: the force phase rewrites it only on change
-__global__ void k_slot_act(int n, const int32_t* spos, const uint8_t* eact, uint8_t* sact) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  const uint8_t a = eact[e] & 1;
-  sact[spos[2 * e]] = a;
-  sact[spos[2 * e + 1]] = a;
-}
-__global__ void k_heavy_flag(int nb, const int32_t* soff, int heavy_min, int32_t* flag) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b < nb) flag[b] = (soff[b + 1] - soff[b]) > heavy_min ? 1 : 0;
-}
-__global__ void k_heavy_list(int nb, const int32_t* flag, const int32_t* pos, int32_t* heavy) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b < nb && flag[b]) heavy[pos[b]] = b;
-}
-
-// Chunks of 64 slots of the heavy bodies, and the count of heavy bodies that
-// are not passive.  One workgroup: thread 0 lays out the chunk offsets
-// (a few thousand heavy bodies at most), then the threads fill the chunks.
-// The heavy count is the flag scan's last value plus the last flag; out
-// receives the chunk count, the count of heavy bodies that are not passive
-// and the heavy count.
-__global__ void k_heavy_chunks(const int32_t* heavy, const int32_t* pos_last, const int32_t* flag_last,
-                               const int32_t* soff, const uint8_t* passive, int32_t* hch_off, int2* hch, int cap,
-                               int32_t* out) {
-  const int nheavy = *pos_last + *flag_last;
-  if (threadIdx.x == 0) {
-    int off = 0, np = 0;
-    for (int h = 0; h < nheavy; h++) {
-      const int b = heavy[h];
-      hch_off[h] = off;
-      off += (soff[b + 1] - soff[b] + 63) / 64;
-      np += passive[b] ? 0 : 1;
+// index is below b's own range: it is the count of b's j-side entries with a < b, and entry
+// (i, j) takes slot jstart[i] + nlow[i] + e on its owner's side, and on the
+// other the number of j's j-side entries before it, after j's own entries if
+// it comes after them.
+//
+// The j-side counts (whole in the low 32 bits, below the own range in the
+// high ones), every entry's position among its j's, and the first entry of
+// every owner (ei ascends).
+__global__ void k_csr_count(int nb, int n, const int32_t* ei, const int32_t* ej, int32_t* istart, unsigned long long* jcnt,
+                            int32_t* at) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const bool valid = t < n;
+  const int i = valid ? ei[t] : 0, j = valid ? ej[t] : 0;
+  const int q = run_add(jcnt, j, valid, (unsigned long long)(i < j ? 0x100000001ull : 1ull), i < j);
+  if (valid) at[t] = q;
+  if (t > nb) return;
+  // 8 independent loads a round instead of a binary search's one
+  int lo = 0, hi = n;  // the first entry whose owner is t or above lies in [lo, hi]
+  while (hi > lo) {
+    const int st = (hi - lo + 7) / 8;
+    int nlo = lo, nhi = hi;
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const int x = lo + st * q;
+      if (x < hi) {
+        if (ei[x] < t)
+          nlo = x + 1 > nlo ? x + 1 : nlo;
+        else
+          nhi = x < nhi ? x : nhi;
+      }
     }
-    hch_off[nheavy] = off;
-    out[0] = off;
-    out[1] = np;
-    out[2] = nheavy;
+    lo = nlo;
+    hi = nhi;
   }
-  __syncthreads();
-  for (int h = threadIdx.x; h < nheavy; h += blockDim.x) {
-    const int b = heavy[h];
-    const int k0 = soff[b], k1 = soff[b + 1];
-    for (int c = hch_off[h], k = k0; c < hch_off[h + 1] && c < cap; c++, k += 64) hch[c] = make_int2(k, min(k + 64, k1));
+  istart[t] = lo;
+}
+// the j-side entries by body, in any order, and the bodies' slots; jsum is the
+// scan of the counts, whose low 32 bits stay below 2^32
+__global__ void k_csr_fill(int nb, int n, const int32_t* ej, const int32_t* istart, const unsigned long long* jcnt,
+                           const unsigned long long* jsum, const int32_t* at, int32_t* jstart, int32_t* nlow,
+                           int32_t* jlist, int32_t* soff) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) jlist[(int32_t)jsum[ej[t]] + at[t]] = t;
+  if (t <= nb) {
+    const int32_t js = (int32_t)jsum[t];
+    jstart[t] = js;
+    soff[t] = istart[t] + js;
+    nlow[t] = (int32_t)(jcnt[t] >> 32);
   }
+}
+struct SlotIn {
+  int n;
+  const int32_t* ei;
+  const int32_t* ej;
+  const int32_t* istart;
+  const int32_t* jstart;
+  const int32_t* jlist;
+  const int32_t* nlow;
+  const uint8_t* eact;
+  int32_t* spos;
+  uint8_t* sact;
+  int32_t* nbig;
+  int32_t* big;
+};
+// the slot of j-side entry e, `before` of b's j-side entries being below it
+// (slot activity of a fresh list: the force phase rewrites it only on change)
+__device__ __forceinline__ void put_slot_j(const SlotIn& S, int b, int e, int before) {
+  const int i0 = S.istart[b];
+  const int at = i0 + S.jstart[b] + before + (e >= i0 ? S.istart[b + 1] - i0 : 0);
+  S.spos[2 * e + 1] = at;
+  S.sact[at] = S.eact[e] & 1;
+}
+__global__ void k_csr_slots(SlotIn S) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= S.n) return;
+  const int i = S.ei[t];
+  const int at = S.jstart[i] + S.nlow[i] + t;
+  S.spos[2 * t] = at;
+  S.sact[at] = S.eact[t] & 1;
+  const int e = S.jlist[t], b = S.ej[e];
+  const int s0 = S.jstart[b], s1 = S.jstart[b + 1];
+  if (s1 - s0 > kSegMax) {
+    if (t == s0) S.big[atomicAdd(S.nbig, 1)] = b;
+    return;
+  }
+  put_slot_j(S, b, e, seg_below(S.jlist, s0, s1, e));
+}
+__global__ void __launch_bounds__(kWinThreads) k_csr_slots_big(SlotIn S) {
+  __shared__ WinLds L;
+  const int nbig = *S.nbig, win = (int)blockIdx.y;
+  for (int q = (int)blockIdx.x; q < nbig; q += (int)gridDim.x) {
+    const int b = S.big[q];
+    const int s0 = S.jstart[b], s1 = S.jstart[b + 1];
+    const int below = win_mark(L, S.jlist, s0, s1, win);
+    for (int t = s0 + (int)threadIdx.x; t < s1; t += kWinThreads) {
+      const int e = S.jlist[t];
+      if ((e >> kWinBits) == win) put_slot_j(S, b, e, below + win_rank(L, e));
+    }
+  }
+}
+// The heavy bodies (more than heavy_min slots) in any order: no sum depends on
+// it.  Body and chunk offsets come from one 64-bit counter, so that they
+// ascend together: heavy body h has the chunks [hch_off[h], hch_off[h + 1]),
+// each a chunk of 64 of its slots.  out: the chunk count in the low and the
+// heavy count in the high 32 bits; np the heavy bodies that are not passive.
+// (One kernel instead of a flag, a scan, a compaction and a serial pass over
+// the list, 38 us in the last alone for 50 005 bodies: 22 us in all.)
+__global__ void k_heavy_list(int nb, const int32_t* soff, int heavy_min, const uint8_t* passive, int32_t* heavy,
+                             int32_t* hch_off, int2* hch, int cap, unsigned long long* out, int32_t* np) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= nb) return;
+  const int k0 = soff[b], k1 = soff[b + 1];
+  if (k1 - k0 <= heavy_min) return;
+  const int nch = (k1 - k0 + 63) / 64;
+  const unsigned long long at = atomicAdd(out, (1ull << 32) + (unsigned long long)nch);
+  const int h = (int)(at >> 32), c0 = (int)(uint32_t)at;
+  if (!passive[b]) atomicAdd(np, 1);
+  heavy[h] = b;
+  hch_off[h] = c0;
+  hch_off[h + 1] = c0 + nch;  // the next heavy body writes the same
+  for (int c = 0; c < nch && c0 + c < cap; c++) hch[c0 + c] = make_int2(k0 + 64 * c, min(k0 + 64 * c + 64, k1));
 }
 
 inline int nblk(long n) { return (int)((n + kBlock - 1) / kBlock); }
@@ -1578,63 +1719,39 @@ static int ensure(NLWork& w, T*& p, size_t& cap, size_t n) {
   return 0;
 }
 
-static int scan_exclusive(NLWork& w, const int32_t* in, int32_t* out, int n, hipStream_t s) {
+template <class T>
+static int scan_exclusive(NLWork& w, const T* in, T* out, int n, hipStream_t s) {
   size_t bytes = 0;
-  RK_CHECK(rocprim::exclusive_scan(nullptr, bytes, in, out, 0, (size_t)n, rocprim::plus<int32_t>(), s));
+  RK_CHECK(rocprim::exclusive_scan(nullptr, bytes, in, out, (T)0, (size_t)n, rocprim::plus<T>(), s));
   if (ensure(w, w.tmp, w.tmp_cap, bytes) != 0) return -1;
-  RK_CHECK(rocprim::exclusive_scan((void*)w.tmp, bytes, in, out, 0, (size_t)n, rocprim::plus<int32_t>(), s));
+  RK_CHECK(rocprim::exclusive_scan((void*)w.tmp, bytes, in, out, (T)0, (size_t)n, rocprim::plus<T>(), s));
   return 0;
 }
 
-template <class K, class Vv>
-static int sort_pairs(NLWork& w, const K* kin, K* kout, const Vv* vin, Vv* vout, int n, int bits, hipStream_t s) {
-  size_t bytes = 0;
-  RK_CHECK(rocprim::radix_sort_pairs(nullptr, bytes, kin, kout, vin, vout, (size_t)n, 0u, (unsigned)bits, s));
-  if (ensure(w, w.tmp, w.tmp_cap, bytes) != 0) return -1;
-  RK_CHECK(rocprim::radix_sort_pairs((void*)w.tmp, bytes, kin, kout, vin, vout, (size_t)n, 0u, (unsigned)bits, s));
-  return 0;
-}
-
-static int bits_for(uint64_t maxval) {
-  int b = 1;
-  while (b < 64 && (maxval >> b) != 0) b++;
-  return b;
-}
+// windows of values below n for the long segments
+static int windows(long n) { return (int)std::max(1L, (n + (1L << kWinBits) - 1) >> kWinBits); }
 
 int nl_build_csr(NLWork& w, int nb, EntryArrays& E, const uint8_t* passive, hipStream_t s) {
   const int n = E.n;
   if (ensure(w, E.istart, E.istart_cap, (size_t)nb + 1) || ensure(w, E.jstart, E.jstart_cap, (size_t)nb + 1) ||
       ensure(w, E.jlist, E.jlist_cap, (size_t)(n > 0 ? n : 1)) || ensure(w, w.i32a, w.i32a_cap, (size_t)nb + 1) ||
-      ensure(w, w.i32b, w.i32b_cap, (size_t)(n > 0 ? n : 1)) || ensure(w, w.i32c, w.i32c_cap, (size_t)(n > 0 ? n : 1)) ||
-      ensure(w, E.edesc, E.edesc_cap, 2 * (size_t)(n > 0 ? n : 1)))
+      ensure(w, w.i32b, w.i32b_cap, (size_t)(n > 0 ? n : 1)) || ensure(w, w.jsum, w.jsum_cap, 2 * (size_t)nb + 3) ||
+      ensure(w, E.edesc, E.edesc_cap, 2 * (size_t)(n > 0 ? n : 1)) ||
+      ensure(w, E.soff, E.soff_cap, (size_t)nb + 1) || ensure(w, w.big, w.big_cap, (size_t)nb))
     return -1;
-  // istart: counts by owner, exclusive scan over nb + 1 (trailing zero)
-  RK_CHECK(hipMemsetAsync(w.i32a, 0, sizeof(int32_t) * (nb + 1), s));
-  if (n > 0) hipLaunchKernelGGL(k_count_sorted, dim3(nblk(n)), dim3(kBlock), 0, s, n, E.ei, w.i32a);
-  if (scan_exclusive(w, w.i32a, E.istart, nb + 1, s)) return -1;
-  // jlist: stable radix sort of entry indices by j
+  // zeroed: the j-side counts and, behind them, the count of long segments
+  unsigned long long *jcnt = w.jsum, *jsum = jcnt + nb + 2;
+  int32_t *nlow = w.i32a, *nbig = reinterpret_cast<int32_t*>(jcnt + nb + 1);
+  const int grid = nblk(std::max((long)n, (long)nb + 1));
+  RK_CHECK(hipMemsetAsync(jcnt, 0, sizeof(unsigned long long) * ((size_t)nb + 2), s));
+  hipLaunchKernelGGL(k_csr_count, dim3(grid), dim3(kBlock), 0, s, nb, n, E.ei, E.ej, E.istart, jcnt, w.i32b);
+  if (scan_exclusive(w, jcnt, jsum, nb + 1, s)) return -1;
+  hipLaunchKernelGGL(k_csr_fill, dim3(grid), dim3(kBlock), 0, s, nb, n, E.ej, E.istart, jcnt, jsum, w.i32b, E.jstart,
+                     nlow, E.jlist, E.soff);
   if (n > 0) {
-    hipLaunchKernelGGL(k_iota, dim3(nblk(n)), dim3(kBlock), 0, s, n, w.i32b);
-    RK_CHECK(hipMemcpyAsync(w.i32c, E.ej, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, s));
-    if (ensure(w, w.kout, w.kout_cap, (size_t)n)) return -1;
-    if (sort_pairs(w, (const uint32_t*)w.i32c, (uint32_t*)w.kout, w.i32b, E.jlist, n,
-                   bits_for((uint64_t)(nb > 1 ? nb - 1 : 1)), s))
-      return -1;
-  }
-  // jstart: counts of the sorted j keys (a wall is the j of thousands of
-  // entries: counted by atomics, they would serialise on its counter)
-  RK_CHECK(hipMemsetAsync(w.i32a, 0, sizeof(int32_t) * (nb + 1), s));
-  if (n > 0) hipLaunchKernelGGL(k_count_sorted, dim3(nblk(n)), dim3(kBlock), 0, s, n, (const int32_t*)w.kout, w.i32a);
-  if (scan_exclusive(w, w.i32a, E.jstart, nb + 1, s)) return -1;
-  // resultant slots
-  if (ensure(w, E.soff, E.soff_cap, (size_t)nb + 1)) return -1;
-  hipLaunchKernelGGL(k_slot_body, dim3(nblk(nb + 1)), dim3(kBlock), 0, s, nb, E.istart, E.jstart, E.jlist, E.soff,
-                     w.i32a);
-  if (n > 0) {
-    hipLaunchKernelGGL(k_slot_i, dim3(nblk(n)), dim3(kBlock), 0, s, n, E.ei, E.istart, E.soff, w.i32a, E.spos);
-    hipLaunchKernelGGL(k_slot_j, dim3(nblk(n)), dim3(kBlock), 0, s, n, E.ej, E.jlist, E.jstart, E.istart, E.soff,
-                       E.spos);
-    hipLaunchKernelGGL(k_slot_act, dim3(nblk(n)), dim3(kBlock), 0, s, n, E.spos, E.eact, E.sact);
+    SlotIn S{n, E.ei, E.ej, E.istart, E.jstart, E.jlist, nlow, E.eact, E.spos, E.sact, nbig, w.big};
+    hipLaunchKernelGGL(k_csr_slots, dim3(nblk(n)), dim3(kBlock), 0, s, S);
+    if (n > kSegMax) hipLaunchKernelGGL(k_csr_slots_big, dim3(kBigGrid, windows(n)), dim3(kWinThreads), 0, s, S);
   }
   RK_CHECK(hipGetLastError());
   return nl_build_heavy(w, nb, E, passive, s);
@@ -1672,12 +1789,7 @@ int nl_build_heavy(NLWork& w, int nb, EntryArrays& E, const uint8_t* passive, hi
   E.nhch = 0;
   E.nheavy_np = 0;
   if (nb <= 0 || !E.soff) return 0;
-  if (ensure(w, E.heavy, E.heavy_cap, (size_t)nb) || ensure(w, w.i32a, w.i32a_cap, (size_t)nb + 1) ||
-      ensure(w, w.i32c, w.i32c_cap, (size_t)nb + 1) || ensure(w, w.counter, w.counter_cap, 4))
-    return -1;
-  hipLaunchKernelGGL(k_heavy_flag, dim3(nblk(nb)), dim3(kBlock), 0, s, nb, E.soff, w.heavy_min, w.i32a);
-  if (scan_exclusive(w, w.i32a, w.i32c, nb, s)) return -1;
-  hipLaunchKernelGGL(k_heavy_list, dim3(nblk(nb)), dim3(kBlock), 0, s, nb, w.i32a, w.i32c, E.heavy);
+  if (ensure(w, E.heavy, E.heavy_cap, (size_t)nb) || ensure(w, w.hcount, w.hcount_cap, 2)) return -1;
   // chunk table sized as if every body were heavy: at most (slots of all
   // bodies) / 64 + one per body, so that the heavy count is read once, with
   // the chunks'
@@ -1693,17 +1805,18 @@ int nl_build_heavy(NLWork& w, int nb, EntryArrays& E, const uint8_t* passive, hi
     }
     E.hpart_cap = cap;
   }
-  hipLaunchKernelGGL(k_heavy_chunks, dim3(1), dim3(kBlock), 0, s, E.heavy, w.i32c + nb - 1, w.i32a + nb - 1, E.soff,
-                     passive, E.hch_off, E.hch, (int)cap, w.counter);
-  int32_t cnt[3] = {0, 0, 0};
-  if (read_small(w, s, {{cnt, {w.counter, 3 * sizeof(int32_t)}}})) return -1;
+  RK_CHECK(hipMemsetAsync(w.hcount, 0, 2 * sizeof(unsigned long long), s));
+  hipLaunchKernelGGL(k_heavy_list, dim3(nblk(nb)), dim3(kBlock), 0, s, nb, E.soff, w.heavy_min, passive, E.heavy,
+                     E.hch_off, E.hch, (int)cap, w.hcount, reinterpret_cast<int32_t*>(w.hcount + 1));
+  int32_t cnt[3] = {0, 0, 0};  // chunks, heavy, not passive
+  if (read_small(w, s, {{cnt, {w.hcount, 3 * sizeof(int32_t)}}})) return -1;
   if ((size_t)cnt[0] > cap) {
     snprintf(w.err, sizeof(w.err), "heavy-body chunk table overflow");
     return -1;
   }
   E.nhch = cnt[0];
-  E.nheavy_np = cnt[1];
-  E.nheavy = cnt[2];
+  E.nheavy = cnt[1];
+  E.nheavy_np = cnt[2];
   return 0;
 }
 
@@ -1715,6 +1828,22 @@ int nl_rebuild(NLWork& w, Dev& d, const NLParams& p, EntryArrays& cur, EntryArra
   if (ensure(w, w.baabb, w.baabb_cap, (size_t)6 * nb)) return -1;
   hipLaunchKernelGGL(k_obb, dim3(nblk(nb)), dim3(kBlock), 0, s, d, w.bobb, w.baabb);
   const double half = 0.5 * p.DVerlet;
+
+  // ---- groups of the current list (their count is read with the candidates')
+  const int nold = cur.n;
+  int ng_old = 0, oend[2] = {0, 0};
+  if (ensure(w, w.i32b, w.i32b_cap, (size_t)std::max(nold, 1) + 1) ||
+      ensure(w, w.i32c, w.i32c_cap, (size_t)std::max(nold, 1) + 1) ||
+      ensure(w, w.okey, w.okey_cap, (size_t)std::max(nold, 1)) ||
+      ensure(w, w.ostart, w.ostart_cap, (size_t)std::max(nold, 1) + 1))
+    return -1;
+  if (nold > 0) {
+    hipLaunchKernelGGL(k_old_heads, dim3(nblk(nold)), dim3(kBlock), 0, s, nold, cur.ei, cur.ej, w.i32b);
+    if (scan_exclusive(w, w.i32b, w.i32c, nold, s)) return -1;
+    hipLaunchKernelGGL(k_old_compact, dim3(nblk(nold)), dim3(kBlock), 0, s, nold, cur.ei, cur.ej, w.i32b, w.i32c,
+                       w.okey, w.ostart);
+  }
+  const int32_t* olast = w.i32c + std::max(nold, 1) - 1;
 
   // ---- broad phase: candidate pairs
   if (ensure(w, w.counter, w.counter_cap, 4) || ensure(w, w.scnt, w.scnt_cap, (size_t)kStripes * kStripeStride) ||
@@ -1792,8 +1921,15 @@ int nl_rebuild(NLWork& w, Dev& d, const NLParams& p, EntryArrays& cur, EntryArra
     }
     hipLaunchKernelGGL(k_stripe_scan, dim3(1), dim3(kStripes), 0, s, w.scnt, w.soff, w.counter + 2);
     int tm[2] = {0, 0};
-    if (read_small(w, s, {{tm, {w.counter + 2, sizeof(int) * 2}}})) return -1;
+    if (nold > 0) {
+      if (read_small(w, s, {{tm, {w.counter + 2, sizeof(int) * 2}}, {&oend[0], {olast, sizeof(int)}},
+                            {&oend[1], {w.i32b + nold - 1, sizeof(int)}}}))
+        return -1;
+    } else if (read_small(w, s, {{tm, {w.counter + 2, sizeof(int) * 2}}})) {
+      return -1;
+    }
     nc = tm[0];
+    ng_old = oend[0] + oend[1];
     if (tm[1] <= rcap) {
       if (ensure(w, w.cand, w.cand_cap, (size_t)std::max(nc, 1))) return -1;
       hipLaunchKernelGGL(k_stripe_gather, dim3((rcap + kBlock - 1) / kBlock, kStripes), dim3(kBlock), 0, s, w.cstripe,
@@ -1874,59 +2010,53 @@ int nl_rebuild(NLWork& w, Dev& d, const NLParams& p, EntryArrays& cur, EntryArra
     if (launch_narrow(narrow_rcap)) return -1;
   }
 
-  // ---- old groups
-  const int nold = cur.n;
-  int ng_old = 0;
-  if (ensure(w, w.i32b, w.i32b_cap, (size_t)std::max(nold, 1) + 1) ||
-      ensure(w, w.i32c, w.i32c_cap, (size_t)std::max(nold, 1) + 1) ||
-      ensure(w, w.okey, w.okey_cap, (size_t)std::max(nold, 1)) ||
-      ensure(w, w.ostart, w.ostart_cap, (size_t)std::max(nold, 1) + 1))
-    return -1;
-  if (nold > 0) {
-    hipLaunchKernelGGL(k_old_heads, dim3(nblk(nold)), dim3(kBlock), 0, s, nold, cur.ei, cur.ej, w.i32b);
-    if (scan_exclusive(w, w.i32b, w.i32c, nold, s)) return -1;
-    hipLaunchKernelGGL(k_old_compact, dim3(nblk(nold)), dim3(kBlock), 0, s, nold, cur.ei, cur.ej, w.i32b, w.i32c,
-                       w.okey, w.ostart);
-    int last[2];
-    if (read_small(w, s, {{&last[0], {w.i32c + nold - 1, sizeof(int)}}, {&last[1], {w.i32b + nold - 1, sizeof(int)}}}))
-      return -1;
-    ng_old = last[0] + last[1];
-  }
-  RK_CHECK(hipMemcpyAsync(w.ostart + ng_old, &nold, sizeof(int), hipMemcpyHostToDevice, s));
-
-  // ---- unique directed groups
+  // ---- directed groups, ordered by (owner, other)
   const int ngk = 2 * nc + ng_old;
-  int ng = 0;
-  if (ensure(w, w.gk, w.gk_cap, (size_t)std::max(ngk, 1)) || ensure(w, w.gk2, w.gk2_cap, (size_t)std::max(ngk, 1)) ||
-      ensure(w, w.gv, w.gv_cap, (size_t)std::max(ngk, 1)) || ensure(w, w.gv2, w.gv2_cap, (size_t)std::max(ngk, 1)) ||
-      ensure(w, w.gflag, w.gflag_cap, (size_t)std::max(ngk, 1)) ||
-      ensure(w, w.gpos, w.gpos_cap, (size_t)std::max(ngk, 1)) ||
+  const size_t nz = (size_t)nb + 2;  // zeroed: counts, the count of long segments
+  if (ensure(w, w.gstart, w.gstart_cap, (size_t)nb + 1) || ensure(w, w.i32a, w.i32a_cap, nz) ||
+      ensure(w, w.big, w.big_cap, (size_t)nb) || ensure(w, w.gseg, w.gseg_cap, 8 * (size_t)std::max(nc, 1)) ||
       ensure(w, w.ukey, w.ukey_cap, (size_t)std::max(ngk, 1)) ||
-      ensure(w, w.ucand, w.ucand_cap, (size_t)std::max(ngk, 1)) ||
-      ensure(w, w.uold, w.uold_cap, (size_t)std::max(ngk, 1)) ||
+      ensure(w, w.uref, w.uref_cap, 2 * (size_t)std::max(ngk, 1)) ||
       ensure(w, w.gcount, w.gcount_cap, (size_t)std::max(ngk, 1) + 1) ||
       ensure(w, w.goff, w.goff_cap, (size_t)std::max(ngk, 1) + 1))
     return -1;
   if (ngk > 0) {
-    int bb = 1;
-    while ((1ll << bb) < (long long)nb) bb++;
-    hipLaunchKernelGGL(k_fill_groups, dim3(nblk(nc + ng_old)), dim3(kBlock), 0, s, nc, w.cand, ng_old, w.okey, w.gk,
-                       w.gv, bb);
-    if (sort_pairs(w, w.gk, w.gk2, w.gv, w.gv2, ngk, 2 * bb, s)) return -1;
-    hipLaunchKernelGGL(k_group_heads, dim3(nblk(ngk)), dim3(kBlock), 0, s, ngk, w.gk2, w.gflag);
-    if (scan_exclusive(w, w.gflag, w.gpos, ngk, s)) return -1;
-    hipLaunchKernelGGL(k_group_compact, dim3(nblk(ngk)), dim3(kBlock), 0, s, ngk, w.gk2, w.gv2, w.gflag, w.gpos,
-                       w.ukey, w.ucand, w.uold, bb);
+    int2* at = reinterpret_cast<int2*>(w.gseg + 6 * (size_t)nc);
+    GroupIn G;
+    G.nc2 = 2 * nc;
+    G.ng_old = ng_old;
+    G.nold = nold;
+    G.gstart = w.gstart;
+    G.gowner = w.gseg;
+    G.gother = w.gseg + 2 * (size_t)nc;
+    G.gref = w.gseg + 4 * (size_t)nc;
+    G.istart = cur.istart;
+    G.opos = w.i32c;
+    G.okey = w.okey;
+    G.ukey = w.ukey;
+    G.ucand = w.uref;
+    G.uold = w.uref + ngk;
+    G.nbig = w.i32a + nb + 1;
+    G.big = w.big;
+    RK_CHECK(hipMemsetAsync(w.i32a, 0, sizeof(int32_t) * nz, s));
+    RK_CHECK(hipMemsetAsync(w.uref, 0xff, sizeof(int32_t) * 2 * (size_t)ngk, s));
+    if (nc > 0) hipLaunchKernelGGL(k_group_count, dim3(nblk(nc)), dim3(kBlock), 0, s, nc, w.cand, w.i32a, at);
+    if (scan_exclusive(w, w.i32a, w.gstart, nb + 1, s)) return -1;
+    if (nc > 0)
+      hipLaunchKernelGGL(k_group_fill, dim3(nblk(nc)), dim3(kBlock), 0, s, nc, w.cand, at, w.gstart, w.gseg,
+                         w.gseg + 2 * (size_t)nc, w.gseg + 4 * (size_t)nc);
+    hipLaunchKernelGGL(k_group_place, dim3(nblk(ngk)), dim3(kBlock), 0, s, G);
+    if (2 * nc > kSegMax)
+      hipLaunchKernelGGL(k_group_place_big, dim3(kBigGrid, windows(nb)), dim3(kWinThreads), 0, s, G);
+    RK_CHECK(hipGetLastError());
   }
 
   // ---- merge: count, scan, allocate, write
   MergeIn in;
   in.ng = ngk;
-  in.ng_pos = ngk > 0 ? w.gpos + ngk - 1 : nullptr;
-  in.ng_flag = ngk > 0 ? w.gflag + ngk - 1 : nullptr;
   in.ukey = w.ukey;
-  in.ucand = w.ucand;
-  in.uold = w.uold;
+  in.ucand = w.uref;
+  in.uold = w.uref + ngk;
   in.ostart = w.ostart;
   in.cbase = w.cbase;
   in.cnf = w.cnf;
@@ -1949,56 +2079,54 @@ int nl_rebuild(NLWork& w, Dev& d, const NLParams& p, EntryArrays& cur, EntryArra
   out.offset = w.goff;
   int nnew = 0;
   if (ngk > 0) {
-    // count pass over the groups' upper bound, its scan, then one read: the
-    // group count, the merged length and the narrow phase's stripe totals
+    // count pass over the groups' slots, its scan, then one read: the merged
+    // length and the narrow phase's stripe totals
     auto count_pass = [&]() -> int {
       hipLaunchKernelGGL(k_merge<false>, dim3(nblk((long)ngk + 1)), dim3(kBlock), 0, s, d, in, out);
       if (scan_exclusive(w, w.gcount, w.goff, ngk + 1, s)) return -1;
-      hipLaunchKernelGGL(k_merge_total, dim3(1), dim3(1), 0, s, in.ng_pos, in.ng_flag, w.goff, w.counter);
       return 0;
     };
     if (count_pass()) return -1;
-    int rd[4] = {0, 0, 0, 0}, nrest = 0;
+    int rd[2] = {0, 0}, nrest = 0;
     if (launch_narrow) {
-      if (read_small(w, s, {{rd, {w.counter, 4 * sizeof(int)}}, {&nrest, {w.scnt + 1, sizeof(int)}}})) return -1;
-    } else {
-      if (read_small(w, s, {{rd, {w.counter, 2 * sizeof(int)}}})) return -1;
+      if (read_small(w, s, {{&nnew, {w.goff + ngk, sizeof(int)}},
+                            {rd, {w.counter + 2, 2 * sizeof(int)}},
+                            {&nrest, {w.scnt + 1, sizeof(int)}}}))
+        return -1;
+    } else if (read_small(w, s, {{&nnew, {w.goff + ngk, sizeof(int)}}})) {
+      return -1;
     }
     bool again = false;
     if (launch_narrow && nrest > narrow_done) {  // more pairs than the grid covered
       launch_rest(narrow_rcap, narrow_done, nrest - narrow_done);
       hipLaunchKernelGGL(k_stripe_scan, dim3(1), dim3(kStripes), 0, s, w.scnt, w.soff, w.counter + 2);
-      if (read_small(w, s, {{rd + 2, {w.counter + 2, 2 * sizeof(int)}}})) return -1;
+      if (read_small(w, s, {{rd, {w.counter + 2, 2 * sizeof(int)}}})) return -1;
       again = true;
     }
     if (launch_narrow) w.rest_hint = nrest;
-    if (launch_narrow && rd[3] > narrow_rcap) {
+    if (launch_narrow && rd[1] > narrow_rcap) {
       for (int attempt = 0;; attempt++) {
         if (attempt == 2) {
           snprintf(w.err, sizeof(w.err), "narrow phase overflow");
           return -1;
         }
-        w.near_hint = kStripes * (rd[3] + rd[3] / 4 + 64);
+        w.near_hint = kStripes * (rd[1] + rd[1] / 4 + 64);
         narrow_rcap = std::max(64, (w.near_hint + kStripes - 1) / kStripes);
         if (launch_narrow(narrow_rcap)) return -1;
-        if (read_small(w, s, {{rd + 2, {w.counter + 2, 2 * sizeof(int)}}})) return -1;
-        if (rd[3] <= narrow_rcap) break;
+        if (read_small(w, s, {{rd, {w.counter + 2, 2 * sizeof(int)}}})) return -1;
+        if (rd[1] <= narrow_rcap) break;
       }
       in.nearbuf = w.nearbuf;
       again = true;
     }
     if (again) {
       if (count_pass()) return -1;
-      if (read_small(w, s, {{rd, {w.counter, 2 * sizeof(int)}}})) return -1;
+      if (read_small(w, s, {{&nnew, {w.goff + ngk, sizeof(int)}}})) return -1;
     }
-    ng = rd[0];
-    nnew = rd[1];
   }
-  in.ng = ng;
-  in.ng_pos = in.ng_flag = nullptr;
   if (entries_reserve(w, nxt, nnew) != 0) return -1;
   nxt.n = nnew;
-  if (ng > 0 && nnew > 0) {
+  if (nnew > 0) {
     out.ei = nxt.ei;
     out.ej = nxt.ej;
     out.esub = nxt.esub;
@@ -2011,13 +2139,11 @@ int nl_rebuild(NLWork& w, Dev& d, const NLParams& p, EntryArrays& cur, EntryArra
     out.ekey = nxt.ekey;
     if (ensure(w, w.msrc, w.msrc_cap, (size_t)nnew)) return -1;
     out.src = w.msrc;
-    hipLaunchKernelGGL(k_merge<true>, dim3(nblk(ng)), dim3(kBlock), 0, s, d, in, out);
+    hipLaunchKernelGGL(k_merge<true>, dim3(nblk(ngk)), dim3(kBlock), 0, s, d, in, out);
     hipLaunchKernelGGL(k_merge_fill, dim3(nblk(nnew)), dim3(kBlock), 0, s, d, nnew, in, out);
   }
   RK_CHECK(hipGetLastError());
-  if (nl_build_csr(w, nb, nxt, d.passive, s) != 0) return -1;
-  RK_CHECK(hipStreamSynchronize(s));
-  return 0;
+  return nl_build_csr(w, nb, nxt, d.passive, s);  // (ends with a read)
 }
 
 int entries_reserve(NLWork& w, EntryArrays& E, int n) {
@@ -2072,9 +2198,9 @@ void entries_free(EntryArrays& E) {
 void nl_work_free(NLWork& w) {
   void* ps[] = {w.plist,
                 w.cstripe, w.scnt, w.soff, w.bobb,  w.baabb, w.counter, w.cand,  w.cbase, w.cnf,   w.cnb,   w.nearbuf, w.okey,  w.ostart,
-                w.gk,    w.gk2,   w.gv,      w.gv2,   w.gflag, w.gpos,  w.ukey,  w.ucand,   w.uold,  w.gcount,
+                w.gstart, w.gseg, w.big, w.jsum, w.hcount, w.ukey,  w.uref,  w.gcount,
                 w.goff,  w.tmp,   w.i32a,    w.i32b,  w.i32c,  w.f64a,  w.cell_of, w.ccount, w.cstart, w.cfill,
-                w.cbody, w.over, w.gedge, w.gface, w.kout, w.msrc};
+                w.cbody, w.over, w.gedge, w.gface, w.msrc};
   for (void* q : ps)
     if (q) (void)hipFree(q);
   if (w.pin) (void)hipHostFree(w.pin);

@@ -38,7 +38,7 @@ struct EntryArrays {
   size_t istart_cap = 0;
   int32_t* jstart = nullptr;
   size_t jstart_cap = 0;
-  int32_t* jlist = nullptr;
+  int32_t* jlist = nullptr;  // entries by j, in any order within a body
   size_t jlist_cap = 0;
   int32_t* soff = nullptr;
   size_t soff_cap = 0;
@@ -92,7 +92,6 @@ struct NLWork {
   RK_BUF(int32_t, plist)  // narrow phase: the candidates left to the wavefronts (their count in scnt[1])
   RK_BUF(float, gedge)
   RK_BUF(float, gface)
-  RK_BUF(int32_t, kout)
   RK_BUF(int, counter)
   RK_BUF(uint64_t, cand)
   RK_BUF(uint64_t, cstripe)
@@ -104,15 +103,13 @@ struct NLWork {
   RK_BUF(uint32_t, nearbuf)
   RK_BUF(uint64_t, okey)
   RK_BUF(int32_t, ostart)
-  RK_BUF(uint64_t, gk)
-  RK_BUF(uint64_t, gk2)
-  RK_BUF(uint32_t, gv)
-  RK_BUF(uint32_t, gv2)
-  RK_BUF(int32_t, gflag)
-  RK_BUF(int32_t, gpos)
+  RK_BUF(int32_t, gstart)  // per body: its first directed candidate
+  RK_BUF(int32_t, gseg)    // directed candidates by owner: owner, other, reference; then the candidates' positions
+  RK_BUF(unsigned long long, jsum)    // j-side counts, their scan
+  RK_BUF(unsigned long long, hcount)  // heavy bodies and chunks, heavy bodies that are not passive
+  RK_BUF(int32_t, big)     // owners of long segments
   RK_BUF(uint64_t, ukey)
-  RK_BUF(int32_t, ucand)
-  RK_BUF(int32_t, uold)
+  RK_BUF(int32_t, uref)    // per group slot: its candidate, then its old group (-1: none)
   RK_BUF(int32_t, gcount)
   RK_BUF(int32_t, goff)
   RK_BUF(int32_t, msrc)  // merge: per new entry, the old entry it keeps (-1 for a fresh one)

@@ -1,0 +1,71 @@
+"""Places by counts in the neighbour-list rebuild: a body's directed groups
+and its entries as second body are placed by loops over short segments and by
+bitmaps over long ones, in windows of 2^18 values."""
+import numpy as np
+import pytest
+
+from tests.test_gpu_parity import assert_bodies_equal, assert_interactions_equal
+
+pytestmark = pytest.mark.gpu
+
+
+def _engine(tmp_path, dims, spacing=2.002, **kw):
+    from rockable_amd import decks as D
+    from rockable_amd.engine import Engine
+    shapes, deck = D.sphere_lattice_deck(dims=dims, spacing_factor=spacing, seed=5, nl="linkCells", **kw)
+    path = D.write_deck(str(tmp_path), shapes, deck)
+    return Engine(path), path
+
+
+@pytest.mark.parametrize("dims", [(1, 1, 1), (16, 16, 1), (16, 32, 1), (27, 19, 1), (40, 40, 2)])
+def test_lists_match_oracle(tmp_path, dims):
+    """Floors of 1, 256, 512, 513 and 1 600 spheres, so segments of both kinds
+    and at the line between them, rebuilt from an empty list and from their
+    own: the lists and the motion equal the serial oracle's bit for bit."""
+    from oracle.rk_oracle import Oracle
+    e, path = _engine(tmp_path, dims)
+    o = Oracle(path)
+    for _ in range(3):
+        e.update_nl()
+        o.update_nl()
+        assert_interactions_equal(e.interactions(), o.interactions(), fields=("dn", "fn", "ft", "mom", "damp", "stick"))
+        e.step(5)
+        o.run_steps(5)
+        assert_bodies_equal(e.bodies(), o.bodies())
+
+
+def test_windows_past_the_first(tmp_path):
+    """265 200 spheres on a floor: body indices and entry indices beyond one
+    window.  The list is that of the lattice: every sphere with its axis
+    neighbours, with the floor and with the walls, in ascending order, each
+    pair once and unchanged by a rebuild; the resultants add up over it."""
+    dims = (340, 260, 3)
+    e, _ = _engine(tmp_path, dims, vmax=0.0)
+    e.set_option("exact_sums", 1)
+    e.update_nl()
+    a = e.interactions()
+    e.update_nl()
+    assert_interactions_equal(e.interactions(), a)
+    nw, (nx, ny, nz) = 5, dims
+    i, j = a["i"].astype(np.int64), a["j"].astype(np.int64)
+    key = i * (nw + nx * ny * nz) + j
+    assert np.all(np.diff(key) >= 0)
+    ss = (i >= nw) & (j >= nw)
+    idx = np.arange(nx * ny * nz).reshape(nx, ny, nz) + nw
+    want = np.concatenate([np.stack([p.ravel(), q.ravel()], 1) for p, q in
+                           ((idx[1:], idx[:-1]), (idx[:, 1:], idx[:, :-1]), (idx[:, :, 1:], idx[:, :, :-1]))])
+    want = np.unique(np.sort(want, axis=1), axis=0)
+    got = np.sort(np.stack([i[ss], j[ss]], 1), axis=1)
+    assert len(got) == len(want)
+    assert np.array_equal(np.unique(got, axis=0), want)
+    floor = np.unique(np.concatenate([i[(j < nw)], j[(i < nw)]]))
+    edge = np.unique(np.concatenate([idx[:, :, 0].ravel(), idx[0].ravel(), idx[-1].ravel(), idx[:, 0].ravel(),
+                                     idx[:, -1].ravel()]))
+    assert np.array_equal(floor, edge)
+    b, _ = _engine(tmp_path, dims, vmax=0.0)
+    b.set_option("exact_sums", 1)
+    b.set_option("heavy_min", 8)
+    b.update_nl()
+    e.step(20)
+    b.step(20)
+    assert_bodies_equal(e.bodies(), b.bodies())
