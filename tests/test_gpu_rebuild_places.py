@@ -69,3 +69,33 @@ def test_windows_past_the_first(tmp_path):
     e.step(20)
     b.step(20)
     assert_bodies_equal(e.bodies(), b.bodies())
+
+
+def test_more_pairs_left_than_the_last_rebuild(tmp_path):
+    """The narrow phase's grid comes from the last rebuild's count of the pairs
+    left to it: hulls far apart first, so that the second rebuild has thousands
+    more than the grid covers, against an engine that starts from the second
+    state."""
+    from rockable_amd import decks as D
+    from rockable_amd.engine import Engine
+    shapes, deck = D.compact_pour_deck(n_bodies=2000, seed=2, n_shapes=8, box_in_sizes=(12, 12, 60))
+    deck.DVerlet = deck.dVerlet = 3e-3  # every pair of neighbours listed
+    path = D.write_deck(str(tmp_path), shapes, deck)
+    a, b = Engine(path), Engine(path)
+    near = a.bodies()["pos"].copy()
+    far = near * 4.0
+    a.set_bodies(pos=far)
+    a.update_nl()
+    few = a.counts()["nlisted"]
+    a.set_bodies(pos=near)
+    a.update_nl()
+    b.set_bodies(pos=near)
+    b.update_nl()
+    assert b.counts()["nlisted"] > few + 2000
+    keys = ("i", "j", "type", "isub", "jsub")
+    x, y = a.interactions(), b.interactions()
+    have = set(zip(*(x[k].tolist() for k in keys)))
+    want = set(zip(*(y[k].tolist() for k in keys)))
+    assert want <= have
+    kept = have - want  # entries of the far list that no near test looks at again stay listed
+    assert len(kept) <= few
