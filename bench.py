@@ -53,7 +53,8 @@ PEAK_HBM_GBS = 8000.0
 # HBM bytes per force-phase launch on the 50 005-body settled pour:
 # rocprofv3 FETCH_SIZE and WRITE_SIZE, each scaled by what it reads for a
 # plain 256 MiB device copy (factors 2.0 and 1.0).  With the far-entry skip
-# (k_interact_seg + k_gather + k_heavy_finish): 137.0 MB read + 27.9 MB
+# (the per-step entry test that k_interact_list replaced, k_gather and
+# k_heavy_finish; not counted again since): 137.0 MB read + 27.9 MB
 # written, profiles/c2_force_phase_traffic.md; without it (k_interact +
 # k_gather + k_heavy_finish, measured before the skip): 171.3 + 36.3 MB.
 TRAFFIC_BYTES_PER_LAUNCH = {1: 164.9e6, 0: 207.6e6}
@@ -719,7 +720,7 @@ def main():
                    "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": achieved / PEAK_HBM_GBS, "traffic": TRAFFIC_BYTES_PER_LAUNCH[skip_far],
-                     "kernel": "force phase (k_interact_seg with the far-entry skip, else k_interact or k_geom + "
+                     "kernel": "force phase (k_interact_list with the far-entry skip, else k_interact or k_geom + "
                                "k_law; then k_gather + k_heavy_finish)",
                      "algorithmic_bytes_per_launch": bytes_per},
     }
