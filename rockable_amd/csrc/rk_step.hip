@@ -1335,19 +1335,25 @@ __device__ __forceinline__ void add_motion_bound_with(const Dev& d, const StepPa
   const double mag = fabs(P.px) + fabs(P.py) + fabs(P.pz);
   set_bound(d, b, cb + (step + 1e-15 * (1.0 + mag)), step, limit, par);
 }
-// The driven bodies' bounds (by one workgroup): those without a control stay
-// where they are, which in the moving frame is a motion of |D|.  predict: the
-// step is taken now; relisted: the list in use was written in this step.
-__device__ __forceinline__ void driven_bounds(const Dev& d, const StepParams& sp, bool predict, bool relisted, int par) {
+// The bound of driven body b, by one thread: without a control it stays where
+// it is, which in the moving frame is a motion of |D|.  predict: the step is
+// taken now; relisted: the list in use was written in this step, for the
+// allowance before it.  A body's limit and allowance have no other writer
+// in the launch, so that the limit is the allowance the list was written for.
+__device__ __forceinline__ void driven_bound(const Dev& d, const StepParams& sp, int b, bool predict, bool relisted,
+                                             int par) {
   if (!d.skip_far) return;
+  const double limit = relisted ? d.ahead[b] : d.climit[b];
+  if (relisted) d.climit[b] = limit;
+  const double cb = d.cbound[b];
+  if (!predict || !(cb < INFINITY)) return;
   const double ux = sp.dt * d.drift[0], uy = sp.dt * d.drift[1], uz = sp.dt * d.drift[2];
   const double step = sqrt(ux * ux + uy * uy + uz * uz);
-  for (int b = threadIdx.x; b < d.nDriven; b += blockDim.x) {
-    const double limit = relisted ? d.ahead[b] : d.climit[b];
-    if (relisted) d.climit[b] = limit;
-    const double cb = d.cbound[b];
-    if (predict && cb < INFINITY) set_bound(d, b, cb + (step + 1e-15), step, limit, par);
-  }
+  set_bound(d, b, cb + (step + 1e-15), step, limit, par);
+}
+// all of them by one workgroup, in a predictor's launch
+__device__ __forceinline__ void driven_bounds(const Dev& d, const StepParams& sp, int par) {
+  for (int b = threadIdx.x; b < d.nDriven; b += blockDim.x) driven_bound(d, sp, b, true, false, par);
 }
 __device__ __forceinline__ void add_motion_bound(const Dev& d, const StepParams& sp, int b, const BodyKin& old,
                                                  const BodyKin& P, int par) {
@@ -1502,7 +1508,6 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
       d.ls->want[1 - A.par] = 1;
     }
   }
-  if (blockIdx.x == 0 && (predict || relisted)) driven_bounds(d, sp, predict, relisted, 1 - A.par);
   GuardAcc ga;
   ga.kp = 0ull;
   ga.kw = ~0ull;
@@ -1524,6 +1529,8 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
     k0 = d.soff[b0];
     kend = d.soff[b0 + nbk];
   }
+  // (a driven body has a workgroup of its own, also where it is heavy)
+  if (driven && t == 0 && (predict || relisted)) driven_bound(d, sp, b0, predict, relisted, 1 - A.par);
   if (chunks || (driven && kend - k0 > d.heavy_min)) {  // no body to finish
     if (guard && t == 0) {
       if (A.fuse && !chunks) guard_body(d, sp, b0, d.kin[b0], rst, ga);  // (else k_heavy_finish does)
@@ -1553,7 +1560,7 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
       rmx = d.rmax[b];
       lim = relisted ? d.ahead[b] : d.climit[b];
     }
-    if (relisted) d.climit[b] = d.ahead[b];
+    if (relisted && !driven) d.climit[b] = d.ahead[b];
   }
   // the summing lanes' bodies and slot ranges
   const int lb = t / kLanes, lc = t % kLanes;
@@ -2271,7 +2278,7 @@ __global__ void __launch_bounds__(kBlock) k_predict(Dev d, StepParams sp, int gl
   const int gid = blockIdx.x * blockDim.x + threadIdx.x;
   if (blockIdx.x == 0) {
     drive_controls_block(d, sp);
-    driven_bounds(d, sp, true, false, par);
+    driven_bounds(d, sp, par);
   }
   // free bodies (Rockable.cpp:2036-2055), a grid-stride loop
   for (int b = gid; b < d.nb; b += gridDim.x * blockDim.x) {
@@ -2306,7 +2313,7 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
   const int t = threadIdx.x;
   if (blockIdx.x == 0) {
     drive_controls_block(d, sp);
-    driven_bounds(d, sp, true, false, par);
+    driven_bounds(d, sp, par);
     if (driven_glob) {
       __syncthreads();  // the driven poses, written by thread 0, are visible to the workgroup
       for (int k = t; k < d.nvdriven; k += blockDim.x) {
@@ -2397,7 +2404,7 @@ __global__ void __launch_bounds__(kBlock) k_predict_vtx(Dev d, StepParams sp, in
   if (frozen(d)) return;
   if (blockIdx.x == 0) {
     drive_controls_block(d, sp);
-    driven_bounds(d, sp, true, false, par);
+    driven_bounds(d, sp, par);
   }
   const int lane = threadIdx.x & 63;
   for (int wv = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6); wv < d.nwv;

@@ -53,3 +53,40 @@ def test_list_equals_full_evaluation(tmp_path, n, flow):
         assert_interactions_equal(a.interactions(), b.interactions(), fields=("dn", "fn", "ft", "mom", "damp", "stick"))
         contacts += a.counts()["nactive"]
     assert contacts > 0 or n < 200  # the bodies met
+
+
+@pytest.mark.parametrize("gap", [201.05, 201.25, 201.45])
+@pytest.mark.parametrize("ndriven,heavy_min", [(1, None), (1, 1), (3, None), (3, 1)])
+def test_limit_of_an_uncontrolled_driven_body(tmp_path, gap, ndriven, heavy_min):
+    """A still driven sphere and a free one closing on it, whose allowances run
+    out a fraction of a step apart: in the frame of the free bodies' mean
+    velocity the driven sphere moves s = dt |mean| per step and the free one
+    0.995 s, either's allowance is 100.5 s, and the pair is left off the list of
+    step 2 at a gap a little above the two together, which is gone 101 steps
+    later.  The driven sphere's bound passes its limit at just that step,
+    which therefore has to test every entry again."""
+    from rockable_amd.engine import Engine
+    R, dt, u = 0.05, 1e-6, 0.1
+    s = dt * u
+    deck = D.Deck(dt=dt, tmax=1e3, interVerlet=1e3, interConf=1e3, DVerlet=5e-3, dVerlet=100.5 * s / 0.01,
+                  density={0: 1000.0}, gravity=(0.0, 0.0, 0.0), nDriven=ndriven,
+                  params=D.contact_params(1e5, 8e4, 0.25, 0.3))
+    # the last driven sphere is the one that is met; the others are far away
+    deck.bodies = [D.Body("S", pos=(0.0, 10.0 * (ndriven - 1 - k), 0.0)) for k in range(ndriven)]
+    deck.bodies.append(D.Body("S", pos=(2 * R + (gap + 2 * 1.995) * s, 0.0, 0.0), vel=(-1.995 * u, 0.0, 0.0)))
+    deck.bodies.append(D.Body("S", pos=(-2 * R - 5e-4, 0.0, 0.0), vel=(-0.005 * u, 0.0, 0.0)))
+    path = D.write_deck(str(tmp_path), [D.sphere_shape("S", R)], deck)
+    a, b = Engine(path), Engine(path)
+    for e, skip in ((a, 1), (b, 0)):
+        e.set_option("record_geometry", 0)
+        e.set_option("skip_far", skip)
+        if heavy_min is not None:
+            e.set_option("heavy_min", heavy_min)
+        e.update_nl()
+        assert e.counts()["nlisted"] == 2
+    for steps, active in ((102, 0), (1, 1), (5, 1)):
+        a.step(steps)
+        b.step(steps)
+        assert b.counts()["nactive"] == active
+        assert a.counts()["nactive"] == active
+        assert_bodies_equal(a.bodies(), b.bodies())
