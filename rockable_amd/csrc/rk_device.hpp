@@ -421,7 +421,7 @@ void launch_stats(const Dev& d, double* part, double* out, hipStream_t s);
 // device, looked up once per device (0, or -1 with err set).
 constexpr int kStatScratchDoubles = 1 << 20;
 int stat_scratch(double** ptr, char* err, size_t errlen);
-// the end of a guarded step: broken bonds, a freeze, the displacement check
+// the end of a guarded step: the displacement check, a freeze
 void launch_guard(const Dev& d, const StepParams& sp, int fuse, hipStream_t s);
 // the step index the next guard check ends (the checks count on from it)
 void launch_guard_set_step(const Dev& d, long long step, hipStream_t s);

@@ -1006,7 +1006,7 @@ int run_accelerations(rk_engine* eng, int kick, int write_geom, bool guard = fal
   launch_interact(eng->d, sp, geom_all, eng->parity, eng->stream);
   toc(eng, "interact", 2);
   const bool bonds = eng->m.law == LAW_STICKED && eng->live_interfaces > 0;
-  if (bonds && !guard) {  // (a guarded step breaks its bonds at its end)
+  if (bonds && !guard) {  // (a guarded step's bonds break when the host has read the freeze)
     tic(eng, 2);
     launch_breakage(eng->d, sp, eng->stream);
     toc(eng, "breakage", 2);
@@ -1658,11 +1658,11 @@ int wait_progress(rk_engine* eng, int64_t target) {
 // the host has work (a conf file, a scheduled rebuild), after guard_batch
 // iterations (no network), or once the host has seen the check freeze the
 // steps (with a network).  When the device finds a rebuild due after
-// iteration s (the check fired the iteration before, or a bond broke in s),
+// iteration s (the check fired the iteration before, or a bond breaks in s),
 // the step kernels of the later iterations do nothing: the host reads the
 // guard at the end of the batch, keeps the loop scalars of iteration s,
-// accounts the broken interfaces, rebuilds and continues.  The schedule of
-// rebuilds is exactly the reference's.
+// breaks and accounts the marked interfaces, rebuilds and continues.  The
+// schedule of rebuilds is exactly the reference's.
 int run_guarded(rk_engine* eng, const char* outdir, int64_t nmax, bool until_tmax, int64_t* ndone) {
   Model& m = eng->m;
   int64_t done = 0;
@@ -1776,8 +1776,10 @@ int run_guarded(rk_engine* eng, const char* outdir, int64_t nmax, bool until_tma
       if (eng->note) *(volatile int32_t*)&eng->note->frozen = 0;
     }
     if (broke) {
-      // a breakage freezes the steps after its own
+      // a marked bond freezes the steps after its own; the interfaces break now
       if (!g.frozen) return fail(eng, "device guard: a bond broke without a freeze");
+      launch_breakage(eng->d, step_params(eng), eng->stream);
+      HIPCHK(hipStreamSynchronize(eng->stream));
       if (account_breakage(eng) != 0) return -1;
     }
     if (conf_at[executed] && outdir) {

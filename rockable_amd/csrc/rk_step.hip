@@ -18,9 +18,10 @@
 //               serial order of the reference, + compute_accelerations_from_
 //               resultants (3419-3552) + the closing kick (2120-2155)
 //   k_gather_heavy  the same for bodies with many slots, one workgroup each
-//   k_guard_check  the end of a guarded step: breakage_of_interfaces
-//               (3350-3413; k_breakage in steps without the guard) and the
-//               displacement check
+//   k_guard_check  the end of a guarded step: the displacement check, and the
+//               freeze after a bond was marked
+//   k_breakage  breakage_of_interfaces (3350-3413), once the host knows of a
+//               marked bond (every step without the guard)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1834,9 +1835,14 @@ __device__ int find_entry(const Dev& d, int owner, int other, uint32_t sub) {
   return -1;
 }
 
-// breakage_of_interfaces (Rockable.cpp:3350-3413) for interface k
-__device__ void break_interface(const Dev& d, int k) {
-  if (!d.ifc.brk[k]) return;
+// breakage_of_interfaces (Rockable.cpp:3350-3413), a thread per interface.  In
+// the guarded loop one launch per step that breaks a bond.  (By the one
+// workgroup of k_guard_check, 1 024 marks at a time, such a step of 226 000
+// interfaces took 2.95 ms with its rebuild, instead of 2.83.)
+__global__ void k_breakage(Dev d) {
+  if (frozen(d)) return;
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= d.ifc.n || !d.ifc.brk[k]) return;
   d.ifc.brk[k] = 0;
   if (!d.ifc.alive[k]) return;
   const uint64_t key = d.ifc.key[k];
@@ -1871,11 +1877,6 @@ __device__ void break_interface(const Dev& d, int k) {
   d.ifc.broken[atomicAdd(d.ifc.nbroken, 1)] = k;
   d.flags[0] = 1;  // needUpdate
 }
-__global__ void k_breakage(Dev d) {
-  if (frozen(d)) return;
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < d.ifc.n) break_interface(d, k);
-}
 
 // the end of a step of the integrate() loop (Rockable.cpp:2690-2740): a
 // needUpdate left by the previous check makes the rebuild due now (the step
@@ -1884,18 +1885,15 @@ __global__ void k_breakage(Dev d) {
 // on the order).  The step index lives on the device, so that a captured
 // sequence of steps replays as is.
 constexpr int kCheckBlock = 1024;
-// One launch ends the step: where the law marked a bond (flags), the interfaces
-// are broken here, and where a fused step turns out to be the last before a
-// rebuild, the passive heavy bodies are finished here (fused steps that go on
-// leave them: nothing reads their sums).  Apart, the breakage kernel and
-// k_heavy_finish took a launch each at every step, 4 to 6 us of nothing.
+// A bond that the law marked (flags) freezes the steps after this one; the host
+// then breaks the interfaces (k_breakage) before it rebuilds.  Where a fused
+// step turns out to be the last before a rebuild, the passive heavy bodies are
+// finished here (fused steps that go on leave them: nothing reads their sums).
+// A breakage kernel and k_heavy_finish at every step took a launch each, 4 to
+// 6 us of nothing.
 __global__ void __launch_bounds__(kCheckBlock) k_guard_check(Dev d, StepParams sp, int nparts, int fuse) {
   __shared__ unsigned long long red[2][kCheckBlock / 64];
   if (frozen(d)) return;
-  if (*(volatile const int*)d.flags != 0 && d.ifc.n > 0) {
-    for (int k = threadIdx.x; k < d.ifc.n; k += kCheckBlock) break_interface(d, k);
-    __syncthreads();
-  }
   if (fuse && rebuild_due(d))
     for (int h = 0; h < d.nheavy; h++) heavy_finish(d, sp, 1, 0, h);
   unsigned long long kp = 0ull, kw = ~0ull;
@@ -1939,7 +1937,7 @@ __global__ void __launch_bounds__(kCheckBlock) k_guard_check(Dev d, StepParams s
     }
   }
   // a rebuild is due after this step: the check of the step before asked
-  // for it, or an interface broke in this step (breakage_of_interfaces sets
+  // for it, or an interface breaks in this step (breakage_of_interfaces sets
   // needUpdate, Rockable.cpp:3410, and the loop rebuilds at once, 2693)
   if (rebuild_now || *(volatile const int*)d.flags != 0) {
     G->frozen = 1;

@@ -105,3 +105,27 @@ def test_broken_bond_active_set_step_by_step(tmp_path, batch):
         assert (c["nactive"], c["ninterfaces"], c["nl_updates"]) == (o.nactive, o.ninterfaces, o.nl_updates)
         seen = seen or (o.ninterfaces == 0 and o.nactive == 1)
     assert o.ninterfaces == 0 and (seen or batch > 1)
+
+
+def test_many_interfaces_bit_exact(tmp_path):
+    """2 820 interfaces, more than a workgroup has threads, under the guard:
+    the interfaces broken and what they leave equal the oracle's."""
+    from oracle.rk_oracle import Oracle
+    from rockable_amd import decks as D
+    from rockable_amd.engine import Engine
+    shapes, deck = D.bonded_clusters_deck(n_clusters=12, clearance=1e-5, strength_mean=20.0)
+    path = D.write_deck(str(tmp_path), shapes, deck)
+    e, o = Engine(path), Oracle(path, threads=8)
+    e.set_option("record_geometry", 0)
+    assert e.counts()["ninterfaces"] == o.ninterfaces == 2820
+    e.update_nl()
+    o.update_nl()
+    for n in (1000, 600):
+        e.step(n)
+        o.run_steps(n)
+        assert_bodies_equal(e.bodies(), o.bodies())
+        assert_interactions_equal(e.interactions(), o.interactions(), fields=("dn", "fn", "ft", "mom", "damp", "stick"))
+        c = e.counts()
+        assert (c["ninterfaces"], c["nl_updates"]) == (o.ninterfaces, o.nl_updates)
+        assert c["total_broken_area"] == o.total_broken_area
+    assert o.ninterfaces < 2820
