@@ -391,9 +391,9 @@ void launch_reset_list(const Dev& d, hipStream_t s);
 // the next step's predictor, unless a rebuild falls due after this one
 // (launch_drive then follows, after the check), with the global vertices
 // (GLOB_LISTED or GLOB_NONE); listed: this step took the evaluation list
-// In a fused step nothing but a freeze reads the passive heavy bodies' sums
-// (all heavy ones there): their chunks are summed only then, and launch_guard
-// finishes them.
+// Nothing reads the passive heavy bodies' sums (all heavy ones there) in a fused
+// step: neither the host, which acts only after unfused ones, nor a rebuild or
+// a later step.  They are left alone.
 struct GatherArgs {
   int kick, guard, fuse, glob, listed, par;
 };
@@ -422,7 +422,7 @@ void launch_stats(const Dev& d, double* part, double* out, hipStream_t s);
 constexpr int kStatScratchDoubles = 1 << 20;
 int stat_scratch(double** ptr, char* err, size_t errlen);
 // the end of a guarded step: the displacement check, a freeze
-void launch_guard(const Dev& d, const StepParams& sp, int fuse, hipStream_t s);
+void launch_guard(const Dev& d, int fuse, hipStream_t s);
 // the step index the next guard check ends (the checks count on from it)
 void launch_guard_set_step(const Dev& d, long long step, hipStream_t s);
 // part: (nb / 256 + 1) * 9 doubles; feat: 16 floats

@@ -1100,7 +1100,7 @@ int vv_step(rk_engine* eng, int write_geom, bool guard, bool next) {
   if (run_accelerations(eng, 1, write_geom, guard, fuse) != 0) return -1;
   if (guard) {
     tic(eng, 2);
-    launch_guard(eng->d, sp, fuse ? 1 : 0, eng->stream);
+    launch_guard(eng->d, fuse ? 1 : 0, eng->stream);
     toc(eng, "guard", 2);
   }
   if (fuse) {

@@ -1279,11 +1279,6 @@ __device__ __forceinline__ void guard_body(const Dev& d, const StepParams& sp, i
     a.kw = k2 < a.kw ? k2 : a.kw;
   }
 }
-// A rebuild falls due after the current step: the check of the step before
-// asked for it, or a bond broke in this one.
-__device__ __forceinline__ bool rebuild_due(const Dev& d) {
-  return d.guard_on && (*(volatile const int*)&d.guard->nu != 0 || *(volatile const int*)d.flags != 0);
-}
 __device__ __forceinline__ bool guard_reset(const Dev& d) { return *(volatile const int*)&d.guard->reset != 0; }
 
 // predict_free: the new pose and velocities of free body b (Rockable.cpp:
@@ -1513,7 +1508,7 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
   ga.kp = 0ull;
   ga.kw = ~0ull;
   // (gather_blocks sizes the grid by the same rule)
-  const int nchunk = A.fuse && !d.guard_on ? 0 : (d.nhch + T / 64 - 1) / (T / 64);
+  const int nchunk = A.fuse ? 0 : (d.nhch + T / 64 - 1) / (T / 64);
   const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
   const bool driven = tile < d.nDriven, chunks = !driven && tile < d.nDriven + nchunk;
   const int b0 = driven ? tile : d.nDriven + (tile - d.nDriven - nchunk) * NB;
@@ -1521,7 +1516,7 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
   int k0 = 0, kend = 0;
   if (chunks) {
     const int c = (tile - d.nDriven) * (T / 64) + wv;
-    if (c < d.nhch && !predict) {
+    if (c < d.nhch) {
       const int2 r = d.hch[c];
       const double s = sum_chunk(d, r.x, r.y, lane, vals + 64 * 6 * wv);
       if (lane < 6) d.hpart[6 * (size_t)c + lane] = s;
@@ -1717,14 +1712,15 @@ __device__ __forceinline__ void guard_heavy(const Dev& d, const StepParams& sp, 
   if (a.kw != ~0ull) atomicMin(&d.guard->minw, a.kw);
 }
 
-static_assert(kBlock == 256, "heavy_finish combines four wavefronts");
-// heavy body h, by the first 256 threads of a workgroup (every thread calls it)
-__device__ __forceinline__ void heavy_finish(const Dev& d, const StepParams& sp, int kick, int guard, int h) {
+static_assert(kBlock == 256, "k_heavy_finish combines four wavefronts");
+__global__ void __launch_bounds__(kBlock) k_heavy_finish(Dev d, StepParams sp, int kick, int guard) {
   __shared__ double red[kBlock / 64][6];
+  if (frozen(d)) return;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int b = d.heavy[h];
-  if (!d.passive[b] || d.exact_sums) return;  // the same for the whole workgroup
-  if (t < kBlock) {
+  for (TileLoop T = xcd_tiles(d.nheavy); T.t < T.end; T.t += T.step) {
+    const int h = T.t;
+    const int b = d.heavy[h];
+    if (!d.passive[b] || d.exact_sums) continue;  // the same for the whole workgroup
     double a[6] = {-0.0, -0.0, -0.0, -0.0, -0.0, -0.0};
     for (int c = d.hch_off[h] + t; c < d.hch_off[h + 1]; c += kBlock) {
       const double* p = d.hpart + 6 * (size_t)c;
@@ -1738,26 +1734,21 @@ __device__ __forceinline__ void heavy_finish(const Dev& d, const StepParams& sp,
     if (lane == 0)
 #pragma unroll
       for (int q = 0; q < 6; q++) red[wv][q] = a[q];
-  }
-  __syncthreads();
-  if (t == 0) {
-    double a[6];
+    __syncthreads();
+    if (t == 0) {
 #pragma unroll
-    for (int q = 0; q < 6; q++) a[q] = (red[0][q] + red[1][q]) + (red[2][q] + red[3][q]);
-    BodyKin P = d.kin[b];
-    const bool driven = b < d.nDriven;
-    v3 F, M;
-    int c0, c1;
-    init_resultants(d, b, P, driven, F, M, c0, c1);
-    finish_body(d, sp, kick, b, P, driven, vadd(F, V(a[0], a[1], a[2])), vadd(M, V(a[3], a[4], a[5])), c0, c1,
-                d.mass[b], ld3(d.inertia + 3 * (size_t)b));
-    if (guard) guard_heavy(d, sp, b, P);
+      for (int q = 0; q < 6; q++) a[q] = (red[0][q] + red[1][q]) + (red[2][q] + red[3][q]);
+      BodyKin P = d.kin[b];
+      const bool driven = b < d.nDriven;
+      v3 F, M;
+      int c0, c1;
+      init_resultants(d, b, P, driven, F, M, c0, c1);
+      finish_body(d, sp, kick, b, P, driven, vadd(F, V(a[0], a[1], a[2])), vadd(M, V(a[3], a[4], a[5])), c0, c1,
+                  d.mass[b], ld3(d.inertia + 3 * (size_t)b));
+      if (guard) guard_heavy(d, sp, b, P);
+    }
+    __syncthreads();
   }
-  __syncthreads();
-}
-__global__ void __launch_bounds__(kBlock) k_heavy_finish(Dev d, StepParams sp, int kick, int guard) {
-  if (frozen(d)) return;
-  for (TileLoop T = xcd_tiles(d.nheavy); T.t < T.end; T.t += T.step) heavy_finish(d, sp, kick, guard, T.t);
 }
 
 // compute_resultants for a heavy body that is not passive (or any heavy
@@ -1886,16 +1877,11 @@ __global__ void k_breakage(Dev d) {
 // sequence of steps replays as is.
 constexpr int kCheckBlock = 1024;
 // A bond that the law marked (flags) freezes the steps after this one; the host
-// then breaks the interfaces (k_breakage) before it rebuilds.  Where a fused
-// step turns out to be the last before a rebuild, the passive heavy bodies are
-// finished here (fused steps that go on leave them: nothing reads their sums).
-// A breakage kernel and k_heavy_finish at every step took a launch each, 4 to
-// 6 us of nothing.
-__global__ void __launch_bounds__(kCheckBlock) k_guard_check(Dev d, StepParams sp, int nparts, int fuse) {
+// then breaks the interfaces (k_breakage) before it rebuilds.  A launch of that
+// at every step took 4 us for nothing.
+__global__ void __launch_bounds__(kCheckBlock) k_guard_check(Dev d, int nparts) {
   __shared__ unsigned long long red[2][kCheckBlock / 64];
   if (frozen(d)) return;
-  if (fuse && rebuild_due(d))
-    for (int h = 0; h < d.nheavy; h++) heavy_finish(d, sp, 1, 0, h);
   unsigned long long kp = 0ull, kw = ~0ull;
   for (int k = threadIdx.x; k < nparts; k += kCheckBlock) {
     const unsigned long long p = d.gpart[2 * (size_t)k], w = d.gpart[2 * (size_t)k + 1];
@@ -2728,7 +2714,7 @@ int gather_threads(const Dev& d) {
 // wavefront, the free bodies
 int gather_blocks(const Dev& d, int fuse) {
   const int nb = gather_bodies(d), wv = gather_threads(d) / 64;
-  return d.nDriven + (fuse && !d.guard_on ? 0 : (d.nhch + wv - 1) / wv) + (d.nb - d.nDriven + nb - 1) / nb;
+  return d.nDriven + (fuse ? 0 : (d.nhch + wv - 1) / wv) + (d.nb - d.nDriven + nb - 1) / nb;
 }
 
 int gather_blocks_max(int nb, int nhch) { return nb + (nhch + 1) / 2 + 8; }
@@ -2910,9 +2896,9 @@ __global__ void k_guard_set_step(Dev d, long long step) {
   if (threadIdx.x == 0) d.guard->step = step;
 }
 
-void launch_guard(const Dev& d, const StepParams& sp, int fuse, hipStream_t s) {
+void launch_guard(const Dev& d, int fuse, hipStream_t s) {
   const int nparts = (d.disp_check && d.nb > 0) ? gather_blocks(d, fuse) : 0;
-  hipLaunchKernelGGL(k_guard_check, dim3(1), dim3(kCheckBlock), 0, s, d, sp, nparts, fuse);
+  hipLaunchKernelGGL(k_guard_check, dim3(1), dim3(kCheckBlock), 0, s, d, nparts);
 }
 
 void launch_guard_set_step(const Dev& d, long long step, hipStream_t s) {

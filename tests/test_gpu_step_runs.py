@@ -46,3 +46,30 @@ def test_run_equals_single_steps(tmp_path, name, record):
         assert a.counts()["nl_updates"] == b.counts()["nl_updates"]
     assert_interactions_equal(a.interactions(), b.interactions(), fields=("dn", "fn", "ft", "mom", "damp", "stick"))
     assert_bodies_equal(a.bodies(), b.bodies())
+
+
+def test_heavy_walls_under_the_guard(tmp_path):
+    """A floor and walls with more slots than heavy_min, left alone by the steps
+    that go on, under a displacement check that freezes the steps inside
+    most batches: at every read-out their resultants are those of a run of
+    single steps, and the rebuild steps are the same."""
+    from rockable_amd.engine import Engine
+    shapes, deck = D.sphere_lattice_deck(dims=(24, 20, 2), spacing_factor=2.002, seed=6, vmax=0.05, nl="linkCells")
+    deck.gravity = (30.0, -20.0, -400.0)
+    deck.interVerlet = 1e3
+    deck.dynamic_update_nl = 1
+    deck.disp_update_nl, deck.angle_update_nl = 5e-7, 57.0
+    path = D.write_deck(str(tmp_path), shapes, deck)
+    a, b = Engine(path), Engine(path)
+    for e in (a, b):
+        e.set_option("record_geometry", 0)
+        e.set_option("heavy_min", 20)
+        e.update_nl()
+    for n in (1, 90, 161):
+        a.step(n)
+        for _ in range(n):
+            b.step(1)
+        assert a.counts()["nl_updates"] == b.counts()["nl_updates"]
+        assert_bodies_equal(a.bodies(), b.bodies())
+    assert a.counts()["nl_updates"] > 10
+    assert abs(a.bodies()["force"][0, 2]) > 0.0
