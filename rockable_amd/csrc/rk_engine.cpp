@@ -1200,12 +1200,18 @@ int step_graph(rk_engine* eng, int n, bool with_guard, hipGraphExec_t* out) {
 // Launch the deferred steps: whole runs of graph_steps as captured graphs,
 // the rest one by one.  Every host action that reads or changes the device
 // state (rebuild, conf file, guard read, counts) comes after a flush.
-int flush_steps(rk_engine* eng) {
+// more: another step follows with no host action in between, so that the last
+// one may take its predictor.
+int flush_steps(rk_engine* eng, bool more = false) {
   int64_t n = eng->pending;
   const bool with_guard = eng->pending_guard;
   eng->pending = 0;
   const int G = eng->graph_steps;
   if (G > 1 && n >= G && eng->profile == 0) {
+    if (eng->predicted) {  // a graph starts with a predictor of its own
+      if (launch_one_step(eng, with_guard, false) != 0) return -1;
+      n--;
+    }
     for (; n >= G; n -= G) {
       hipGraphExec_t exec = nullptr;
       if (step_graph(eng, G, with_guard, &exec) != 0) return -1;  // (the step's parity is part of its key)
@@ -1217,7 +1223,7 @@ int flush_steps(rk_engine* eng) {
     eng->gv_state = uses_list(eng->d, eng->record_geometry) ? rk_engine::GV_STALE : rk_engine::GV_LISTED;
   }
   for (; n > 0; n--)
-    if (launch_one_step(eng, with_guard, n > 1) != 0) return -1;
+    if (launch_one_step(eng, with_guard, n > 1 || more) != 0) return -1;
   return 0;
 }
 
@@ -1636,9 +1642,13 @@ int propose_batch(rk_engine* eng) {
 // Waits until the device has completed target steps (the check's progress
 // word) or frozen the steps; 1 if frozen, 0 if not, -1 on an error.  The
 // deferred steps are launched first; a drained stream ends the wait (the
-// words are then final).
+// words are then final).  Another step follows unless the steps are frozen, so
+// the flushed ones stay fused: with the device behind, a wait falls after
+// nearly every step, and without this every step of a paced loop on captured
+// steps took a predictor of its own (30 001 bodies, graph_steps 32: 48.6 us
+// per step, with it 35.1; 34.0 without graphs).
 int wait_progress(rk_engine* eng, int64_t target) {
-  if (flush_steps(eng) != 0) return -1;
+  if (flush_steps(eng, true) != 0) return -1;
   const volatile HostNote* n = eng->note;
   for (unsigned spin = 0;; spin++) {
     if (n->frozen) return 1;

@@ -93,3 +93,39 @@ def test_graph_steps_integrate_conf_files(tmp_path):
     for f in files:
         ok, k, x, y = compare_conf(str(outs[1] / os.path.basename(f)), f)
         assert ok, "%s differs at line %s" % (os.path.basename(f), k)
+
+
+@pytest.mark.parametrize("graph_steps", [3, 8])
+def test_paced_steps_stay_fused(tmp_path, graph_steps):
+    """With the network the host waits after nearly every step, and each wait
+    launches what is deferred: these steps still take the next one's predictor
+    with the resultants.  Only the steps that start after a freeze, a read-out or
+    a captured run have one of their own.  On the evaluation list, also with
+    captured runs of an odd length (one per parity of the step)."""
+    from rockable_amd import decks as D
+    from rockable_amd.engine import Mlp
+    shapes, deck = D.sphere_lattice_deck(dims=(24, 20, 4), spacing_factor=2.002, seed=6, vmax=0.05, nl="linkCells")
+    deck.gravity = (30.0, -20.0, -400.0)
+    deck.interVerlet = 1e3
+    deck.dynamic_update_nl = 1
+    deck.disp_update_nl, deck.angle_update_nl = 1e-5, 57.0
+    path = D.write_deck(str(tmp_path), shapes, deck)
+    mlps = [Mlp(seed=1), Mlp(seed=1)]
+    W = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "rockable_amd", "data",
+                     "rebuild_mlp.npy")
+
+    def setup(e):
+        mlps[-1].set_params(np.load(W))
+        e.set_option("record_geometry", 0)
+        e.set_rebuild_model(mlps.pop())
+    a, b = _pair(path, (200, 301), graph_steps, setup=setup)
+    assert b.counts()["graph_launches"] > 0
+    b.set_option("profile", 2)
+    b.reset_kernel_time()
+    before = b.counts()
+    a.step(400)
+    b.step(400)
+    own = b.kernel_time("predict")[0]
+    assert own <= b.counts()["guard_reads"] - before["guard_reads"]
+    assert_bodies_equal(b.bodies(), a.bodies())
+    assert b.counts()["nl_updates"] == a.counts()["nl_updates"] > before["nl_updates"]
