@@ -1347,9 +1347,10 @@ __device__ __forceinline__ void driven_bound(const Dev& d, const StepParams& sp,
   const double step = sqrt(ux * ux + uy * uy + uz * uz);
   set_bound(d, b, cb + (step + 1e-15), step, limit, par);
 }
-// all of them by one workgroup, in a predictor's launch
+// all of them, spread over a predictor's launch
 __device__ __forceinline__ void driven_bounds(const Dev& d, const StepParams& sp, int par) {
-  for (int b = threadIdx.x; b < d.nDriven; b += blockDim.x) driven_bound(d, sp, b, true, false, par);
+  for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < d.nDriven; b += gridDim.x * blockDim.x)
+    driven_bound(d, sp, b, true, false, par);
 }
 __device__ __forceinline__ void add_motion_bound(const Dev& d, const StepParams& sp, int b, const BodyKin& old,
                                                  const BodyKin& P, int par) {
@@ -1429,8 +1430,8 @@ __device__ __forceinline__ unsigned byte_bits(unsigned x) { return ((x & 0x01010
 // uses, are not stored.  Apart, the two kernels took 14.8 + 11.3 us for
 // 50 005 bodies, fused 22.4 us; 6.6 + 7.5 and 8.7 us for 706 bodies, where a
 // launch counts most.
-// Driven bodies come first, one workgroup each (a wall's many slots fill it);
-// then, a wavefront each, the 64-slot chunks of the heavy bodies, whose
+// Driven bodies come first, one workgroup each (a wall's many slots fill it),
+// or with MANY driven_per of them (below); then, a wavefront each, the 64-slot chunks of the heavy bodies, whose
 // partial sums (from -0.0, the identity of addition) k_heavy_finish takes.
 // Bodies with more than heavy_min slots are left to the heavy kernels.  With
 // guard, the displacement check accumulates each finished body and every
@@ -1464,7 +1465,20 @@ __device__ __forceinline__ double sum_chunk(const Dev& d, int k0, int k1, int la
   return s;
 }
 
-template <int T, int NB, bool BF>  // T threads; BF: the deck has a body force
+// Driven bodies per workgroup: one up to 2 047 of them, whose workgroups are
+// resident at once with many others'; beyond (a bed of glued grains) as
+// many as leave 1 024 to 2 047 workgroups, at most 32.  A step of 40 005 spheres,
+// 10 005 of them driven, took 70.6 us with a workgroup each and the driven
+// bodies' bounds moved by one workgroup, 27.0 us so; 171 and 51 us for 160 005
+// spheres, 40 005 of them driven.
+constexpr int kDrivenMany = 2048;
+__host__ __device__ __forceinline__ int driven_per(int nDriven) {
+  const int n = nDriven / 1024;
+  return n < 1 ? 1 : n > 32 ? 32 : n;
+}
+
+// T threads; BF: the deck has a body force; MANY: kDrivenMany driven bodies or more
+template <int T, int NB, bool BF, bool MANY>
 __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArgs A) {
   constexpr int kLanes = T / NB;  // lanes per body in the sums (8, 4 or 2)
   constexpr int kComp = kLanes >= 6 ? 1 : kLanes >= 3 ? 2 : 3;  // components per lane
@@ -1477,6 +1491,7 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
   __shared__ unsigned short act[T];
   __shared__ int wsum[T / 64];
   __shared__ double fm[NB][6];
+  __shared__ unsigned long long heavy;  // MANY: bit k: body b0 + k is left to the heavy kernels
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int kick = A.kick, guard = A.guard;
   // every control word in one round of loads
@@ -1510,12 +1525,13 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
   // (gather_blocks sizes the grid by the same rule)
   const int nchunk = A.fuse ? 0 : (d.nhch + T / 64 - 1) / (T / 64);
   const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
-  const bool driven = tile < d.nDriven, chunks = !driven && tile < d.nDriven + nchunk;
-  const int b0 = driven ? tile : d.nDriven + (tile - d.nDriven - nchunk) * NB;
-  const int nbk = driven ? 1 : min(NB, d.nb - b0);
+  const int per = MANY ? driven_per(d.nDriven) : 1, ndt = MANY ? (d.nDriven + per - 1) / per : d.nDriven;
+  const bool driven = tile < ndt, chunks = !driven && tile < ndt + nchunk;
+  const int b0 = driven ? tile * per : d.nDriven + (tile - ndt - nchunk) * NB;
+  const int nbk = driven ? min(per, d.nDriven - b0) : min(NB, d.nb - b0);
   int k0 = 0, kend = 0;
   if (chunks) {
-    const int c = (tile - d.nDriven) * (T / 64) + wv;
+    const int c = (tile - ndt) * (T / 64) + wv;
     if (c < d.nhch) {
       const int2 r = d.hch[c];
       const double s = sum_chunk(d, r.x, r.y, lane, vals + 64 * 6 * wv);
@@ -1525,9 +1541,9 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
     k0 = d.soff[b0];
     kend = d.soff[b0 + nbk];
   }
-  // (a driven body has a workgroup of its own, also where it is heavy)
-  if (driven && t == 0 && (predict || relisted)) driven_bound(d, sp, b0, predict, relisted, 1 - A.par);
-  if (chunks || (driven && kend - k0 > d.heavy_min)) {  // no body to finish
+  // (also of the heavy ones)
+  if (driven && t < nbk && (predict || relisted)) driven_bound(d, sp, b0 + t, predict, relisted, 1 - A.par);
+  if (chunks || (driven && nbk == 1 && kend - k0 > d.heavy_min)) {  // no body to finish
     if (guard && t == 0) {
       if (A.fuse && !chunks) guard_body(d, sp, b0, d.kin[b0], rst, ga);  // (else k_heavy_finish does)
       d.gpart[2 * (size_t)blockIdx.x] = ga.kp;
@@ -1558,6 +1574,11 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
     }
     if (relisted && !driven) d.climit[b] = d.ahead[b];
   }
+  static_assert(NB <= 64, "the first wavefront's threads have a body each");
+  if (MANY) {
+    const unsigned long long h = __ballot(t < nbk && !run);
+    if (t == 0) heavy = h;
+  }
   // the summing lanes' bodies and slot ranges
   const int lb = t / kLanes, lc = t % kLanes;
   const bool sums = lb < nbk && lc * kComp < 6;
@@ -1576,14 +1597,25 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
   }
   double s[kComp];
   bool first = true;
-  for (int w0 = k0 & ~15; w0 < kend; w0 += kWin) {
+  // MANY leaves a heavy body's slots (a wall's among glued grains) out: [ka, kb)
+  // are those up to the next one
+  unsigned long long skip = MANY ? heavy : 0ull;
+  int ka = k0, kb = MANY && skip ? d.soff[b0 + __ffsll(skip) - 1] : kend;
+  for (int w0 = ka & ~15;; w0 += kWin) {
+    while (MANY && skip && w0 >= kb) {
+      ka = d.soff[b0 + __ffsll(skip)];
+      skip &= skip - 1ull;
+      kb = skip ? d.soff[b0 + __ffsll(skip) - 1] : kend;
+      w0 = ka & ~15;
+    }
+    if (w0 >= kb) break;
     const int pos = w0 + 16 * t;
     unsigned m = 0u;
-    if (pos < kend) {
+    if (pos < kb) {
       const uint4 x = *reinterpret_cast<const uint4*>(d.sact + pos);
       m = byte_bits(x.x) | byte_bits(x.y) << 4 | byte_bits(x.z) << 8 | byte_bits(x.w) << 12;
-      if (pos < k0) m &= 0xffffu << (k0 - pos);
-      if (pos + 16 > kend) m &= 0xffffu >> (pos + 16 - kend);
+      if (pos < ka) m &= 0xffffu << (ka - pos);
+      if (pos + 16 > kb) m &= 0xffffu >> (pos + 16 - kb);
     }
     int incl = __popc(m);
     const int mine = incl;
@@ -1669,6 +1701,8 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
       store_resultants(d, b, F, M, acc, arot);
     }
     if (kick) rec_store_motion(rec + t * kRec, P);
+  } else if (MANY && t < nbk && guard && A.fuse) {  // (in other steps k_heavy_finish does it)
+    guard_body(d, sp, b, rec_load(rec + t * kRec), rst, ga);
   }
   __syncthreads();
   if (kick)
@@ -1685,7 +1719,6 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
     }
   if (!guard) return;
   // only the threads t < NB (the first wavefront) finish bodies
-  static_assert(NB <= 64, "the first wavefront finishes the bodies");
   for (int off = 32; off > 0; off >>= 1) {
     const unsigned long long op = __shfl_xor(ga.kp, off, 64), ow = __shfl_xor(ga.kw, off, 64);
     ga.kp = op > ga.kp ? op : ga.kp;
@@ -2260,10 +2293,8 @@ __global__ void __launch_bounds__(kBlock) k_drive(Dev d, StepParams sp, int driv
 __global__ void __launch_bounds__(kBlock) k_predict(Dev d, StepParams sp, int glob, int par) {
   if (frozen(d)) return;
   const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  if (blockIdx.x == 0) {
-    drive_controls_block(d, sp);
-    driven_bounds(d, sp, par);
-  }
+  if (blockIdx.x == 0) drive_controls_block(d, sp);
+  driven_bounds(d, sp, par);
   // free bodies (Rockable.cpp:2036-2055), a grid-stride loop
   for (int b = gid; b < d.nb; b += gridDim.x * blockDim.x) {
     if (b < d.nDriven) continue;
@@ -2295,9 +2326,9 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
   __shared__ int shp[64];           // shape, or -1 if the body is not listed
   if (frozen(d)) return;
   const int t = threadIdx.x;
+  driven_bounds(d, sp, par);
   if (blockIdx.x == 0) {
     drive_controls_block(d, sp);
-    driven_bounds(d, sp, par);
     if (driven_glob) {
       __syncthreads();  // the driven poses, written by thread 0, are visible to the workgroup
       for (int k = t; k < d.nvdriven; k += blockDim.x) {
@@ -2386,10 +2417,8 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
 // k_glob after it.
 __global__ void __launch_bounds__(kBlock) k_predict_vtx(Dev d, StepParams sp, int par) {
   if (frozen(d)) return;
-  if (blockIdx.x == 0) {
-    drive_controls_block(d, sp);
-    driven_bounds(d, sp, par);
-  }
+  if (blockIdx.x == 0) drive_controls_block(d, sp);
+  driven_bounds(d, sp, par);
   const int lane = threadIdx.x & 63;
   for (int wv = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6); wv < d.nwv;
        wv += (int)((gridDim.x * blockDim.x) >> 6)) {
@@ -2695,7 +2724,8 @@ void launch_interact(const Dev& d, const StepParams& sp, int write_geom_all, int
 // from 131 072 bodies, where workgroups abound and the lanes that finish
 // the bodies count.
 constexpr int kGatherLarge = 1 << 17;
-int gather_bodies(const Dev& d) { return d.nb - d.nDriven >= kGatherLarge ? 64 : 32; }
+bool gather_many(const Dev& d) { return d.nDriven >= kDrivenMany; }
+int gather_bodies(const Dev& d) { return !gather_many(d) && d.nb - d.nDriven >= kGatherLarge ? 64 : 32; }
 
 // and its threads: 256 where all workgroups are resident at once anyway (up to
 // 1024 of them) or bodies have many slots, whose terms then take fewer passes;
@@ -2705,16 +2735,17 @@ int gather_bodies(const Dev& d) { return d.nb - d.nDriven >= kGatherLarge ? 64 :
 // for 706 hulls, but 28.7 and 22.7 us for the 90 006-body slope, 12.3 and 9.2
 // us for 47 000 spheres.
 int gather_threads(const Dev& d) {
-  if (gather_bodies(d) == 64) return 128;
+  if (gather_bodies(d) == 64 || gather_many(d)) return 128;
   const bool few = (d.nb - d.nDriven + 31) / 32 <= 1024, many_slots = 2.0 * d.ne > 56.0 * d.nb;
   return few || many_slots ? 256 : 128;
 }
 
-// k_gather's workgroups: one per driven body, the heavy chunks one to a
+// k_gather's workgroups: the driven bodies, the heavy chunks one to a
 // wavefront, the free bodies
 int gather_blocks(const Dev& d, int fuse) {
   const int nb = gather_bodies(d), wv = gather_threads(d) / 64;
-  return d.nDriven + (fuse ? 0 : (d.nhch + wv - 1) / wv) + (d.nb - d.nDriven + nb - 1) / nb;
+  const int per = gather_many(d) ? driven_per(d.nDriven) : 1;
+  return (d.nDriven + per - 1) / per + (fuse ? 0 : (d.nhch + wv - 1) / wv) + (d.nb - d.nDriven + nb - 1) / nb;
 }
 
 int gather_blocks_max(int nb, int nhch) { return nb + (nhch + 1) / 2 + 8; }
@@ -2725,18 +2756,22 @@ void launch_gather(const Dev& d, const StepParams& sp, GatherArgs A, hipStream_t
   const int kick = A.kick, guard = A.guard;
   const dim3 blocks(gather_blocks(d, A.fuse));
   const bool bf = d.bf != BF_NONE, large = gather_bodies(d) == 64, wide = gather_threads(d) == 256;
-  if (large && bf)
-    hipLaunchKernelGGL((k_gather<128, 64, true>), blocks, dim3(128), 0, s, d, sp, A);
+  if (gather_many(d) && bf)
+    hipLaunchKernelGGL((k_gather<128, 32, true, true>), blocks, dim3(128), 0, s, d, sp, A);
+  else if (gather_many(d))
+    hipLaunchKernelGGL((k_gather<128, 32, false, true>), blocks, dim3(128), 0, s, d, sp, A);
+  else if (large && bf)
+    hipLaunchKernelGGL((k_gather<128, 64, true, false>), blocks, dim3(128), 0, s, d, sp, A);
   else if (large)
-    hipLaunchKernelGGL((k_gather<128, 64, false>), blocks, dim3(128), 0, s, d, sp, A);
+    hipLaunchKernelGGL((k_gather<128, 64, false, false>), blocks, dim3(128), 0, s, d, sp, A);
   else if (wide && bf)
-    hipLaunchKernelGGL((k_gather<256, 32, true>), blocks, dim3(256), 0, s, d, sp, A);
+    hipLaunchKernelGGL((k_gather<256, 32, true, false>), blocks, dim3(256), 0, s, d, sp, A);
   else if (wide)
-    hipLaunchKernelGGL((k_gather<256, 32, false>), blocks, dim3(256), 0, s, d, sp, A);
+    hipLaunchKernelGGL((k_gather<256, 32, false, false>), blocks, dim3(256), 0, s, d, sp, A);
   else if (bf)
-    hipLaunchKernelGGL((k_gather<128, 32, true>), blocks, dim3(128), 0, s, d, sp, A);
+    hipLaunchKernelGGL((k_gather<128, 32, true, false>), blocks, dim3(128), 0, s, d, sp, A);
   else
-    hipLaunchKernelGGL((k_gather<128, 32, false>), blocks, dim3(128), 0, s, d, sp, A);
+    hipLaunchKernelGGL((k_gather<128, 32, false, false>), blocks, dim3(128), 0, s, d, sp, A);
   if (d.nheavy > 0 && !A.fuse) {
     hipLaunchKernelGGL(k_heavy_finish, grid_for(d, d.nheavy), dim3(kBlock), 0, s, d, sp, kick, guard);
     if (d.nheavy_exact > 0)
