@@ -1314,48 +1314,47 @@ __device__ __forceinline__ void predict_free(const Dev& d, const StepParams& sp,
 // |Q' v Q'* - Q v Q*| <= 2 |Q' - Q| |v|), plus a rounding allowance.
 // It also sets the allowance ahead of it (24 steps of this motion, at least
 // ahead_min) and asks for a new evaluation list when the bound passes limit,
-// what the list in use was written for (a NaN does too).
+// what the list in use was written for (a NaN does too).  Not where the next
+// step takes no list (par -1): the bound stays past the limit and the
+// predictor of the first step that takes one asks.
 constexpr double kAheadSteps = 24.0;
 __device__ __forceinline__ void set_bound(const Dev& d, int b, double bound, double step, double limit, int par) {
   d.cbound[b] = bound;
   d.ahead[b] = bound + fmax(kAheadSteps * step, d.ahead_min);
-  if (!(bound <= limit)) d.ls->want[par] = 1;
+  if (par >= 0 && !(bound <= limit)) d.ls->want[par] = 1;
 }
 __device__ __forceinline__ void add_motion_bound_with(const Dev& d, const StepParams& sp, int b, const BodyKin& old,
-                                                      const BodyKin& P, double cb, double rmax, double limit, int par) {
+                                                      const BodyKin& P, double cb, double rmax, double limit,
+                                                      v3 drift, int par) {
   if (!d.skip_far) return;
-  const double dx = P.px - old.px - sp.dt * d.drift[0], dy = P.py - old.py - sp.dt * d.drift[1],
-               dz = P.pz - old.pz - sp.dt * d.drift[2];
+  const double dx = P.px - old.px - sp.dt * drift.x, dy = P.py - old.py - sp.dt * drift.y,
+               dz = P.pz - old.pz - sp.dt * drift.z;
   const double qw = P.qw - old.qw, qx = P.qx - old.qx, qy = P.qy - old.qy, qz = P.qz - old.qz;
   const double step = sqrt(dx * dx + dy * dy + dz * dz) + 2.0 * sqrt(qw * qw + qx * qx + qy * qy + qz * qz) * rmax;
   const double mag = fabs(P.px) + fabs(P.py) + fabs(P.pz);
   set_bound(d, b, cb + (step + 1e-15 * (1.0 + mag)), step, limit, par);
 }
-// The bound of driven body b, by one thread: without a control it stays where
-// it is, which in the moving frame is a motion of |D|.  predict: the step is
-// taken now; relisted: the list in use was written in this step, for the
-// allowance before it.  A body's limit and allowance have no other writer
-// in the launch, so that the limit is the allowance the list was written for.
-__device__ __forceinline__ void driven_bound(const Dev& d, const StepParams& sp, int b, bool predict, bool relisted,
+// The bound of driven body b, from cb: without a control it stays where it is,
+// which in the moving frame is a motion of |D|.  One thread of a launch
+// writes a body's limit, bound and allowance, so that the limit is the
+// allowance the list was written for.
+__device__ __forceinline__ void driven_bound(const Dev& d, const StepParams& sp, int b, double cb, double limit, v3 drift,
                                              int par) {
-  if (!d.skip_far) return;
-  const double limit = relisted ? d.ahead[b] : d.climit[b];
-  if (relisted) d.climit[b] = limit;
-  const double cb = d.cbound[b];
-  if (!predict || !(cb < INFINITY)) return;
-  const double ux = sp.dt * d.drift[0], uy = sp.dt * d.drift[1], uz = sp.dt * d.drift[2];
+  if (!(cb < INFINITY)) return;
+  const double ux = sp.dt * drift.x, uy = sp.dt * drift.y, uz = sp.dt * drift.z;
   const double step = sqrt(ux * ux + uy * uy + uz * uz);
   set_bound(d, b, cb + (step + 1e-15), step, limit, par);
 }
-// all of them, spread over a predictor's launch
-__device__ __forceinline__ void driven_bounds(const Dev& d, const StepParams& sp, int par) {
-  for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < d.nDriven; b += gridDim.x * blockDim.x)
-    driven_bound(d, sp, b, true, false, par);
+// all of them, spread over a predictor's threads (thread `first` of `stride`)
+__device__ __forceinline__ void driven_bounds(const Dev& d, const StepParams& sp, int first, int stride, int par) {
+  if (!d.skip_far) return;
+  for (int b = first; b < d.nDriven; b += stride)
+    driven_bound(d, sp, b, d.cbound[b], d.climit[b], ld3(d.drift), par);
 }
 __device__ __forceinline__ void add_motion_bound(const Dev& d, const StepParams& sp, int b, const BodyKin& old,
                                                  const BodyKin& P, int par) {
   if (!d.skip_far) return;
-  add_motion_bound_with(d, sp, b, old, P, d.cbound[b], d.rmax[b], d.climit[b], par);
+  add_motion_bound_with(d, sp, b, old, P, d.cbound[b], d.rmax[b], d.climit[b], ld3(d.drift), par);
 }
 
 typedef double d2 __attribute__((ext_vector_type(2)));  // one 16-byte access
@@ -1494,7 +1493,16 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
   __shared__ unsigned long long heavy;  // MANY: bit k: body b0 + k is left to the heavy kernels
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int kick = A.kick, guard = A.guard;
-  // every control word in one round of loads
+  // (gather_blocks sizes the grid by the same rule)
+  const int nchunk = A.fuse ? 0 : (d.nhch + T / 64 - 1) / (T / 64);
+  const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
+  const int per = MANY ? driven_per(d.nDriven) : 1, ndt = MANY ? (d.nDriven + per - 1) / per : d.nDriven;
+  const bool driven = tile < ndt, chunks = !driven && tile < ndt + nchunk;
+  const int b0 = driven ? tile * per : d.nDriven + (tile - ndt - nchunk) * NB;
+  const int nbk = chunks ? 0 : driven ? min(per, d.nDriven - b0) : min(NB, d.nb - b0);
+  // one round of loads: the control words, the slot ranges, the records and
+  // what finishing a body needs (in turn they took two latencies more: 7.5 us
+  // for 517 spheres, 17.2 us for 50 005 hulls; so 6.6 and 16.5 us)
   int stop = 0, due = 0, again = 0;
   if (d.guard_on) {
     const volatile DevGuard* G = d.guard;
@@ -1504,12 +1512,42 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
     again = re;
   }
   const int want = *(volatile const int*)&d.ls->want[A.par];
+  constexpr int kLoads = (8 * NB + T - 1) / T;
+  static_assert(NB <= 64, "the first wavefront's threads have a body each");
+  d2* kd = reinterpret_cast<d2*>(d.kin + b0);
+  d2 x[kLoads];
+#pragma unroll
+  for (int r = 0; r < kLoads; r++)
+    if (t + r * T < 8 * nbk) x[r] = kd[t + r * T];
+  const int k0 = chunks ? 0 : d.soff[b0], kend = chunks ? 0 : d.soff[b0 + nbk];
+  const int b = b0 + t;
+  double mb = 1.0, cb = 0.0, rmx = 0.0, lim = 0.0, ah = 0.0;
+  v3 Ib = V(1.0, 1.0, 1.0), drift = V(0.0, 0.0, 0.0);
+  bool run = false;
+  if (t < nbk) {
+    mb = d.mass[b];
+    Ib = ld3(d.inertia + 3 * (size_t)b);
+    run = d.soff[b + 1] - d.soff[b] <= d.heavy_min;
+    if (d.skip_far) {
+      cb = d.cbound[b];
+      rmx = d.rmax[b];
+      lim = d.climit[b];
+      ah = d.ahead[b];
+      drift = ld3(d.drift);
+    }
+  }
+  // the summing lanes' bodies and slot ranges
+  const int lb = t / kLanes, lc = t % kLanes;
+  const bool sums = lb < nbk && lc * kComp < 6;
+  const int sb0 = sums ? d.soff[b0 + lb] : 0, sb1 = sums ? d.soff[b0 + lb + 1] : 0;
   if (stop) return;
   const bool rst = guard && again;
   // (the check that follows this step freezes the later ones on the same words)
   const bool predict = A.fuse && !due;
-  // this step's force phase wrote a new evaluation list
+  // this step's force phase wrote a new evaluation list, for the allowances
   const bool relisted = A.listed && want != 0;
+  const int npar = A.listed ? 1 - A.par : -1;  // (a run's steps all take the list, or none but its last does)
+  if (relisted) lim = ah;
   if (relisted && blockIdx.x == 0 && t == 0) {
     const int g = d.ls->gen + 1;
     for (int k = 0; k < 8; k++) d.ls->cnt[(g + 1) & 1][k] = 0;
@@ -1522,14 +1560,6 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
   GuardAcc ga;
   ga.kp = 0ull;
   ga.kw = ~0ull;
-  // (gather_blocks sizes the grid by the same rule)
-  const int nchunk = A.fuse ? 0 : (d.nhch + T / 64 - 1) / (T / 64);
-  const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
-  const int per = MANY ? driven_per(d.nDriven) : 1, ndt = MANY ? (d.nDriven + per - 1) / per : d.nDriven;
-  const bool driven = tile < ndt, chunks = !driven && tile < ndt + nchunk;
-  const int b0 = driven ? tile * per : d.nDriven + (tile - ndt - nchunk) * NB;
-  const int nbk = driven ? min(per, d.nDriven - b0) : min(NB, d.nb - b0);
-  int k0 = 0, kend = 0;
   if (chunks) {
     const int c = (tile - ndt) * (T / 64) + wv;
     if (c < d.nhch) {
@@ -1537,12 +1567,13 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
       const double s = sum_chunk(d, r.x, r.y, lane, vals + 64 * 6 * wv);
       if (lane < 6) d.hpart[6 * (size_t)c + lane] = s;
     }
-  } else {
-    k0 = d.soff[b0];
-    kend = d.soff[b0 + nbk];
   }
-  // (also of the heavy ones)
-  if (driven && t < nbk && (predict || relisted)) driven_bound(d, sp, b0 + t, predict, relisted, 1 - A.par);
+  // every body's limit, also a heavy one's; here the driven ones' bounds too
+  // (a body's limit, bound and allowance are written by this thread alone)
+  if (d.skip_far && t < nbk) {
+    if (relisted) d.climit[b] = lim;
+    if (driven && predict) driven_bound(d, sp, b, cb, lim, drift, npar);
+  }
   if (chunks || (driven && nbk == 1 && kend - k0 > d.heavy_min)) {  // no body to finish
     if (guard && t == 0) {
       if (A.fuse && !chunks) guard_body(d, sp, b0, d.kin[b0], rst, ga);  // (else k_heavy_finish does)
@@ -1551,38 +1582,18 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
     }
     return;
   }
-  // the records, and what finishing a body needs, ahead of the sums
-  d2* kd = reinterpret_cast<d2*>(d.kin + b0);
-  for (int k = t; k < 8 * nbk; k += T) {
-    const d2 x = kd[k];
-    double* r = rec + (k >> 3) * kRec + 2 * (k & 7);
-    r[0] = x.x;
-    r[1] = x.y;
-  }
-  const int b = b0 + t;
-  double mb = 1.0, cb = 0.0, rmx = 0.0, lim = 0.0;
-  v3 Ib = V(1.0, 1.0, 1.0);
-  bool run = false;
-  if (t < nbk) {
-    mb = d.mass[b];
-    Ib = ld3(d.inertia + 3 * (size_t)b);
-    run = d.soff[b + 1] - d.soff[b] <= d.heavy_min;
-    if (predict && d.skip_far) {
-      cb = d.cbound[b];
-      rmx = d.rmax[b];
-      lim = relisted ? d.ahead[b] : d.climit[b];
+#pragma unroll
+  for (int r = 0; r < kLoads; r++)
+    if (t + r * T < 8 * nbk) {
+      const int k = t + r * T;
+      double* to = rec + (k >> 3) * kRec + 2 * (k & 7);
+      to[0] = x[r].x;
+      to[1] = x[r].y;
     }
-    if (relisted && !driven) d.climit[b] = d.ahead[b];
-  }
-  static_assert(NB <= 64, "the first wavefront's threads have a body each");
   if (MANY) {
     const unsigned long long h = __ballot(t < nbk && !run);
     if (t == 0) heavy = h;
   }
-  // the summing lanes' bodies and slot ranges
-  const int lb = t / kLanes, lc = t % kLanes;
-  const bool sums = lb < nbk && lc * kComp < 6;
-  const int sb0 = sums ? d.soff[b0 + lb] : 0, sb1 = sums ? d.soff[b0 + lb + 1] : 0;
   __syncthreads();
   int c0 = 0, c1 = 0;
   if (t < nbk) {
@@ -1696,7 +1707,7 @@ __global__ void __launch_bounds__(T, 4) k_gather(Dev d, StepParams sp, GatherArg
     if (predict && !driven) {
       const BodyKin old = P;
       predict_free_with(sp, P, acc, arot);
-      add_motion_bound_with(d, sp, b, old, P, cb, rmx, lim, 1 - A.par);
+      add_motion_bound_with(d, sp, b, old, P, cb, rmx, lim, drift, npar);
     } else {
       store_resultants(d, b, F, M, acc, arot);
     }
@@ -2294,7 +2305,7 @@ __global__ void __launch_bounds__(kBlock) k_predict(Dev d, StepParams sp, int gl
   if (frozen(d)) return;
   const int gid = blockIdx.x * blockDim.x + threadIdx.x;
   if (blockIdx.x == 0) drive_controls_block(d, sp);
-  driven_bounds(d, sp, par);
+  driven_bounds(d, sp, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, par);
   // free bodies (Rockable.cpp:2036-2055), a grid-stride loop
   for (int b = gid; b < d.nb; b += gridDim.x * blockDim.x) {
     if (b < d.nDriven) continue;
@@ -2317,6 +2328,8 @@ __global__ void __launch_bounds__(kBlock) k_predict(Dev d, StepParams sp, int gl
 // new state in between and keeps the pose in LDS; then the 256 threads share
 // those bodies' vertices (global vertices of the listed ones).  Rewriting a
 // record's unchanged fields (R, h, shape, group) stores the bits it read.
+// The driven bodies' motion bounds are kept by the wavefronts that wait for the
+// first one (ahead of the bodies they took 1.4 us of a step of 300 hulls).
 // The driven bodies are moved by thread 0 of workgroup 0 (controls); with
 // driven_glob, workgroup 0 then writes their listed global vertices (else
 // k_glob does after this kernel).
@@ -2326,7 +2339,6 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
   __shared__ int shp[64];           // shape, or -1 if the body is not listed
   if (frozen(d)) return;
   const int t = threadIdx.x;
-  driven_bounds(d, sp, par);
   if (blockIdx.x == 0) {
     drive_controls_block(d, sp);
     if (driven_glob) {
@@ -2350,6 +2362,7 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
     // latencies overlap
     v3 acc = V(0.0, 0.0, 0.0), arot = acc;
     double cb = 0.0, rmx = 0.0, lim = 0.0;
+    v3 drift = acc;
     bool listed = false;
     if (t < 64 && b0 + t < bend) {
       const int b = b0 + t;
@@ -2359,8 +2372,17 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
         cb = d.cbound[b];
         rmx = d.rmax[b];
         lim = d.climit[b];
+        drift = ld3(d.drift);
       }
       listed = d.soff[b + 1] != d.soff[b];
+    }
+    // a driven body's for a thread of the other wavefronts
+    const int db = (int)blockIdx.x * (kBlock - 64) + t - 64;
+    const bool drv = t >= 64 && tile == (int)blockIdx.x && db < d.nDriven && d.skip_far;
+    if (drv) {
+      cb = d.cbound[db];
+      lim = d.climit[db];
+      drift = ld3(d.drift);
     }
     __syncthreads();
     if (t < 64) {
@@ -2372,7 +2394,7 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
         const BodyKin old = P;
         predict_free_with(sp, P, acc, arot);
         rec_store_motion(r, P);
-        add_motion_bound_with(d, sp, b, old, P, cb, rmx, lim, par);
+        add_motion_bound_with(d, sp, b, old, P, cb, rmx, lim, drift, par);
         if (listed) {
           pose[t][0] = P.px;
           pose[t][1] = P.py;
@@ -2385,6 +2407,10 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
           shp[t] = P.shape;
         }
       }
+    } else if (drv) {
+      driven_bound(d, sp, db, cb, lim, drift, par);
+      const int stride = (int)gridDim.x * (kBlock - 64);
+      driven_bounds(d, sp, db + stride, stride, par);
     }
     __syncthreads();
     for (int k = t; k < nd; k += blockDim.x) kd[k] = rec[(k >> 4) * kRec + (k & 15)];
@@ -2418,7 +2444,7 @@ __global__ void __launch_bounds__(kBlock) k_predict_blk(Dev d, StepParams sp, in
 __global__ void __launch_bounds__(kBlock) k_predict_vtx(Dev d, StepParams sp, int par) {
   if (frozen(d)) return;
   if (blockIdx.x == 0) drive_controls_block(d, sp);
-  driven_bounds(d, sp, par);
+  driven_bounds(d, sp, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, par);
   const int lane = threadIdx.x & 63;
   for (int wv = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6); wv < d.nwv;
        wv += (int)((gridDim.x * blockDim.x) >> 6)) {
@@ -2588,6 +2614,7 @@ void launch_predict(const Dev& d, const StepParams& sp, int glob, int par, hipSt
     hipLaunchKernelGGL(k_predict, grid_for(d, (n + bs - 1) / bs), dim3(bs), 0, s, d, sp, 0, par);
     return;
   }
+  par = -1;  // the step takes no list
   const bool listed = glob == GLOB_LISTED && d.soff;  // else every body's vertices
   if (listed && d.fuse_glob == 3 && d.nb > d.nDriven) {
     // workgroups of 64 free bodies, their vertices from the poses in LDS; a
