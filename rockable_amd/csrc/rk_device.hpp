@@ -403,9 +403,11 @@ void launch_drive(const Dev& d, const StepParams& sp, int glob, hipStream_t s);
 // capacity of gpart for any launch shape
 int gather_blocks_max(int nb, int nhch);
 void launch_breakage(const Dev& d, const StepParams& sp, hipStream_t s);
-// Read-outs packed on the device.  The bodies' kinematics as four arrays (3,
-// 4, 3 and 3 doubles per body: pos, Q, vel, vrot), out holding 13 nb doubles;
-void launch_pack_bodies(const Dev& d, double* out, hipStream_t s);
+// Read-outs packed on the device.  The bodies' state as arrays one after the
+// other: pos, Q, vel, vrot (3, 4, 3 and 3 doubles a body) and with all also
+// acc, arot, force, moment (3 each); out, on the device or mapped host memory,
+// holds 13 nb or 25 nb doubles;
+void launch_pack_bodies(const Dev& d, double* out, int all, hipStream_t s);
 // the active entries' count (block: active_blocks(d) + 1 integers, the last
 // one the count) and their records in entry order, at most cap of them.
 int active_blocks(const Dev& d);

@@ -2465,20 +2465,28 @@ __global__ void __launch_bounds__(kBlock) k_predict_vtx(Dev d, StepParams sp, in
   }
 }
 
-// The bodies' kinematics as the arrays the caller reads (pos, Q, vel, vrot):
-// one thread per double of the 13, so that the records are read and the arrays
-// written in near-contiguous runs.
-__global__ void __launch_bounds__(kBlock) k_pack_bodies(Dev d, double* out) {
-  const long n = 13l * d.nb;
+// The bodies' state as the arrays the caller reads: pos, Q, vel and vrot (13
+// doubles a body), with all also acc, arot, force and moment (25).  One thread
+// per double written, in order: out may lie in host memory, which is written
+// in whole lines then.
+__global__ void __launch_bounds__(kBlock) k_pack_bodies(Dev d, double* out, int all) {
+  const long nb = d.nb, n = (all ? 25l : 13l) * nb;
   const double* kin = reinterpret_cast<const double*>(d.kin);
   for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (long)gridDim.x * blockDim.x) {
-    const long b = k / 13;
-    const int c = (int)(k - 13 * b);
-    const double x = kin[16 * b + c];
-    const long nb = d.nb;
-    const long at = c < 3 ? 3 * b + c : c < 7 ? 3 * nb + 4 * b + (c - 3) : c < 10 ? 7 * nb + 3 * b + (c - 7)
-                                                                       : 10 * nb + 3 * b + (c - 10);
-    out[at] = x;
+    double x;
+    if (k < 3 * nb) {
+      x = kin[16 * (k / 3) + k % 3];
+    } else if (k < 7 * nb) {
+      const long q = k - 3 * nb;
+      x = kin[16 * (q / 4) + 3 + q % 4];
+    } else if (k < 13 * nb) {
+      const long q = k - 7 * nb, at = q < 3 * nb ? 7 : 10, r = q < 3 * nb ? q : q - 3 * nb;
+      x = kin[16 * (r / 3) + at + r % 3];
+    } else {
+      const long q = k - 13 * nb;
+      x = q < 3 * nb ? d.acc[q] : q < 6 * nb ? d.arot[q - 3 * nb] : q < 9 * nb ? d.force[q - 6 * nb] : d.moment[q - 9 * nb];
+    }
+    out[k] = x;
   }
 }
 
@@ -2637,9 +2645,9 @@ void launch_predict(const Dev& d, const StepParams& sp, int glob, int par, hipSt
   launch_glob(d, listed ? 0 : 1, fused ? d.nvdriven : d.nvtot, s);
 }
 
-void launch_pack_bodies(const Dev& d, double* out, hipStream_t s) {
-  const long n = (13l * d.nb + kBlock - 1) / kBlock;
-  hipLaunchKernelGGL(k_pack_bodies, dim3((int)std::min(n, 65536L)), dim3(kBlock), 0, s, d, out);
+void launch_pack_bodies(const Dev& d, double* out, int all, hipStream_t s) {
+  const long n = ((all ? 25l : 13l) * d.nb + kBlock - 1) / kBlock;
+  hipLaunchKernelGGL(k_pack_bodies, dim3((int)std::min(n, 65536L)), dim3(kBlock), 0, s, d, out, all);
 }
 
 int active_blocks(const Dev& d) { return (d.ne + kActiveTile - 1) / kActiveTile; }
