@@ -90,3 +90,25 @@ def test_limit_of_an_uncontrolled_driven_body(tmp_path, gap, ndriven, heavy_min)
         assert b.counts()["nactive"] == active
         assert a.counts()["nactive"] == active
         assert_bodies_equal(a.bodies(), b.bodies())
+
+
+@pytest.mark.parametrize("dims", [(8, 8, 4), (13, 13, 7), (32, 31, 24)])
+def test_every_entry_listed(tmp_path, dims):
+    """A squeezed lattice, every contact active: the parts of the list are full,
+    with a lane for each of their entries and, past 65 536 entries, with fewer."""
+    from rockable_amd.engine import Engine
+    shapes, deck = D.sphere_lattice_deck(dims=dims, spacing_factor=1.9999, seed=7, vmax=0.01, nl="linkCells")
+    path = D.write_deck(str(tmp_path), shapes, deck)
+    a, b = Engine(path), Engine(path)
+    for e, skip in ((a, 1), (b, 0)):
+        e.set_option("record_geometry", 0)
+        e.set_option("skip_far", skip)
+        e.update_nl()
+    for steps in (1, 30):
+        a.step(steps)
+        b.step(steps)
+        c = a.counts()
+        assert c["nactive"] == c["nlisted"] or steps > 1  # (half of them open as the lattice springs back)
+        assert_bodies_equal(a.bodies(), b.bodies())
+    assert (c["nlisted"] > 65536) == (dims[0] == 32)
+    assert_interactions_equal(a.interactions(), b.interactions(), fields=("dn", "fn", "ft", "mom", "damp", "stick"))
