@@ -384,8 +384,6 @@ void launch_interact(const Dev& d, const StepParams& sp, int write_geom_all, int
 void launch_refresh_gaps(const Dev& d, hipStream_t s);
 // Every entry evaluated at the next step (after the poses were set from outside).
 void launch_reset_keys(const Dev& d, hipStream_t s);
-// The evaluation list written anew at the next step.
-void launch_reset_list(const Dev& d, hipStream_t s);
 // kick: the closing half kick; guard: also the displacement check's
 // accumulation (k_guard_check then follows); fuse: the free bodies also take
 // the next step's predictor, unless a rebuild falls due after this one

@@ -82,6 +82,8 @@ struct rk_engine {
   double *ahead = nullptr, *climit = nullptr;  // and the evaluation list's limits on them
   double* drift = nullptr;
   ListState* ls = nullptr;
+  ListItem* elist = nullptr;  // the evaluation list, one for both entry buffers (null: no room, no list)
+  size_t elist_cap = 0;
   int parity = 0;  // of the next step (ListState)
   int skip_far = 1;
   int skip_seg = 1024;  // entries tested and compacted per workgroup under the skip (256: no compaction)
@@ -252,6 +254,22 @@ int grow(rk_engine* eng, T*& p, size_t& cap, size_t n) {
   return 0;
 }
 
+// Room for the evaluation list of the current entries, whose list starts anew
+// after this.  A device without it keeps testing every entry.
+void reserve_list(rk_engine* eng) {
+  const EntryArrays& E = eng->E[eng->cur];
+  if (eng->elist_cap >= (size_t)E.n) return;
+  if (eng->elist) (void)hipFree(eng->elist);
+  eng->elist = eng->d.elist = nullptr;
+  eng->elist_cap = 0;
+  if (hipMalloc(&eng->elist, E.cap * sizeof(ListItem)) == hipSuccess) {
+    eng->elist_cap = E.cap;
+  } else {
+    eng->elist = nullptr;
+    (void)hipGetLastError();
+  }
+}
+
 void free_graphs(rk_engine* eng) {
   for (auto& g : eng->graphs)
     if (g.exec) (void)hipGraphExecDestroy(g.exec);
@@ -267,7 +285,7 @@ void free_device(rk_engine* eng) {
                 eng->ifc_key,  eng->ifc_istart, eng->ifc_par,  eng->ifc_inner, eng->ifc_alive, eng->ifc_bond_off, eng->ifc_bond_key,
                 eng->ifc_brk,  eng->ifc_broken, eng->ifc_nbroken, eng->ctrl,      eng->ctrl_off,  eng->ctrl_idx,  eng->flags,    eng->passive,
                 eng->gv,       eng->bvoff,     eng->bvbody,    eng->guard,     eng->gdpos,    eng->gdq,      eng->gpart,
-                eng->beoff,    eng->bfoff,     eng->cbound,    eng->rmax,  eng->ahead, eng->climit, eng->drift, eng->ls,
+                eng->beoff,    eng->bfoff,     eng->cbound,    eng->rmax,  eng->ahead, eng->climit, eng->drift, eng->ls, eng->elist,
                 eng->pack_bodies, eng->active_block, eng->active_rec,
                 eng->feat,     eng->pred,      eng->feat_part, eng->stat_part, eng->stat_out};
   for (void* p : ps)
@@ -276,6 +294,8 @@ void free_device(rk_engine* eng) {
   eng->acc = eng->arot = eng->force = eng->moment = eng->mass = eng->inertia = eng->bf_surface = nullptr;
   eng->cbound = eng->rmax = eng->ahead = eng->climit = eng->drift = nullptr;
   eng->ls = nullptr;
+  eng->elist = nullptr;
+  eng->elist_cap = 0;
   eng->pack_bodies = nullptr;
   eng->active_block = nullptr;
   eng->active_rec = nullptr;
@@ -449,7 +469,7 @@ void assemble_dev(rk_engine* eng) {
   d.ahead_min = 0.01 * m.dVerlet;
   d.drift = eng->drift;
   d.ls = eng->ls;
-  d.elist = E.elist;
+  d.elist = eng->elist;
   d.edesc_s = E.edesc + E.n;
   d.skip_far = eng->skip_far;
   d.skip_count = eng->skip_count;
@@ -918,6 +938,7 @@ int upload_model(rk_engine* eng) {
   eng->nlp.cellMinSizes[1] = m.cellMinSizes.y;
   eng->nlp.cellMinSizes[2] = m.cellMinSizes.z;
   eng->nlp.boxForLinkCellsOpt = m.boxForLinkCellsOpt;
+  reserve_list(eng);
   if (ensure_gpart(eng) != 0) return -1;
   assemble_dev(eng);
   launch_entry_desc(eng->d, eng->stream);
@@ -1062,6 +1083,7 @@ int do_update_nl(rk_engine* eng) {
   if (nl_rebuild(eng->w, eng->d, eng->nlp, eng->E[eng->cur], eng->E[nxt], eng->stream) != 0)
     return fail(eng, std::string("neighbour list: ") + eng->w.err);
   eng->cur = nxt;
+  reserve_list(eng);
   if (ensure_gpart(eng) != 0) return -1;
   assemble_dev(eng);
   launch_entry_desc(eng->d, eng->stream);

@@ -2157,7 +2157,6 @@ int entries_reserve(NLWork& w, EntryArrays& E, int n) {
             hipMalloc(&E.egeo, c * sizeof(EGeom)) == hipSuccess && hipMalloc(&E.edamp, c * sizeof(double)) == hipSuccess &&
             hipMalloc(&E.estick, c * sizeof(int32_t)) == hipSuccess && hipMalloc(&E.eact, c * sizeof(uint8_t)) == hipSuccess &&
             hipMalloc(&E.ekey, c * sizeof(double)) == hipSuccess &&
-            hipMalloc(&E.elist, c * sizeof(ListItem)) == hipSuccess &&
             hipMalloc(&E.spos, c * 2 * sizeof(int32_t)) == hipSuccess &&
             hipMalloc(&E.sact, c * 2 * sizeof(uint8_t) + 64) == hipSuccess  /* read 16 bytes at a time */ &&
             hipMalloc(&E.sval, c * 12 * sizeof(double)) == hipSuccess &&
@@ -2174,11 +2173,10 @@ int entries_reserve(NLWork& w, EntryArrays& E, int n) {
 
 void entries_free(EntryArrays& E) {
   void* ps[] = {E.ei, E.ej, E.esub, E.est, E.edn, E.egeo, E.edamp, E.estick, E.eact, E.ekey, E.spos, E.sact, E.sval,
-                E.akin, E.acount, E.elist};
+                E.akin, E.acount};
   for (void* q : ps)
     if (q) (void)hipFree(q);
   E.ekey = nullptr;
-  E.elist = nullptr;
   E.ei = E.ej = nullptr;
   E.esub = nullptr;
   E.est = nullptr;

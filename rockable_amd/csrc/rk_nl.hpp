@@ -33,7 +33,6 @@ struct EntryArrays {
   int32_t* acount = nullptr; // 1 per geometry block (64 entries or more)
   int4* edesc = nullptr;     // 2 per entry: vertex indices of its geometry (global, then in the shapes' table)
   size_t edesc_cap = 0;
-  ListItem* elist = nullptr; // 1 per entry: room for the evaluation list
   int32_t* istart = nullptr;
   size_t istart_cap = 0;
   int32_t* jstart = nullptr;

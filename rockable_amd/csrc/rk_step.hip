@@ -134,9 +134,6 @@ __device__ __forceinline__ void reset_list(const Dev& d) {
   d.ls->want[0] = d.ls->want[1] = 1;
   d.ls->again = 1;
 }
-__global__ void k_reset_list(Dev d) {
-  if (threadIdx.x == 0) reset_list(d);
-}
 __global__ void __launch_bounds__(kBlock) k_entry_desc(Dev d) {
   if (blockIdx.x == 0) {
     // a new list: the evaluation list starts anew, and the motion bounds'
@@ -2602,10 +2599,6 @@ void launch_refresh_gaps(const Dev& d, hipStream_t s) {
   hipLaunchKernelGGL(k_refresh_gaps, dim3(std::min((d.ne + kBlock - 1) / kBlock, 65536)), dim3(kBlock), 0, s, d);
 }
 
-void launch_reset_list(const Dev& d, hipStream_t s) {
-  hipLaunchKernelGGL(k_reset_list, dim3(1), dim3(64), 0, s, d);
-}
-
 void launch_reset_keys(const Dev& d, hipStream_t s) {
   if (d.ne <= 0 || !d.ekey) return;
   hipLaunchKernelGGL(k_reset_keys, dim3(std::min((d.ne + kBlock - 1) / kBlock, 65536)), dim3(kBlock), 0, s, d);
@@ -2692,7 +2685,7 @@ void launch_fused_sorted(const Dev& d, const StepParams& sp, int write_geom_all,
 }
 
 bool uses_list(const Dev& d, int write_geom_all) {
-  return !write_geom_all && d.fuse_law && d.skip_far && d.skip_seg >= 512;
+  return !write_geom_all && d.fuse_law && d.skip_far && d.skip_seg >= 512 && (d.elist || d.ne <= 0);
 }
 
 // The grid of the list kernel: a lane for each second entry (a list holds a

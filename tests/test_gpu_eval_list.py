@@ -112,3 +112,22 @@ def test_every_entry_listed(tmp_path, dims):
         assert_bodies_equal(a.bodies(), b.bodies())
     assert (c["nlisted"] > 65536) == (dims[0] == 32)
     assert_interactions_equal(a.interactions(), b.interactions(), fields=("dn", "fn", "ft", "mom", "damp", "stick"))
+
+
+def test_one_list_for_both_entry_buffers(tmp_path):
+    """A rebuild that fills the other entry buffer for the first time takes no
+    room for a second evaluation list: 640 bytes a listed entry (buffers are
+    reserved for half as many again), 96 fewer than with one."""
+    import ctypes
+    from rockable_amd.engine import Engine
+    shapes, deck = D.sphere_lattice_deck(dims=(60, 60, 30), spacing_factor=2.002, seed=3, vmax=0.0, nl="linkCells")
+    e = Engine(D.write_deck(str(tmp_path), shapes, deck))
+    hip = ctypes.CDLL("libamdhip64.so")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    left = []
+    for _ in range(2):
+        e.update_nl()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        left.append(free.value)
+    assert e.counts()["nlisted"] > 300000
+    assert (left[0] - left[1]) / e.counts()["nlisted"] < 700
