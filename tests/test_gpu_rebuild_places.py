@@ -38,9 +38,11 @@ def test_windows_past_the_first(tmp_path):
     """265 200 spheres on a floor: body indices and entry indices beyond one
     window.  The list is that of the lattice: every sphere with its axis
     neighbours, with the floor and with the walls, in ascending order, each
-    pair once and unchanged by a rebuild; the resultants add up over it."""
+    pair once and unchanged by a rebuild; the resultants of the contacts that
+    form, on bodies and in slots past the first window, equal the serial sums
+    of the heavy-body kernel."""
     dims = (340, 260, 3)
-    e, _ = _engine(tmp_path, dims, vmax=0.0)
+    e, _ = _engine(tmp_path, dims, vmax=0.05)
     e.set_option("exact_sums", 1)
     e.update_nl()
     a = e.interactions()
@@ -62,12 +64,16 @@ def test_windows_past_the_first(tmp_path):
     edge = np.unique(np.concatenate([idx[:, :, 0].ravel(), idx[0].ravel(), idx[-1].ravel(), idx[:, 0].ravel(),
                                      idx[:, -1].ravel()]))
     assert np.array_equal(floor, edge)
-    b, _ = _engine(tmp_path, dims, vmax=0.0)
+    b, _ = _engine(tmp_path, dims, vmax=0.05)
     b.set_option("exact_sums", 1)
-    b.set_option("heavy_min", 8)
+    b.set_option("heavy_min", 1)
     b.update_nl()
-    e.step(20)
-    b.step(20)
+    b.update_nl()
+    for x in (e, b):
+        x.step(60)
+    act = e.interactions()
+    act = np.nonzero((act["dn"] < 0) & (act["i"] > 2 ** 18))[0]
+    assert len(act) > 100 and act.max() > 2 ** 18
     assert_bodies_equal(e.bodies(), b.bodies())
 
 

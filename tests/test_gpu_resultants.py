@@ -123,3 +123,25 @@ def test_many_driven_bodies_with_heavy_ones(tmp_path, dynamic):
         assert a.counts()["nl_updates"] == b.counts()["nl_updates"] == c.counts()["nl_updates"]
     assert a.counts()["nactive"] > 1000
     assert not dynamic or a.counts()["nl_updates"] > 2
+
+
+@pytest.mark.parametrize("dims", [(60, 60, 1), (200, 170, 1), (363, 363, 1)])
+def test_body_force_forms_match_serial_sums(tmp_path, dims):
+    """The resultant kernel's forms with a body force: 256 threads to a group of
+    32 bodies, 128, and 128 to a group of 64 from 131 072 bodies, against the
+    serial sums of k_gather_heavy (heavy_min 1)."""
+    from rockable_amd import decks as D
+    from rockable_amd.engine import Engine
+    shapes, deck = D.sphere_lattice_deck(dims=dims, spacing_factor=2.002, seed=4, vmax=0.05, nl="linkCells")
+    deck.gravity = (3.0, -2.0, -400.0)
+    deck.body_force = "ViscousFluid 1000.0"
+    path = D.write_deck(str(tmp_path), shapes, deck)
+    a, b = Engine(path), Engine(path)
+    b.set_option("heavy_min", 1)
+    for e in (a, b):
+        e.set_option("exact_sums", 1)
+        e.set_option("record_geometry", 0)
+        e.update_nl()
+        e.step(120)
+    assert a.counts()["nactive"] > dims[0] * dims[1] // 8
+    assert_bodies_equal(a.bodies(), b.bodies())

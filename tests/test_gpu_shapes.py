@@ -1,11 +1,12 @@
 """Launch shapes and the autotuner: every choice of fuse_law, law_group,
-geom_block, gather_lanes, gather_groups, fuse_glob, gather_waves,
-body_block, persistent, graph_steps, type_sort and narrow_pairs (candidate pairs per
-narrow-phase wavefront; the default for these hulls is 1) computes the
-same state bit for bit (the default engine, against which they are compared, fuses the
-geometry and law kernels; the first three shapes use them apart), and the
-steps the autotuner takes while timing candidates are the steps rk_step
-takes."""
+geom_block, fuse_glob, body_block, persistent, graph_steps, type_sort and
+narrow_pairs (candidate pairs per narrow-phase wavefront; the default for
+these hulls is 1), and of gather_lanes, gather_groups and gather_waves, which
+are kept without effect, computes the same state bit for bit (the default
+engine, against which they are compared, fuses the geometry and law kernels;
+the first three shapes use them apart), with geometry records and then, on
+the evaluation list where the shape takes it, without; and the steps the
+autotuner takes while timing candidates are the steps rk_step takes."""
 import pytest
 
 from tests.test_gpu_parity import _dynamic_hull_deck, assert_bodies_equal, assert_interactions_equal
@@ -50,6 +51,13 @@ def test_launch_shapes_bit_exact(tmp_path, k):
     for e in (a, b):
         e.update_nl()
     for n in (300, 700):
+        a.step(n)
+        b.step(n)
+        assert_bodies_equal(b.bodies(), a.bodies())
+        assert_interactions_equal(b.interactions(), a.interactions(), fields=FIELDS)
+    for e in (a, b):
+        e.set_option("record_geometry", 0)
+    for n in (1, 300):
         a.step(n)
         b.step(n)
         assert_bodies_equal(b.bodies(), a.bodies())
