@@ -124,7 +124,8 @@ def form_autotune(e, a):
     engine's defaults (no captured graphs), as a profiled run takes them."""
     if a.no_autotune:
         return 0, {k: int(e.get_option(k)) for k in e.TUNED}
-    return e.autotune(steps_per_trial=a.tune_trial)
+    n, choice = e.autotune(steps_per_trial=a.tune_trial)
+    return n, {k: choice[k] for k in e.TUNED}
 
 
 def interverlet_steps(e):
@@ -648,7 +649,7 @@ def main():
             choice[k.strip()] = int(float(v))
         tuned = 0
     else:
-        tuned, choice = (0, None) if a.no_autotune else e.autotune(steps_per_trial=a.tune_trial)
+        tuned, choice = (0, None) if a.no_autotune else form_autotune(e, a)
     e.step(max(0, a.warmup - tuned))
     e.synchronize()
     log("warm-up: %d steps (%d of them autotuning: %s) in %.2f s" % (max(a.warmup, tuned), tuned, choice,
@@ -721,7 +722,8 @@ def main():
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": achieved / PEAK_HBM_GBS, "traffic": TRAFFIC_BYTES_PER_LAUNCH[skip_far],
                      "kernel": "force phase (k_interact_list with the far-entry skip, else k_interact or k_geom + "
-                               "k_law; then k_gather + k_heavy_finish)",
+                               "k_law; then k_gather, which takes the next step's predictor, and at a run's end "
+                               "k_heavy_finish)",
                      "algorithmic_bytes_per_launch": bytes_per},
     }
     sk = skip_accounting(e, period, nb, nl_listed, "Avalanche", t_force)

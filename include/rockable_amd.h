@@ -158,9 +158,10 @@ int rk_set_body_force(rk_engine* eng, const char* name, const double* args, int 
  * 0: every listed entry every step), "skip_segment" (512, 1024, 2048 or 4096:
  * under skip_far the steps work from a list of the entries to evaluate, which
  * the device writes anew when a body outruns its allowance; 256: every entry
- * is tested at every step; default 1024), "count_skips" (1: the geometry pass
- * counts entries skipped, inactive with zero history, and looked at, read
- * back with rk_get_option as "skipped_entries", "zero_history_entries" and
+ * is tested at every step; default 1024), "count_skips" (1: every step counts
+ * the entries that may be skipped by the bounds as they stand (a few of them
+ * are on the list all the same), those inactive with zero history, and all,
+ * read back with rk_get_option as "skipped_entries", "zero_history_entries" and
  * "entries_looked_at"; setting it again clears them; 0 stops counting),
  * launch shapes: "fuse_law" (1, the default: contact kinematics and force law
  * in one kernel; 0: two), "type_sort" (1, the default: the fused kernel takes
@@ -184,7 +185,9 @@ int rk_set_option(rk_engine* eng, const char* name, double value);
  * "dVerlet" and "tmax". */
 int rk_get_option(rk_engine* eng, const char* name, double* value);
 /* Autotuner (no counterpart in the reference) of fuse_law, law_group,
- * geom_block, fuse_glob, body_block, persistent, graph_steps, type_sort and skip_segment, one after the other: the
+ * geom_block, fuse_glob (not where the steps take the evaluation list, which
+ * reads no global vertices), body_block, persistent, graph_steps, type_sort
+ * and skip_segment, one after the other: the
  * simulation runs on, trial after trial of steps_per_trial steps, each
  * candidate value twice, and the fastest is kept: by the step kernels' own
  * durations per step (events around each kernel) for the kernel shapes, by

@@ -86,7 +86,7 @@ struct rk_engine {
   size_t elist_cap = 0;
   int parity = 0;  // of the next step (ListState)
   int skip_far = 1;
-  int skip_seg = 1024;  // entries tested and compacted per workgroup under the skip (256: no compaction)
+  int skip_seg = 1024;  // under the skip: 512 or more the evaluation list, 256 every entry tested where it stands
   unsigned long long* skip_count = nullptr;  // count_skips: the geometry pass's counts
   int32_t* cluster = nullptr;
   int32_t *sh_nv = nullptr, *sh_ne = nullptr, *sh_nf = nullptr, *sh_voff = nullptr, *sh_eoff = nullptr,
@@ -2400,6 +2400,8 @@ int rk_autotune(rk_engine* eng, int steps_per_trial, int64_t* steps_done) {
   double t_last = 1e30;
   for (const Knob& k : knobs) {
     if (rc != 0) break;
+    // (on the evaluation list no step writes global vertices: nothing to time)
+    if (!strcmp(k.name, "fuse_glob") && uses_list(eng->d, eng->record_geometry)) continue;
     std::vector<double> best(k.values.size(), 1e30);
     for (int rep = 0; rep < 2 && rc == 0; rep++)
       for (size_t c = 0; c < k.values.size() && rc == 0; c++) {

@@ -25,7 +25,8 @@
 //                    sorted by (i, j, type, isub, jsub)
 //   k_merge_fill     one thread per new entry: its state record, copied from
 //                    the old entry it keeps or started from zero
-//   CSR              istart by owner; jlist = entries sorted (stably) by j
+//   CSR              istart by owner; jlist = entries by j, in any order within
+//                    a body's
 #include <hip/hip_runtime.h>
 
 #include <rocprim/device/device_scan.hpp>

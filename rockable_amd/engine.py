@@ -217,16 +217,17 @@ class Engine:
         dVerlet or tmax."""
         return self.get_option(name)
 
-    TUNED = ("fuse_law", "type_sort", "skip_segment", "law_group", "geom_block", "gather_lanes", "gather_groups", "fuse_glob", "gather_waves",
-             "body_block", "persistent",
-             "graph_steps")
+    TUNED = ("fuse_law", "type_sort", "skip_segment", "law_group", "geom_block", "fuse_glob", "body_block",
+             "persistent", "graph_steps")
+    KEPT = ("gather_lanes", "gather_groups", "gather_waves")  # accepted and read back, without effect
 
     def autotune(self, steps_per_trial=100):
         """Pick the launch shapes by timing them on the running simulation
-        (the steps taken are real steps); returns (steps taken, choices)."""
+        (the steps taken are real steps); returns (steps taken, choices),
+        with the options of KEPT as they stand among the choices."""
         n = ctypes.c_int64(0)
         self._check(self.L.rk_autotune(self.h, int(steps_per_trial), ctypes.byref(n)))
-        return int(n.value), {k: int(self.get_option(k)) for k in self.TUNED}
+        return int(n.value), {k: int(self.get_option(k)) for k in self.TUNED + self.KEPT}
 
     def update_nl(self):
         self._check(self.L.rk_update_nl(self.h))
