@@ -32,6 +32,7 @@
 #include <rocprim/device/device_scan.hpp>
 
 #include <algorithm>
+#include <climits>
 #include <cstdio>
 #include <cstring>
 #include <functional>
@@ -509,13 +510,20 @@ __device__ int win_mark(WinLds& L, const int32_t* val, int s0, int s1, int win) 
   if (t == 0) L.below = 0;
   __syncthreads();
   int under = 0;
-  for (int q = s0 + t; q < s1; q += kWinThreads) {
-    const int v = val[q];
-    const int vw = v >> kWinBits;
-    if (vw < win)
-      under++;
-    else if (vw == win)
-      atomicOr(&L.bits[(v & ((1 << kWinBits) - 1)) >> 6], 1ull << (v & 63));
+  // (four members a round, so that their loads share a latency)
+  for (int q0 = s0 + t; q0 < s1; q0 += 4 * kWinThreads) {
+    int v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = q0 + k * kWinThreads < s1 ? val[q0 + k * kWinThreads] : INT_MAX;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if (q0 + k * kWinThreads >= s1) continue;
+      const int vw = v[k] >> kWinBits;
+      if (vw < win)
+        under++;
+      else if (vw == win)
+        atomicOr(&L.bits[(v[k] & ((1 << kWinBits) - 1)) >> 6], 1ull << (v[k] & 63));
+    }
   }
   if (under) atomicAdd(&L.below, under);
   __syncthreads();
@@ -648,10 +656,18 @@ __global__ void __launch_bounds__(kWinThreads) k_group_place_big(GroupIn G) {
     const int s0 = G.gstart[b], s1 = G.gstart[b + 1];
     const int o0 = old_first(G, b), o1 = old_first(G, b + 1);
     const int below = win_mark(L, G.gother, s0, s1, win);
-    for (int t = s0 + (int)threadIdx.x; t < s1; t += kWinThreads) {
-      const int v = G.gother[t];
-      if ((v >> kWinBits) == win)
-        put_cand(G, s0 + o0 + below + win_rank(L, v) + old_below(G, o0, o1, v), b, v, G.gref[t]);
+    for (int t0 = s0 + (int)threadIdx.x; t0 < s1; t0 += 4 * kWinThreads) {
+      int v[4], ref[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const int t = min(t0 + k * kWinThreads, s1 - 1);
+        v[k] = G.gother[t];
+        ref[k] = G.gref[t];
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        if (t0 + k * kWinThreads < s1 && (v[k] >> kWinBits) == win)
+          put_cand(G, s0 + o0 + below + win_rank(L, v[k]) + old_below(G, o0, o1, v[k]), b, v[k], ref[k]);
     }
     for (int g = o0 + (int)threadIdx.x; g < o1; g += kWinThreads) {
       const uint64_t key = G.okey[g];
