@@ -53,11 +53,11 @@ PEAK_HBM_GBS = 8000.0
 # HBM bytes per force-phase launch on the 50 005-body settled pour:
 # rocprofv3 FETCH_SIZE and WRITE_SIZE, each scaled by what it reads for a
 # plain 256 MiB device copy (factors 2.0 and 1.0).  With the far-entry skip
-# (the per-step entry test that k_interact_list replaced, k_gather and
-# k_heavy_finish; not counted again since): 137.0 MB read + 27.9 MB
-# written, profiles/c2_force_phase_traffic.md; without it (k_interact +
-# k_gather + k_heavy_finish, measured before the skip): 171.3 + 36.3 MB.
-TRAFFIC_BYTES_PER_LAUNCH = {1: 164.9e6, 0: 207.6e6}
+# (k_interact_list, and k_gather with the next step's predictor): 110.9 MB
+# read + 31.6 MB written, profiles/c2_force_phase_traffic.md.  Without it the
+# kernels of the force phase were last counted before k_gather took the
+# predictor, so no figure is given.
+TRAFFIC_BYTES_PER_LAUNCH = {1: 142.6e6, 0: None}
 
 
 def make_settled_deck(n_bodies, seed, dirpath, settle_steps, relax_steps, log):

@@ -13,7 +13,7 @@
 //   k_obb            Particle::updateObb (+ AABB for the cell grid)
 //   k_broad_*        candidate body pairs (i < j) whose enlarged OBBs overlap
 //   groups           directed (owner, other) groups = candidates x 2 directions
-//                    merged with the groups of the current list (radix sort)
+//                    merged with the groups of the current list (placed by counts)
 //   k_narrow         one wavefront per candidate pair: global vertices and
 //                    vertex gates in LDS, every predicate of both directions
 //                    evaluated 64 at a time, near bits kept as ballot masks,

@@ -2756,7 +2756,9 @@ void launch_interact(const Dev& d, const StepParams& sp, int write_geom_all, int
 // k_gather's free bodies per workgroup: 32, so that a small packing spreads
 // over more workgroups and a bonded body's many terms fit one LDS pass; 64
 // from 131 072 bodies, where workgroups abound and the lanes that finish
-// the bodies count.
+// the bodies count.  64 against 32, 128 threads: 33.5 and 44.0 us for 288 005
+// spheres, 35.8 and 39.9 us for 160 005 hulls, 89.2 and 91.7 us for 200 001
+// bonded cubes.
 constexpr int kGatherLarge = 1 << 17;
 bool gather_many(const Dev& d) { return d.nDriven >= kDrivenMany; }
 int gather_bodies(const Dev& d) { return !gather_many(d) && d.nb - d.nDriven >= kGatherLarge ? 64 : 32; }
@@ -2765,9 +2767,11 @@ int gather_bodies(const Dev& d) { return !gather_many(d) && d.nb - d.nDriven >= 
 // 1024 of them) or bodies have many slots, whose terms then take fewer passes;
 // 128 where workgroups queue, since only one wavefront finishes the bodies and
 // the others' places are worth more to a second workgroup.  256 against 128:
-// 12.9 and 16.2 us for 13 001 bonded cubes (65 slots each), 9.7 and 10.5 us
-// for 706 hulls, but 28.7 and 22.7 us for the 90 006-body slope, 12.3 and 9.2
-// us for 47 000 spheres.
+// 12.9 and 16.2 us for 13 001 bonded cubes (63 slots each), 9.7 and 10.5 us
+// for 706 hulls, but 28.7 and 22.7 us for the 90 006-body slope (45 slots),
+// 12.3 and 9.2 us for 47 000 spheres.  At 63 slots the many groups of 100 001
+// cubes take 51.9 and 55.1 us, those of 40 001 26.9 and 24.5: the line on
+// slots lies between what was measured, not at a crossing.
 int gather_threads(const Dev& d) {
   if (gather_bodies(d) == 64 || gather_many(d)) return 128;
   const bool few = (d.nb - d.nDriven + 31) / 32 <= 1024, many_slots = 2.0 * d.ne > 56.0 * d.nb;
