@@ -2627,7 +2627,7 @@ int rk_get_counts(rk_engine* eng, rk_counts* out) {
   out->ndriven = eng->m.nDriven;
   out->nlisted = E.n;
   int32_t na = 0;
-  (void)hipSetDevice(eng->device);
+  if (E.n > 0) (void)hipSetDevice(eng->device);
   if (E.n > 0 && E.n <= kCountHost && eng->read_host) {
     HIPCHK(hipMemcpyAsync(eng->read_host, E.eact, E.n, hipMemcpyDeviceToHost, eng->stream));
     HIPCHK(hipStreamSynchronize(eng->stream));

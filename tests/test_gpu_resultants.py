@@ -55,7 +55,7 @@ def test_threads_per_group_match_serial_sums(tmp_path, dims):
     assert_bodies_equal(a.bodies(), b.bodies())
 
 
-def _glued_bed(d, dims, ndriven, dynamic=False):
+def _glued_bed(d, dims, ndriven, dynamic=False, body_force=None):
     """Layers of spheres pressed on each other, the first ndriven of the lowest
     one and the walls driven; controls on four of the grains."""
     from rockable_amd import decks as D
@@ -67,6 +67,7 @@ def _glued_bed(d, dims, ndriven, dynamic=False):
     deck.bodies = walls + low + [b for k, b in enumerate(grains) if k % dims[2]]
     deck.nDriven = ndriven
     deck.gravity = (30.0, -20.0, -400.0)
+    deck.body_force = body_force
     if dynamic:
         deck.interVerlet = 1e3
         deck.dynamic_update_nl = 1
@@ -79,14 +80,15 @@ def _glued_bed(d, dims, ndriven, dynamic=False):
     return path, drv
 
 
+@pytest.mark.parametrize("body_force", [None, "ViscousFluid 1000.0"])
 @pytest.mark.parametrize("dims,ndriven", [((45, 46, 2), 2047), ((45, 46, 2), 2048), ((72, 72, 2), 5123)])
-def test_many_driven_bodies_match_oracle(tmp_path, dims, ndriven):
+def test_many_driven_bodies_match_oracle(tmp_path, dims, ndriven, body_force):
     """Up to and past the 2 048 driven bodies from which a workgroup takes
     several (with a last group that is not full): sums, rebuilds and motion
     equal the serial oracle's."""
     from oracle.rk_oracle import Oracle
     from rockable_amd.engine import Engine
-    path, drv = _glued_bed(tmp_path, dims, ndriven)
+    path, drv = _glued_bed(tmp_path, dims, ndriven, body_force=body_force)
     e, o = Engine(path, driving=drv), Oracle(path, driving=drv, threads=8)
     e.set_option("record_geometry", 0)
     e.set_option("heavy_min", 10 ** 9)
